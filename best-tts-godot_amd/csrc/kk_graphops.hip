@@ -266,6 +266,15 @@ __global__ void __launch_bounds__(kDqlSmallThreads) dql_small(const float* __res
 // double and rounded once to fp32.  The only approximation is the rounding
 // of h to the 2^-s grid (at most 2^-31 once |h| <= 1), far below the fp32
 // rounding of a 256-term dot product.
+//
+// Bound by one CU a direction: a step is a serial chain of two barriers, and
+// between them four waves a SIMD share its VALU and matrix issue (each
+// instruction of the gates' part costs 16 cycles a step).  So that part is
+// kept short: the digit sums recombine in double (no 64-bit integer
+// multiplies), the sigmoid's division is one Newton step, the zero point's
+// sum of h stays in the VALU (its LDS shuffles were 0.5 us a step where
+// R's zero point is not 0), and R is packed through LDS in words at set-up.
+// Bidirectional, 640 -> 256, the whole call: 130 steps 254 -> 189 us.
 constexpr int kLstmThreads = 1024;
 constexpr int kLstmMaxH = kLstmThreads / 4;
 // Steps per chunk of the input projections: a chunk (4 rows of 4H floats,
@@ -277,7 +286,8 @@ typedef int lstm_v4i __attribute__((ext_vector_type(4)));
 typedef int lstm_v8i __attribute__((ext_vector_type(8)));
 
 struct LstmArgs {
-  const float* xw;       // [ndir][seq * batch][4H] x @ deq(W) + (wb + rb)
+  const float* xw;       // [ndir][seq * batch][4H] x @ deq(W)
+  const float* b;        // [ndir][8H] wb then rb, or NULL: wb + rb joins xw[t] as a step reads it
   const int8_t* r;       // [ndir][H][4H]
   const void* r_scale;   // [ndir] (or 1 element)
   int r_scale_dt;
@@ -293,27 +303,43 @@ struct LstmArgs {
   int64_t seq, batch, H, ndir;
 };
 
-// A workgroup barrier that orders LDS only: global loads (the prefetched
-// input projections) and stores (the outputs) stay in flight across it,
-// where __syncthreads would wait for them.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+// Integer sum over a wave's lanes, in lane 63 (DPP: no LDS round trips).
+__device__ __forceinline__ int wave_isum63(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false);   // lane pairs
+  v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false);   // quads
+  v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, false);  // eights
+  v += __builtin_amdgcn_update_dpp(0, v, 0x140, 0xF, 0xF, false);  // rows of sixteen
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row 0 into 1, 2 into 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // rows 0-1 into 2-3
+  return v;
 }
 
+// 1 / b correctly rounded, as the IEEE division gives it: one Newton step on
+// the hardware reciprocal (checked against the division for every mantissa
+// at each exponent from 2^0 to 2^60; beyond, and for NaN, the division).
+__device__ __forceinline__ float recip_from_one(float b) {
+  if (b < 0x1p60f) {
+    const float r = __builtin_amdgcn_rcpf(b);
+    return __builtin_fmaf(__builtin_fmaf(-b, r, 1.0f), r, r);
+  }
+  return 1.0f / b;
+}
+
+// R's staging: column j's 32 k-bytes of a chunk at kRPitch * j (48: four-byte
+// writes of eight k-quads by eight column quads meet two-way conflicts).
+constexpr int kRPitch = 48;
+
 __global__ void __launch_bounds__(kLstmThreads) lstm_recurrence(LstmArgs A) {
-  // R's staging area at set-up, then the double buffer of input projections
-  // [2][kLstmChunk][4H] floats (both 32 KiB)
-  __shared__ __align__(16) unsigned char big[32 * kLstmThreads];
+  // R's staging area at set-up (48 KiB), then the double buffer of input
+  // projections [2][kLstmChunk][4H] floats (32 KiB)
+  __shared__ __align__(16) unsigned char big[kRPitch * kLstmThreads];
   // digits of the scaled h: hd[i][p] holds digit i of the units k with
   // (k / 2) % 2 == p, at (k / 4) * 2 + k % 2 (the sparse A operand's order)
   __shared__ __align__(16) int8_t hd[4][2][kLstmMaxH / 2];
   __shared__ float gs[kLstmThreads];
   __shared__ float hring[kLstmChunk][kLstmMaxH];     // this chunk's h, for ys
   __shared__ float wmax[kLstmMaxH / 64];
-  __shared__ long long wsum[kLstmMaxH / 64];
-  int8_t (*rbuf)[kLstmThreads] = reinterpret_cast<int8_t (*)[kLstmThreads]>(big);
+  __shared__ double wsum[kLstmMaxH / 64];
   float* xs = reinterpret_cast<float*>(big);
   const int H = static_cast<int>(A.H), G4 = 4 * H;
   const int64_t d = blockIdx.x / A.batch, b = blockIdx.x % A.batch;
@@ -323,52 +349,68 @@ __global__ void __launch_bounds__(kLstmThreads) lstm_recurrence(LstmArgs A) {
   // spilled, and its reload would sit in every step)
   const float rs = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(
       int, load_as_f32(A.r_scale, A.r_scale_dt, A.r_scale_n > 1 ? d : 0))));
-  long long rz =
-      A.r_zp ? static_cast<long long>(load_as_i64(A.r_zp, A.r_zp_dt, A.r_zp_n > 1 ? d : 0)) : 0;
-  rz = static_cast<long long>(
-      (static_cast<unsigned long long>(static_cast<unsigned>(
-           __builtin_amdgcn_readfirstlane(static_cast<int>(rz >> 32))))
-       << 32) |
-      static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(rz))));
+  const int rz = __builtin_amdgcn_readfirstlane(static_cast<int>(
+      A.r_zp ? load_as_i64(A.r_zp, A.r_zp_dt, A.r_zp_n > 1 ? d : 0) : 0));
   const int8_t* R = A.r + d * static_cast<int64_t>(H) * G4;
   const float* xw = A.xw + d * A.seq * A.batch * G4;
   // B fragments: wave wv owns columns [64 wv, 64 wv + 64), four tiles of
   // 16; lane (n, g) = (lane % 16, lane / 16) holds R[ks*64 + 16g + e][col].
-  // R arrives through LDS in 32-row chunks (coalesced 4-byte loads).
+  // R arrives through LDS in chunks of 32 rows: a thread loads four rows of
+  // four columns (two such items), swaps the 4 x 4 bytes and leaves each
+  // column's four k as a word, so a fragment is one 16-byte read (as single
+  // bytes, 64 LDS reads a lane a chunk, the set-up took as long as 40 steps).
+  // The next chunk's loads are in flight meanwhile.
   lstm_v8i bf[4][2];  // [tile][k-step of 128]: the 64-row k-steps 2 kk and 2 kk + 1 side by side
+  uint32_t rw[2][4];
+  auto load_r = [&](int chunk) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int rq = tid & 7, col4 = (tid >> 3) + u * (kLstmThreads / 8);
+      const uint32_t col = static_cast<uint32_t>(min(4 * col4, G4 - 4));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int k = chunk * 32 + 4 * rq + e;
+        const uint32_t word = *reinterpret_cast<const uint32_t*>(
+            R + (static_cast<uint32_t>(min(k, H - 1)) * static_cast<uint32_t>(G4) + col));
+        rw[u][e] = k < H && 4 * col4 < G4 ? word : 0u;
+      }
+    }
+  };
+  load_r(0);
 #pragma unroll
   for (int chunk = 0; chunk < kLstmMaxH / 32; ++chunk) {
-    __syncthreads();
-    for (int idx = tid; idx < 32 * kLstmThreads / 4; idx += kLstmThreads) {
-      const int row = idx / (kLstmThreads / 4), col4 = idx % (kLstmThreads / 4);
-      const int k = chunk * 32 + row;
-      int word = 0;
-      if (k < H && 4 * col4 < G4)
-        word = *reinterpret_cast<const int*>(R + static_cast<int64_t>(k) * G4 + 4 * col4);
-      reinterpret_cast<int*>(rbuf[row])[col4] = word;
+    if (chunk > 0) lds_barrier();  // the previous chunk's fragments are read
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int rq = tid & 7, col4 = (tid >> 3) + u * (kLstmThreads / 8);
+      const uint32_t t01l = __builtin_amdgcn_perm(rw[u][1], rw[u][0], 0x05010400u);
+      const uint32_t t01h = __builtin_amdgcn_perm(rw[u][1], rw[u][0], 0x07030602u);
+      const uint32_t t23l = __builtin_amdgcn_perm(rw[u][3], rw[u][2], 0x05010400u);
+      const uint32_t t23h = __builtin_amdgcn_perm(rw[u][3], rw[u][2], 0x07030602u);
+      uint32_t* dst = reinterpret_cast<uint32_t*>(big + 4 * col4 * kRPitch + 4 * rq);
+      dst[0] = __builtin_amdgcn_perm(t23l, t01l, 0x05040100u);
+      dst[kRPitch / 4] = __builtin_amdgcn_perm(t23l, t01l, 0x07060302u);
+      dst[2 * kRPitch / 4] = __builtin_amdgcn_perm(t23h, t01h, 0x05040100u);
+      dst[3 * kRPitch / 4] = __builtin_amdgcn_perm(t23h, t01h, 0x07060302u);
     }
-    __syncthreads();
+    if (chunk + 1 < kLstmMaxH / 32) load_r(chunk + 1);
+    lds_barrier();
     const int ks = chunk / 2;                // 64-row MFMA k-step (constant once unrolled)
     const int g = lane >> 4;                 // this lane's 16 rows: ks*64 + 16g ..
     if ((g >> 1) == (chunk & 1)) {
-      const int r0 = 16 * (g & 1);           // their offset inside the chunk
 #pragma unroll
       for (int ct = 0; ct < 4; ++ct) {
         const int j = (4 * wv + ct) * 16 + (lane & 15);
-        int w[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          uint32_t word = 0;
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            word |= static_cast<uint32_t>(static_cast<uint8_t>(rbuf[r0 + 4 * q + e][j])) << (8 * e);
-          w[q] = static_cast<int>(word);
-        }
+        const lstm_v4i w = *reinterpret_cast<const lstm_v4i*>(big + j * kRPitch + 16 * (g & 1));
 #pragma unroll
         for (int q = 0; q < 4; ++q) bf[ct][ks >> 1][4 * (ks & 1) + q] = w[q];
       }
     }
   }
+  // this lane's column of the gates, and its bias (-0 leaves xw as it is)
+  const int jcol = 64 * wv + lane;
+  float bias = -0.0f;
+  if (A.b && jcol < G4) bias = A.b[d * 2 * G4 + jcol] + A.b[d * 2 * G4 + G4 + jcol];
   float h = 0.0f, c = 0.0f;
   if (tid < H) {
     h = A.init_h ? A.init_h[(d * A.batch + b) * H + tid] : 0.0f;
@@ -424,6 +466,7 @@ __global__ void __launch_bounds__(kLstmThreads) lstm_recurrence(LstmArgs A) {
     put_chunk(0, load_chunk(0));
     pf = load_chunk(1);  // in flight through chunk 0
   }
+  double hscale = ldexp(1.0, -shift);  // block-uniform, exact (so are its products below)
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): nothing loaded before the loop stays pending in it
   for (int step = 0; step < seq; ++step) {
     const int s = step % kLstmChunk, kc = step / kLstmChunk;
@@ -445,16 +488,16 @@ __global__ void __launch_bounds__(kLstmThreads) lstm_recurrence(LstmArgs A) {
       const int hp = (tid >> 1) & 1, hpos = ((tid >> 2) << 1) | (tid & 1);
 #pragma unroll
       for (int i = 0; i < 4; ++i) hd[i][hp][hpos] = static_cast<int8_t>(dd >> (8 * i));
-      if (rz != 0) {
-        long long sum = v0;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-        if (lane == 0) wsum[wv] = sum;
+      if (rz != 0) {  // v0 = 2^15 (v0 >> 15) + (v0 & 32767): both sums fit 32 bits
+        const int sh = wave_isum63(v0 >> 15), sl = wave_isum63(v0 & 32767);
+        if (lane == 63)
+          wsum[wv] = __builtin_fma(static_cast<double>(sh), 32768.0, static_cast<double>(sl));
       }
     }
     lds_barrier();
     if (s == 0 && step > 0) flush_chunk(kc - 1);  // hring is rewritten after the next barrier
-    const long long hsum = rz != 0 ? (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]) : 0;
+    // (wb + rb) + x @ deq(W) of this lane's column
+    const float xb = xs[((kc & 1) * kLstmChunk + s) * G4 + (jcol < G4 ? jcol : 0)] + bias;
     // (c) gates, on the sparse int8 matrix cores: v_smfmac_i32_16x16x128_i8
     // takes A as 2-of-4 structured (per group of four k, two values and
     // their positions) against a dense 128-k slice of R, twice the k of the
@@ -467,7 +510,10 @@ __global__ void __launch_bounds__(kLstmThreads) lstm_recurrence(LstmArgs A) {
     // holds rows 4q .. 4q+3: digits 0 and 1 (even q) or 2 and 3 (odd q), each
     // as its two parities.  Lane l takes tile l / 16, i.e. column 64 wv + l;
     // the other half of its column's digit sums comes from lane l ^ 16
-    // (v_permlane16_swap), and the four recombine exactly in int64.
+    // (v_permlane16_swap of two tiles' sums), and the four recombine exactly
+    // in double: |dot| < 2^46, times a power of two, less the zero point's
+    // share (2^7 * 2^38 at most) -- integer arithmetic in 64 bits took twice
+    // the instructions, and four waves share each SIMD's issue.
     lstm_v4i acc[4] = {};
     {
       const int idx = (lane & 1) ? static_cast<int>(0xEEEEEEEEu) : 0x44444444;  // positions (2, 3) / (0, 1)
@@ -487,23 +533,24 @@ __global__ void __launch_bounds__(kLstmThreads) lstm_recurrence(LstmArgs A) {
       int fa[4];
 #pragma unroll
       for (int ct = 0; ct < 4; ++ct) fa[ct] = (acc[ct][0] + acc[ct][1]) + ((acc[ct][2] + acc[ct][3]) << 8);
-      const int own = q == 0 ? fa[0] : (q == 1 ? fa[1] : (q == 2 ? fa[2] : fa[3]));
-      const int send = q == 0 ? fa[1] : (q == 1 ? fa[0] : (q == 2 ? fa[3] : fa[2]));
-      // each lane keeps its own value in one of the two results and gets its
-      // partner's in the other
-      const auto pr = __builtin_amdgcn_permlane16_swap(send, send, false, false);
-      const int recv = static_cast<int>(static_cast<unsigned>(pr[0]) + static_cast<unsigned>(pr[1]) -
-                                        static_cast<unsigned>(send));
-      const int lo = (q & 1) ? recv : own, hi = (q & 1) ? own : recv;
-      const int j = 64 * wv + lane;
-        if (j < G4) {
-        const long long dot = static_cast<long long>(lo) + (static_cast<long long>(hi) << 16);
-        const float hr = static_cast<float>(ldexp(static_cast<double>(dot - rz * hsum), -shift));
-        const float pre = xs[((kc & 1) * kLstmChunk + s) * G4 + j] + hr * rs;  // (xw + (wb + rb)) + h @ deq(R)
+      // lane groups q = 0, 1 (tiles 0, 1) of the first result and 2, 3 of the
+      // second hold their own tile's digits 0-1 in [0] and 2-3 in [1]
+      const auto p01 = __builtin_amdgcn_permlane16_swap(fa[0], fa[1], false, false);
+      const auto p23 = __builtin_amdgcn_permlane16_swap(fa[2], fa[3], false, false);
+      const int lo = static_cast<int>(q < 2 ? p01[0] : p23[0]);
+      const int hi = static_cast<int>(q < 2 ? p01[1] : p23[1]);
+      const int j = jcol;
+      if (j < G4) {
+        double dot = __builtin_fma(static_cast<double>(hi), hscale * 65536.0,
+                                   static_cast<double>(lo) * hscale);
+        if (rz != 0)
+          dot = __builtin_fma((wsum[0] + wsum[1]) + (wsum[2] + wsum[3]), -rz * hscale, dot);
+        const float hr = static_cast<float>(dot);
+        const float pre = xb + hr * rs;  // (xw + (wb + rb)) + h @ deq(R)
         // (libm's expf and tanhf and the IEEE division: the 84-second
         // utterance's F0 curve feeds a running phase, whose end moves
         // visibly with a few-ulp change here)
-        gs[j] = j < 3 * H ? 1.0f / (1.0f + expf(-pre)) : tanhf(pre);  // i, o, f: sigmoid; c: tanh
+        gs[j] = j < 3 * H ? recip_from_one(1.0f + expf(-pre)) : tanhf(pre);  // i, o, f: sigmoid; c: tanh
       }
     }
     lds_barrier();
@@ -520,6 +567,7 @@ __global__ void __launch_bounds__(kLstmThreads) lstm_recurrence(LstmArgs A) {
       pf = load_chunk(kc + 2);
     }
     shift = 30;  // from now on |h| = |o tanh(c)| <= 1
+    hscale = 0x1p-30;
   }
   __syncthreads();
   if (seq > 0) flush_chunk((seq - 1) / kLstmChunk);
@@ -836,13 +884,13 @@ int kk_lstm(const kk_tensor* ys, const kk_tensor* yh, const kk_tensor* yc, const
       KK_TRY(f32_contig(t, "state"));
       if (numel(t) != ndir * batch * H) return set_error(KK_E_ARG, "kk_lstm: state shape");
     }
-  // Input projections xw[d] = x @ deq(W[d]) + (wb[d] + rb[d]) on the MFMA
-  // GEMM and two elementwise adds (the biases summed first, as op_lstm does).
+  // Input projections xw[d] = x @ deq(W[d]) on the MFMA GEMM; the recurrence
+  // adds wb[d] + rb[d] (summed first, as op_lstm does) to each step's row as
+  // it reads it, which two elementwise passes a direction did before.
   void* xw = nullptr;
   const int64_t xw_n = ndir * seq * batch * 4 * H;
   const int64_t xw_bytes = ((sizeof(float) * std::max<int64_t>(xw_n, 1) + 255) / 256) * 256;
-  KK_TRY(kk_alloc(static_cast<size_t>(xw_bytes + sizeof(float) * 4 * H), &xw));
-  float* bsum = reinterpret_cast<float*>(static_cast<char*>(xw) + xw_bytes);
+  KK_TRY(kk_alloc(static_cast<size_t>(xw_bytes), &xw));
   int rc = KK_OK;
   for (int64_t d = 0; d < ndir && rc == KK_OK && seq * batch > 0; ++d) {
     kk_tensor a{}, wd{}, o{}, sc{}, zpt{};
@@ -863,27 +911,11 @@ int kk_lstm(const kk_tensor* ys, const kk_tensor* yh, const kk_tensor* yc, const
     // the recurrence amplifies the projection's rounding: keep numpy's
     // (each dequantised weight rounded to fp32, exact fp32 products)
     rc = gemm(&o, &a, &wd, &sc, zptr, 1.0f, true);
-    if (rc == KK_OK && b) {
-      kk_tensor wb{}, rb{}, bs{};
-      for (kk_tensor* t : {&wb, &rb, &bs}) {
-        t->dtype = KK_F32; t->rank = 2; t->shape[0] = 1; t->shape[1] = 4 * H;
-        t->strides[0] = 4 * H; t->strides[1] = 1;
-      }
-      wb.data = static_cast<float*>(b->data) + d * 8 * H;
-      rb.data = static_cast<float*>(b->data) + d * 8 * H + 4 * H;
-      bs.data = bsum;
-      rc = kk_binary(KK_OP_ADD, &bs, &wb, &rb);
-      if (rc == KK_OK) {
-        bs.shape[0] = 1;
-        bs.strides[0] = 0;  // broadcast over the rows of xw[d]
-        bs.shape[0] = seq * batch;
-        rc = kk_binary(KK_OP_ADD, &o, &o, &bs);
-      }
-    }
   }
   if (rc == KK_OK) {
     LstmArgs A{};
     A.xw = static_cast<const float*>(xw);
+    A.b = b ? static_cast<const float*>(b->data) : nullptr;
     A.r = static_cast<const int8_t*>(r->data);
     A.r_scale = r_scale->data; A.r_scale_dt = r_scale->dtype; A.r_scale_n = nrs;
     if (r_zp) { A.r_zp = r_zp->data; A.r_zp_dt = r_zp->dtype; A.r_zp_n = numel(r_zp); }

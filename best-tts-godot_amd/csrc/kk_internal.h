@@ -188,6 +188,8 @@ __device__ __forceinline__ float wave_max_dpp(float v) {
 // ordinary write-back stores measured 3-5x slower on MI355X than the same
 // pattern with non-temporal stores.
 typedef float kk_f4v __attribute__((ext_vector_type(4)));
+// four floats at any float's address (one 16-byte load or store)
+typedef float kk_f4u __attribute__((ext_vector_type(4), aligned(4)));
 __device__ __forceinline__ float4 ld_stream4(const float* p) {
   const kk_f4v v = __builtin_nontemporal_load(reinterpret_cast<const kk_f4v*>(p));
   return make_float4(v.x, v.y, v.z, v.w);
@@ -456,5 +458,13 @@ inline int check_xcd_grid(const dim3& g, const char* who) {
 int zp_shift(Dequant* d, const kk_tensor* zp, int64_t count, const char* who);
 
 
+
+// A workgroup barrier that orders LDS only: global loads and stores stay
+// in flight across it, where __syncthreads would wait for them.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 
 }  // namespace kk

@@ -363,6 +363,30 @@ def test_lstm(gpu, oracle, seq, inp, init):
         assert_close(g, wv, 1e-4, floor_rel=1e-5, what=f"LSTM {name} seq={seq}")
 
 
+@pytest.mark.parametrize("H,seq,batch,bias,zp", [(1, 3, 1, True, 5), (17, 9, 2, False, -3),
+                                                 (64, 6, 1, True, 0), (100, 5, 3, True, 127),
+                                                 (255, 11, 1, False, -128)])
+def test_lstm_hidden_sizes(gpu, oracle, H, seq, batch, bias, zp):
+    """Hidden sizes that fill part of a 32-row chunk, a wave or a tile, with
+    and without a bias, and the zero point's share at its extremes."""
+    r = rng(41)
+    inp = 24
+    x = r.normal(0, 1, (seq, batch, inp)).astype(np.float32)
+    w = r.integers(-127, 128, (2, inp, 4 * H)).astype(np.int8)
+    rr = r.integers(-127, 128, (2, H, 4 * H)).astype(np.int8)
+    b = r.normal(0, 0.5, (2, 8 * H)).astype(np.float32) if bias else None
+    h0 = r.normal(0, 0.5, (2, batch, H)).astype(np.float32)
+    c0 = r.normal(0, 1, (2, batch, H)).astype(np.float32)
+    ws = r.uniform(0.002, 0.006, 2).astype(np.float32)
+    rs = r.uniform(0.0005, 0.001, 2).astype(np.float32)
+    ins = [x, w, rr, b, None, h0, c0, None, ws, np.array([0, 1], np.int8), rs, np.array([zp, 0], np.int8)]
+    at = {"hidden_size": H, "direction": "bidirectional"}
+    got = node(gpu, "DynamicQuantizeLSTM", ins, at, nout=3)
+    want = onode(oracle, "DynamicQuantizeLSTM", ins, at, nout=3)
+    for g, wv, name in zip(got, want, ("Y", "Y_h", "Y_c")):
+        assert_close(g, wv, 1e-4, floor_rel=1e-5, what=f"LSTM {name} H={H}")
+
+
 @pytest.mark.parametrize("batch,slen,n,step,onesided", [(1, 3005, 20, 5, 1), (2, 999, 16, 3, 0),
                                                          (1, 1400003, 20, 5, 1)])
 def test_stft(gpu, oracle, batch, slen, n, step, onesided):
