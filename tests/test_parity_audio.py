@@ -42,6 +42,33 @@ def test_fir(gpu, oracle, n, t, c):
     assert (err <= bound).all(), f"max err/bound {float((err / bound).max()):.3g}"
 
 
+@pytest.mark.parametrize("n,t,c", [
+    (1, 256, -1), (1023, 256, 0), (1024, 257, 64), (1027, 271, 5), (5000, 1536, 1535), (5000, 1537, 3),
+    (3 * 1024 + 2, 993, 0), (5000, 255, 7), (1500001, 300, 11), (171 * 8192 + 5, 1024, 1023)])
+def test_fir_matrix_core_tiles(gpu, oracle, n, t, c):
+    """The matrix-core FIR at the edges of its tiles, of its sum's steps and
+    of its range of taps, the bar as above; and a window's infinity, NaN or
+    sample above bf16's largest reaches the outputs that read it, no other."""
+    r = rng(43)
+    x = r.normal(0, 0.3, n).astype(np.float32)
+    h = r.normal(0, 0.1, t).astype(np.float32)
+    cc = (t - 1) // 2 if c < 0 else c
+    for special in (None, np.inf, np.nan, np.float32(3.4e38)):
+        if special is not None:
+            if n > 10000 or not 256 <= t <= 1536:  # (the other kernel pads its last taps)
+                break
+            x[n // 2] = special
+        got = gpu.ops.fir(gpu.to_device(x), gpu.to_device(h), c).numpy()
+        with np.errstate(all="ignore"):
+            want = oracle.fir(x, h, cc)
+            bound = 4e-6 * fir_bound(np.where(np.isfinite(x), x, 0), h, cc) + 1e-30
+        fin = np.isfinite(want)
+        np.testing.assert_array_equal(np.isnan(got[~fin]), np.isnan(want[~fin]))
+        np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)])
+        err = np.abs(got[fin].astype(np.float64) - want[fin])
+        assert (err <= bound[fin]).all(), f"{special}: max err/bound {float((err / bound[fin]).max()):.3g}"
+
+
 def test_fir_notch_removes_the_hop_tones(gpu, oracle):
     """A waveform carrying the iSTFT's 4800 / 9600 Hz ring: the device filter
     takes both tones down by at least 40 dB and leaves a 1 kHz tone within
