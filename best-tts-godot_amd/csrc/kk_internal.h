@@ -286,11 +286,7 @@ __device__ __forceinline__ float kk_sin(float t) {
 // so the odd-k negation, the signed-zero return and k's -0 -> +0 are not
 // needed (they only change the sign of the sine: +-s and +-0 square to the
 // same bits).
-__device__ __forceinline__ float kk_sin_sq(float t) {
-  if (!(fabsf(t) <= 1.0e5f)) {
-    const float s = sinf(t);
-    return s * s;
-  }
+__device__ __forceinline__ float kk_sin_sq_small(float t) {  // |t| <= 1e5
   const float k = rintf(t * 0x1.45f306p-2f);
   float r = __builtin_fmaf(-k, 0x1.921fb6p+1f, t);
   r = __builtin_fmaf(-k, -0x1.777a5cp-24f, r);
@@ -304,6 +300,13 @@ __device__ __forceinline__ float kk_sin_sq(float t) {
   p = __builtin_fmaf(p, r2, -0x1.555556p-3f);
   const float s = __builtin_fmaf(r2 * r, p, r);
   return s * s;
+}
+__device__ __forceinline__ float kk_sin_sq(float t) {
+  if (!(fabsf(t) <= 1.0e5f)) {
+    const float s = sinf(t);
+    return s * s;
+  }
+  return kk_sin_sq_small(t);
 }
 
 // exp(x) for x <= 0 (softmax's x - max): 2^(x log2 e) on the hardware
@@ -346,28 +349,53 @@ __device__ __forceinline__ float kk_div(float a, const KkDivisor& d) {
   if (!(static_cast<int>(d.rb != 0.0f) & kk_div_in_range(a))) q = a / d.b;
   return q;
 }
-// Four quotients; the divisions run only where one of the four is out of range.
+// The largest and smallest magnitude of four (a NaN among other values is
+// passed over: the fast forms below give NaN for it, as the slow ones do).
+__device__ __forceinline__ float kk_max_abs4(float4 a) {
+  return fmaxf(fmaxf(fmaxf(__builtin_fabsf(a.x), __builtin_fabsf(a.y)), __builtin_fabsf(a.z)),
+               __builtin_fabsf(a.w));
+}
+__device__ __forceinline__ float kk_min_abs4(float4 a) {
+  return fminf(fminf(fminf(__builtin_fabsf(a.x), __builtin_fabsf(a.y)), __builtin_fabsf(a.z)),
+               __builtin_fabsf(a.w));
+}
+// Four quotients; the divisions run only where one of the four is out of
+// range (one test of their largest and smallest magnitudes).
 __device__ __forceinline__ float4 kk_div4(float4 a, const KkDivisor& d) {
   float4 q = make_float4(kk_div_fast(a.x, d), kk_div_fast(a.y, d), kk_div_fast(a.z, d),
                          kk_div_fast(a.w, d));
-  const int ok = static_cast<int>(d.rb != 0.0f) & kk_div_in_range(a.x) & kk_div_in_range(a.y) &
-                 kk_div_in_range(a.z) & kk_div_in_range(a.w);
+  const int ok = static_cast<int>(d.rb != 0.0f) & static_cast<int>(kk_max_abs4(a) < 0x1p60f) &
+                 static_cast<int>(kk_min_abs4(a) > 0x1p-60f);
   if (!ok) q = make_float4(a.x / d.b, a.y / d.b, a.z / d.b, a.w / d.b);
   return q;
 }
-
-// DynamicQuantizeLinear's bytes of four values, dql_byte's rounding with
-// the quotients x / scale formed by kk_div4 (the same bits), packed
-// little-endian.
-__device__ __forceinline__ uint32_t dql_byte_of_quotient(float q, float z) {
-  float v = rintf(q) + z;
-  v = v < 0.0f ? 0.0f : (v > 255.0f ? 255.0f : v);
-  return static_cast<uint32_t>(v);
+// kk_sin_sq of four arguments, one range test for them.
+__device__ __forceinline__ float4 kk_sin_sq4(float4 t) {
+  if (!(kk_max_abs4(t) <= 1.0e5f))
+    return make_float4(kk_sin_sq(t.x), kk_sin_sq(t.y), kk_sin_sq(t.z), kk_sin_sq(t.w));
+  return make_float4(kk_sin_sq_small(t.x), kk_sin_sq_small(t.y), kk_sin_sq_small(t.z),
+                     kk_sin_sq_small(t.w));
 }
+
+// DynamicQuantizeLinear's bytes of four values, dql_byte's bits, packed
+// little-endian.  rint(x / scale) is rint(x * (1 / scale)) unless that
+// product lies within 1e-4 of a half: the product is within 2^-22.4 of the
+// rounded quotient, so below 512 within 9.2e-5, and above it both saturate
+// (the zero point is at most 255).  The quotients themselves are formed only
+// then, once in 20 waves.  v_cvt_pk_u8_f32 saturates (NaN gives 0) and puts
+// the byte in its place.
 __device__ __forceinline__ uint32_t dql_bytes4(float4 x, const KkDivisor& sc, float z) {
-  const float4 q = kk_div4(x, sc);
-  return dql_byte_of_quotient(q.x, z) | (dql_byte_of_quotient(q.y, z) << 8) |
-         (dql_byte_of_quotient(q.z, z) << 16) | (dql_byte_of_quotient(q.w, z) << 24);
+  const float4 p = make_float4(x.x * sc.rb, x.y * sc.rb, x.z * sc.rb, x.w * sc.rb);
+  float4 k = make_float4(rintf(p.x), rintf(p.y), rintf(p.z), rintf(p.w));
+  const float4 d = make_float4(p.x - k.x, p.y - k.y, p.z - k.z, p.w - k.w);
+  if (!(static_cast<int>(sc.rb != 0.0f) & static_cast<int>(kk_max_abs4(d) < 0.4999f))) {
+    const float4 q = kk_div4(x, sc);
+    k = make_float4(rintf(q.x), rintf(q.y), rintf(q.z), rintf(q.w));
+  }
+  uint32_t w = __builtin_amdgcn_cvt_pk_u8_f32(k.x + z, 0, 0);
+  w = __builtin_amdgcn_cvt_pk_u8_f32(k.y + z, 1, w);
+  w = __builtin_amdgcn_cvt_pk_u8_f32(k.z + z, 2, w);
+  return __builtin_amdgcn_cvt_pk_u8_f32(k.w + z, 3, w);
 }
 
 // Runs f(integral_constant<U>, t + U) for U = 0 .. R - 1 while t + U < end:

@@ -243,6 +243,21 @@ __device__ __forceinline__ float apply_affine(float q, const RowAffine& ra, cons
   return y;
 }
 
+// The same of four values, the snake's range tested once for the four.
+template <bool SNAKE = true>
+__device__ __forceinline__ float4 apply_affine4(float4 q, const RowAffine& ra, const Affine& af) {
+  if (ra.has_mul) q = make_float4(q.x * ra.mul, q.y * ra.mul, q.z * ra.mul, q.w * ra.mul);
+  if (ra.has_add) q = make_float4(q.x + ra.add, q.y + ra.add, q.z + ra.add, q.w + ra.add);
+  if (af.leaky)
+    q = make_float4(q.x < 0.0f ? q.x * af.alpha : q.x, q.y < 0.0f ? q.y * af.alpha : q.y,
+                    q.z < 0.0f ? q.z * af.alpha : q.z, q.w < 0.0f ? q.w * af.alpha : q.w);
+  if (SNAKE && af.snake_a) {
+    const float4 s = kk_sin_sq4(make_float4(ra.sa * q.x, ra.sa * q.y, ra.sa * q.z, ra.sa * q.w));
+    q = make_float4(q.x + ra.sr * s.x, q.y + ra.sr * s.y, q.z + ra.sr * s.z, q.w + ra.sr * s.w);
+  }
+  return q;
+}
+
 template <int GROUP, int NV, int VEC>
 __global__ void __launch_bounds__(kRowBlock) instnorm_kernel(float* __restrict__ out,
                                                              const float* __restrict__ x,
@@ -542,8 +557,7 @@ __global__ void __launch_bounds__(kRowBlock) instnorm_apply(float* __restrict__ 
       const int64_t i = rsp.hh + 4 * k;
       const float4 v = *reinterpret_cast<const float4*>(xr + i);
       const float4 q = kk_div4(make_float4(v.x - st.x, v.y - st.x, v.z - st.x, v.w - st.x), dden);
-      st_stream4(orow + i, make_float4(apply_affine(q.x, ra, af), apply_affine(q.y, ra, af),
-                                       apply_affine(q.z, ra, af), apply_affine(q.w, ra, af)));
+      st_stream4(orow + i, apply_affine4(q, ra, af));
     }
     int64_t i;
     if (rsp.edge(i))
@@ -555,7 +569,9 @@ __global__ void __launch_bounds__(kRowBlock) instnorm_apply(float* __restrict__ 
 }
 
 // y recomputed exactly as above, then DynamicQuantizeLinear's byte: the
-// float y never reaches memory.  The scale and zero point come from the
+// float y never reaches memory.  Bound by VALU issue on the snake (~35
+// instructions a value: the norm's division and the snake's sine tested four
+// values at a time, the bytes from dql_bytes4).  The scale and zero point come from the
 // npart (min, max) partials in mm, which every block folds (min and max do
 // not depend on the order, so every block finds the same; block (0, 0)
 // stores them: no fold launch), or with mm NULL from params[0] (dql_fold's
@@ -631,13 +647,10 @@ __global__ void __launch_bounds__(kRowBlock) instnorm_quant(uint8_t* __restrict_
       const int64_t i = rsp.hh + 4 * k;
       const float4 v = *reinterpret_cast<const float4*>(xr + i);  // cached: as instnorm_apply
       const float4 q = kk_div4(make_float4(v.x - st.x, v.y - st.x, v.z - st.x, v.w - st.x), dden);
-      const float y0 = apply_affine(q.x, ra, af);
-      const float y1 = apply_affine(q.y, ra, af);
-      const float y2 = apply_affine(q.z, ra, af);
-      const float y3 = apply_affine(q.w, ra, af);
-      lo = fminf(lo, fminf(fminf(y0, y1), fminf(y2, y3)));
-      hi = fmaxf(hi, fmaxf(fmaxf(y0, y1), fmaxf(y2, y3)));
-      const uint32_t w = dql_bytes4(make_float4(y0, y1, y2, y3), dsc, pz.y);
+      const float4 y = apply_affine4(q, ra, af);
+      lo = fminf(fminf(fminf(fminf(lo, y.x), y.y), y.z), y.w);
+      hi = fmaxf(fmaxf(fmaxf(fmaxf(hi, y.x), y.y), y.z), y.w);
+      const uint32_t w = dql_bytes4(y, dsc, pz.y);
       // an ordinary store: the convolution that reads the bytes next finds
       // them in the last-level cache
       *reinterpret_cast<uint32_t*>(qr + i) = w;
@@ -1201,8 +1214,15 @@ __global__ void __launch_bounds__(kNpThreads) np_rows_kernel(float* __restrict__
   const KkDivisor dden = kk_divisor(den);
   if (mode == 3) {  // no output: (mean, den) and the (min, max) of the row's results
     float lo = INFINITY, hi = -INFINITY;
-    for (int e = threadIdx.x; e < n; e += kNpThreads) {
-      const float y = apply_affine(kk_div(np_lds[np_pad(e)] - mean, dden), ra, af);
+    for (int e = 4 * threadIdx.x; e + 4 <= n; e += 4 * kNpThreads) {
+      const float4 v = *reinterpret_cast<const float4*>(np_lds + np_pad(e));
+      const float4 y = apply_affine4(
+          kk_div4(make_float4(v.x - mean, v.y - mean, v.z - mean, v.w - mean), dden), ra, af);
+      lo = fminf(fminf(fminf(fminf(lo, y.x), y.y), y.z), y.w);
+      hi = fmaxf(fmaxf(fmaxf(fmaxf(hi, y.x), y.y), y.z), y.w);
+    }
+    if (static_cast<int>(threadIdx.x) < n % 4) {
+      const float y = apply_affine(kk_div(np_lds[np_pad(n - n % 4 + threadIdx.x)] - mean, dden), ra, af);
       lo = fminf(lo, y);
       hi = fmaxf(hi, y);
     }
@@ -1229,8 +1249,7 @@ __global__ void __launch_bounds__(kNpThreads) np_rows_kernel(float* __restrict__
     for (int e = 4 * threadIdx.x; e < n; e += 4 * kNpThreads) {
       const float4 v = *reinterpret_cast<const float4*>(np_lds + np_pad(e));
       const float4 q = kk_div4(make_float4(v.x - mean, v.y - mean, v.z - mean, v.w - mean), dden);
-      st_stream4(orow + e, make_float4(apply_affine(q.x, ra, af), apply_affine(q.y, ra, af),
-                                       apply_affine(q.z, ra, af), apply_affine(q.w, ra, af)));
+      st_stream4(orow + e, apply_affine4(q, ra, af));
     }
   } else {
     for (int e = threadIdx.x; e < n; e += kNpThreads)
@@ -1478,7 +1497,7 @@ struct ResArgs {
 };
 
 // Instance norm over rows of NB whole 8192-blocks and a partial one
-// (15000 < T < 9 * 8192, T % 4 == 0; the decoder's [1,256,71800]), one
+// (15000 < T < 9 * 8192, for MODE 0 with T % 4 == 0; the decoder's [1,256,71800]), one
 // workgroup of 128 NB threads per row, x read once.  Wave w holds the 4096
 // floats (32 numpy leaves of 128) from 8192 (w / 2) + 4096 (w % 2) as
 // sixteen float4s a lane in load order, k = 0..15 at 256 k + 4 lane: each
@@ -1533,8 +1552,12 @@ __global__ void __launch_bounds__(128 * NB) np_resident_kernel(ResArgs A) {
   // the partial block (buffer loads: past m they return zeros), the tree
   // plan, then the sixteen whole-block vectors
   const float* xt = xr + NB * kNpBlock;
-  const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(xt), 0, 4 * m, 0x00020000);
+  // (its whole float4s, then the m % 4 last elements)
+  const int m4 = m & ~3;
+  const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(xt), 0, 4 * m4, 0x00020000);
+  const auto rend = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(xt), 0, 4 * m, 0x00020000);
   float4 u[TPT];
+  const float ue = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rend, 4 * (m4 + (t & 3)), 0, 0));
 #pragma unroll
   for (int i = 0; i < TPT; ++i) {
     const kk_f4v r = __builtin_bit_cast(
@@ -1557,18 +1580,24 @@ __global__ void __launch_bounds__(128 * NB) np_resident_kernel(ResArgs A) {
   float v[64];
 #pragma unroll
   for (int k = 0; k < 16; ++k) {
-    const float4 e = MODE == 2 ? *reinterpret_cast<const float4*>(xr + wbase + 256 * k)
-                               : ld_stream4(xr + wbase + 256 * k);
-    v[4 * k] = e.x;
-    v[4 * k + 1] = e.y;
-    v[4 * k + 2] = e.z;
-    v[4 * k + 3] = e.w;
+    if constexpr (MODE == 2) {  // rows of any length: four floats at any float's address
+      const kk_f4u e = *reinterpret_cast<const kk_f4u*>(xr + wbase + 256 * k);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[4 * k + q] = e[q];
+    } else {
+      const float4 e = ld_stream4(xr + wbase + 256 * k);
+      v[4 * k] = e.x;
+      v[4 * k + 1] = e.y;
+      v[4 * k + 2] = e.z;
+      v[4 * k + 3] = e.w;
+    }
   }
 #pragma unroll
   for (int i = 0; i < TPT; ++i) {
     const int e = 4 * (t + i * NT);
-    if (e < m) *reinterpret_cast<float4*>(res_tail + np_pad(e)) = u[i];
+    if (e < m4) *reinterpret_cast<float4*>(res_tail + np_pad(e)) = u[i];
   }
+  if (t < m - m4) res_tail[np_pad(m4 + t)] = ue;
   __syncthreads();
 
   // numpy's sums of f over the partial block's leaves, eight lanes a leaf,
@@ -1743,7 +1772,11 @@ __global__ void __launch_bounds__(128 * NB) np_resident_kernel(ResArgs A) {
       lo = fminf(lo, v[k]);
       hi = fmaxf(hi, v[k]);
     }
-    for (int e = 4 * t; e < m; e += 4 * NT) {
+    if (t < m - m4) {
+      lo = fminf(lo, ue);
+      hi = fmaxf(hi, ue);
+    }
+    for (int e = 4 * t; e < m4; e += 4 * NT) {
       const float4 x4 = *reinterpret_cast<const float4*>(res_tail + np_pad(e));
       lo = fminf(fminf(lo, x4.x), fminf(fminf(x4.y, x4.z), x4.w));
       hi = fmaxf(fmaxf(hi, x4.x), fmaxf(fmaxf(x4.y, x4.z), x4.w));
@@ -2034,9 +2067,10 @@ static int np_reduce_rows(float* out, const float* x, int64_t rows, int64_t n, b
 }
 
 // Rows np_resident_kernel takes: 15000 < T < 9 * 8192 (one to eight whole
-// 8192-blocks and a partial one), T % 4 == 0, x 16-byte aligned.
-static bool np_resident_ok(int64_t T, const void* x) {
-  return T > kNpRowMax && T < 9 * kNpBlock && T % 4 == 0 && aligned16(x);
+// 8192-blocks and a partial one); its MODE 0, whose streaming loads and
+// stores are 16-byte ones, with T % 4 == 0 and x 16-byte aligned.
+static bool np_resident_ok(int64_t T, const void* x, bool writes) {
+  return T > kNpRowMax && T < 9 * kNpBlock && (!writes || (T % 4 == 0 && aligned16(x)));
 }
 
 // out set: writes y (MODE 0; no snake); else stats and mm (MODE 2).
@@ -2102,7 +2136,7 @@ static int instnorm_np(const kk_tensor* out, const kk_tensor* x, int64_t rows, i
                        static_cast<float2*>(nullptr), tail);
     return check_launch("np_rows_kernel");
   }
-  if (np_resident_ok(T, x->data) && aligned16(out->data) && !af.snake_a)
+  if (np_resident_ok(T, x->data, true) && aligned16(out->data) && !af.snake_a)
     return np_resident_launch(static_cast<float*>(out->data), xp, rows, C, T, eps, af, nullptr,
                               nullptr);
   if (rows > kRowCounters)
@@ -2227,7 +2261,7 @@ static int instnorm_quant_run(const kk_tensor* q, const kk_tensor* y_scale, cons
                        np_row_lds(T), st, static_cast<float*>(nullptr), xp, C, static_cast<int>(T), 3,
                        eps, af, rows_vec ? 1 : 0, stats, mm, tail);
     rc = check_launch("np_rows_kernel");
-  } else if (np_resident_ok(T, x->data)) {
+  } else if (np_resident_ok(T, x->data, false)) {
     rc = np_resident_launch(nullptr, xp, rows, C, T, eps, af, stats, mm);
   } else {
     const dim3 bgrid(static_cast<unsigned>(nblk), static_cast<unsigned>(rows));

@@ -427,6 +427,42 @@ def test_instance_norm_quant_matches_unfused_device_path(gpu, C, T, rc_mul, leak
         assert_bitexact(gpu.to_host(got_t), gpu.to_host(want_t), f"{what} C={C} T={T}")
 
 
+@pytest.mark.parametrize("C,T,skip", [(8, 15001, 0), (8, 16385, 1), (6, 24579, 2), (5, 32770, 3),
+                                      (12, 67641, 0), (3, 73727, 1), (3, 40960, 2)])
+def test_instance_norm_quant_resident_rows_of_any_length(gpu, C, T, skip):
+    """Rows held in registers that start `skip` floats off a 16-byte line and
+    end inside a float4: the statistics and extremes of the whole row, as the
+    device's unfused chain gives them."""
+    r = rng(44)
+    x = (r.normal(0, 2, (1, C, T)) + r.normal(0, 3, (1, C, 1))).astype(np.float32)
+    x[0, :, -1] = np.where(np.arange(C) % 2, 40, -40)  # an extreme in the last element
+    g = r.normal(0, 1, (1, C, 1)).astype(np.float32)
+    b = (0.3 * r.normal(0, 1, (1, C, 1))).astype(np.float32)
+    D = gpu.to_device
+    want = gpu.ops.dynamic_quantize_linear(gpu.ops.instance_norm_scale_shift(D(x), D(g), D(b), 1e-5))
+    flat = D(np.concatenate([np.zeros(skip, np.float32), x.ravel()]))
+    dx = flat.slice_axis(0, skip, skip + x.size).reshape(x.shape)
+    got = gpu.ops.instance_norm_quant(dx, D(g), D(b), eps=1e-5)
+    for got_t, want_t, what in zip(got, want, ("bytes", "scale", "zero point")):
+        assert_bitexact(gpu.to_host(got_t), gpu.to_host(want_t), f"{what} C={C} T={T} skip={skip}")
+
+
+@pytest.mark.parametrize("n", [300, 20000])
+def test_dynamic_quantize_near_ties(gpu, oracle, n):
+    """Values whose quotient by the scale is a half, or a few ulps from one:
+    the byte is that of the rounded quotient."""
+    r = rng(45)
+    for span, lo in ((255.0, -1.0), (1.7, -0.6), (3e-5, -1e-5)):
+        k = r.integers(0, 255, n).astype(np.float64) + r.choice([0.5, 0.49995, 0.50005, 0.0], n)
+        x = (lo + span / 255.0 * k).astype(np.float32)
+        x = np.nextafter(x, r.choice(np.array([-np.inf, np.inf], np.float32), n))
+        x[:2] = lo, lo + span
+        got = [gpu.to_host(t) for t in gpu.ops.dynamic_quantize_linear(gpu.to_device(x))]
+        env = {"x": x}
+        oracle.dispatch("DynamicQuantizeLinear", ["x"], ["q", "s", "z"], {}, env)
+        assert_bitexact(got[0], env["q"], f"bytes n={n} span={span}")
+
+
 @pytest.mark.parametrize("C,T,kind", [(128, 40000, "affine"), (256, 7180, "leaky"),
                                       (128, 20000, "snake"), (64, 999, "snake"),
                                       (96, 2400, "plain"), (32, 24676, "leaky"),
