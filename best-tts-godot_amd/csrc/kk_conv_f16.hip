@@ -56,6 +56,7 @@
 #include <climits>
 #include <mutex>
 #include <unordered_map>
+#include <utility>
 
 #include "kk_internal.h"
 
@@ -102,6 +103,7 @@ struct PackArgs {
   int zp_stride;
   int Cin, Cout, Kw, P, T, TP, M, KS;
   int transposed;
+  int tap_major;   // convq_kernel's order: k = tap Cin + ci, bf16
   int64_t units;
 };
 
@@ -121,7 +123,9 @@ __global__ void __launch_bounds__(256) convh_pack(PackArgs A) {
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const int k = 8 * g + e;
-    const int ci = s * (16 / A.TP) + k / A.TP, tp = k % A.TP;
+    const int kk = 16 * s + k;
+    const int ci = A.tap_major ? kk % A.Cin : s * (16 / A.TP) + k / A.TP;
+    const int tp = A.tap_major ? kk / A.Cin : k % A.TP;
     const int tap = A.transposed ? r + A.P * (A.T - 1 - tp) : tp;
     float f = 0.0f;
     if (m < A.M && ci < A.Cin && tp < A.T && tap < A.Kw) {
@@ -129,7 +133,8 @@ __global__ void __launch_bounds__(256) convh_pack(PackArgs A) {
                                        : (static_cast<int64_t>(co) * A.Cin + ci) * A.Kw + tap;
       f = static_cast<float>(w[idx]) - z;
     }
-    v[e] = static_cast<_Float16>(f);
+    if (A.tap_major) v[e] = __builtin_bit_cast(_Float16, static_cast<__bf16>(f));
+    else v[e] = static_cast<_Float16>(f);
   }
   *reinterpret_cast<h8*>(A.wp + u) = v;
 }
@@ -154,9 +159,12 @@ __device__ __forceinline__ int scale_exp(unsigned mbits) {
   return min(120, 10 - e);
 }
 
+// TP = 0: weights laid out for convq_kernel (tap-major bf16), for the strides
+// and dilations whose window that kernel does not hold.
 template <int TP, int MI, int WK, int R>
 __global__ void __launch_bounds__(kThreads) convh_kernel(CArgs A) {
-  constexpr int WN = 4 / WK, CPL = 8 / TP, CPS = 16 / TP;
+  constexpr int NPO = TP ? TP : 1;
+  constexpr int WN = 4 / WK, CPL = 8 / NPO, CPS = 16 / NPO;
   constexpr int BM = 32 * MI, BN = 32 * WN;
   constexpr int RED = WK > 1 ? (WK - 1) * WN * MI * 16 * 64 : 1;
   __shared__ float red[RED];       // [wk - 1][wn][register][lane]: the other waves' partials
@@ -184,9 +192,9 @@ __global__ void __launch_bounds__(kThreads) convh_kernel(CArgs A) {
   // outside the signal, past the columns or past the T taps in use, and a
   // channel's offset 0x80000000 past Cin: any sum with either is past the
   // buffer (below 2^31 bytes), so the load returns 0, and no sum wraps
-  uint32_t po[TP];
+  uint32_t po[NPO];
 #pragma unroll
-  for (int t = 0; t < TP; ++t) {
+  for (int t = 0; t < NPO; ++t) {
     const int p = q * A.qs + A.ta + t * A.tm;
     po[t] = q < A.Nq && t < A.T && p >= 0 && p < L ? static_cast<uint32_t>(4 * p) : 0x7fffffffu;
   }
@@ -213,15 +221,25 @@ __global__ void __launch_bounds__(kThreads) convh_kernel(CArgs A) {
   // and weight fragments; issued whatever s (a read past the buffers
   // returns 0), so every slot's loads count the same for the waits
   auto fetch = [&](int s, float (&v)[8], uint4 (&f)[MI]) {
+    uint32_t pt[NPO];
+    int c_first = s * CPS + g * CPL;  // the slice's first channel of this lane
+    if constexpr (TP == 0) {          // (Cin % 16 == 0: a slice lies in one tap)
+      const int t = 16 * s / Cin, p = q * A.qs + A.ta + t * A.tm;
+      c_first = 16 * s - t * Cin + 8 * g;
+      pt[0] = q < A.Nq && t < A.T && p >= 0 && p < L ? static_cast<uint32_t>(4 * p) : 0x7fffffffu;
+    } else {
+#pragma unroll
+      for (int t = 0; t < TP; ++t) pt[t] = po[t];
+    }
 #pragma unroll
     for (int c = 0; c < CPL; ++c) {
-      const int ci = s * CPS + g * CPL + c;
+      const int ci = c_first + c;
       const uint32_t cofs = ci < Cin ? static_cast<uint32_t>(ci * row_bytes) : 0x80000000u;
 #pragma unroll
-      for (int t = 0; t < TP; ++t) {
-        uint32_t off = cofs + po[t];
+      for (int t = 0; t < NPO; ++t) {
+        uint32_t off = cofs + pt[t];
         asm volatile("" : "+v"(off));  // an unconditional load
-        v[c * TP + t] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, off, 0, 0));
+        v[c * NPO + t] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, off, 0, 0));
       }
     }
     const uint32_t a_s = a_lane + static_cast<uint32_t>(s * 1024);
@@ -274,7 +292,15 @@ __global__ void __launch_bounds__(kThreads) convh_kernel(CArgs A) {
     }
 #pragma unroll
     for (int mi = 0; mi < MI; ++mi) {
-      const h8 a = __builtin_bit_cast(h8, f[mi]);
+      h8 a = __builtin_bit_cast(h8, f[mi]);
+      if constexpr (TP == 0) {  // bf16 -> fp16, exact for these integers
+        const uint32_t w[4] = {f[mi].x, f[mi].y, f[mi].z, f[mi].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          a[2 * e] = static_cast<_Float16>(__uint_as_float(w[e] << 16));
+          a[2 * e + 1] = static_cast<_Float16>(__uint_as_float(w[e] & 0xffff0000u));
+        }
+      }
       acc[mi] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, hi, acc[mi], 0, 0, 0);
       acc[mi] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, lo, acc[mi], 0, 0, 0);
     }
@@ -355,14 +381,280 @@ __global__ void __launch_bounds__(kThreads) convh_kernel(CArgs A) {
         for (int t = 0; t < A.T; ++t) {
           const int p = q * A.qs + A.ta + t * A.tm;
           if (p < 0 || p >= L) continue;
-          const int k = (ci % CPS) * TP + t;
-          const int64_t unit = (static_cast<int64_t>(m / 32) * KS + ci / CPS) * 64 + (m % 32) + 32 * (k / 8);
-          sum = sum + static_cast<float>(wh[unit * 8 + k % 8]) * xb[static_cast<int64_t>(ci) * L + p];
+          const int k = TP ? (ci % CPS) * TP + t : (t * Cin + ci) % 16;
+          const int sl = TP ? ci / CPS : (t * Cin + ci) / 16;
+          const int64_t unit = (static_cast<int64_t>(m / 32) * KS + sl) * 64 + (m % 32) + 32 * (k / 8);
+          const _Float16 wv = wh[unit * 8 + k % 8];
+          const float wf = TP ? static_cast<float>(wv) : static_cast<float>(__builtin_bit_cast(__bf16, wv));
+          sum = sum + wf * xb[static_cast<int64_t>(ci) * L + p];
         }
       const float u = A.scale ? sum * __int_as_float(rv.z) : sum;
       A.out[b * A.Cout * A.Lout + rv.x + pos] = A.bias ? u + __int_as_float(rv.w) : u;
     }
   }
+}
+
+// ------------------------------------- 8-bit weights, channels in 128s
+// The same implicit GEMM on the bf16 matrix cores (v_mfma_f32_32x32x16_bf16):
+// an 8-bit weight less its zero point is exact in bf16, and an activation is
+// split exactly into three bf16 parts by rounding (8 + 8 + 8 significant
+// bits), so three products per weight give exact fp32 products with no
+// scaling (bf16 has fp32's exponents).  The reduction runs tap-major (k =
+// t' Cin + ci): no padded taps, and an operand is eight channels at one time.
+//
+// A block owns 64 rows x 64 columns; its four waves take a quarter of the
+// channels each and own nothing in common until they add their tiles.  A wave
+// stages the time window its columns read, 32 channels at a time, in its own
+// LDS (time-major, the three parts side by side, 208 bytes a row: the 32
+// rows of an operand read start on distinct banks), so a value is loaded and
+// split once a block instead of once a tap and 32 columns -- what bound the
+// kernel above here, with ~60 VALU instructions beside four matrix
+// instructions a slice.  While a chunk is multiplied the next one's values and
+// weight fragments are in flight in registers.  Then each wave keeps one
+// 32 x 32 tile of the 64 x 64 and adds the other waves' in wave order.
+//
+// An output that is not finite (an infinity or NaN in reach, or a sample
+// above bf16's range) is summed again with scalar fp32 products.
+//
+// Bound by each wave's chain (a chunk: window, products) at one or two waves
+// a SIMD.  us, the kernel above -> this one: Conv1d 512 -> 512 k3 over 2400
+// steps 32.7 -> 22.9, over 7000 77 -> 46, over 40 18.8 -> 14.2; 256 -> 256 k3
+// over 2400 15.8 -> 11.2; 512 -> 512 k7 over 7000 135 -> 99; ConvTranspose1d
+// 512 -> 256 k20 s10 over 240 16.5 -> 13.7, over 700 28.9 -> 22.1.  No further
+// from 64 bits (2.0e-7 -> 1.9e-7 relative for the first).
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+constexpr int kQPitch = 208;  // bytes a staged row: three parts of 32 channels, 16 to spare
+constexpr int kQExchange = 4 * 3 * 16 * 64 * 4;  // bytes the waves' tiles take
+
+template <int T, int NP>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(T == 7 ? 1 : 2, 2)))
+convq_kernel(CArgs A, int W) {
+  extern __shared__ __align__(16) unsigned char convq_lds[];
+  __shared__ int4 rows[64];  // output row offset, phase offset, scale, bias
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ln = lane & 31, g = lane >> 5;
+  const uint3 tile = xcd_tile();  // row tiles fastest: a column range's blocks share an XCD
+  const int m0 = __builtin_amdgcn_readfirstlane(static_cast<int>(tile.x)) * 64;
+  const int n0 = __builtin_amdgcn_readfirstlane(static_cast<int>(tile.y)) * 64;
+  const int64_t b = __builtin_amdgcn_readfirstlane(static_cast<int>(tile.z));
+  const int Cin = A.Cin, L = A.L, C16 = Cin / 16;
+  const float* xb = A.x + b * Cin * L;
+  const auto xrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(xb), 0, Cin * L * 4, 0x00020000);
+  const auto wrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(A.wp), 0, A.wbytes, 0x00020000);
+  unsigned char* win = convq_lds + wv * W * kQPitch;
+  if (tid < 64) {
+    const int m = m0 + tid;
+    int4 rv = make_int4(-1, 0, __float_as_int(1.0f), 0);
+    if (m < A.M) {
+      const int co = m / A.P, r = m - co * A.P;
+      rv.x = co * A.Lout;
+      rv.y = r + A.oph;
+      if (A.scale) rv.z = __float_as_int(load_as_f32(A.scale, A.scale_dt, co * A.scale_stride));
+      if (A.bias) rv.w = __float_as_int(A.bias[co]);
+    }
+    rows[tid] = rv;
+  }
+  // item p of a lane: eight channels (octet oct of the chunk) of staged row
+  // rr, at byte offset xo of x; 0x7fffffff off the signal (loads give 0; no
+  // sum with a channel's offset, below 2^31, wraps)
+  uint32_t xo[NP];
+  int dst[NP];
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    const int it = lane + 64 * p, oct = it / W, rr = it - oct * W;
+    const int pos = n0 * A.qs + A.ta + rr;
+    const bool ok = oct < 4;
+    dst[p] = ok ? rr * kQPitch + 16 * oct : -1;
+    xo[p] = ok && pos >= 0 && pos < L ? static_cast<uint32_t>(4 * pos) + static_cast<uint32_t>(32 * oct * L)
+                                      : 0x7fffffffu;
+  }
+  const uint32_t row_bytes = static_cast<uint32_t>(4 * L);
+  const int c_lo = Cin / 128 * wv, c_hi = Cin / 128 * (wv + 1);  // this wave's chunks of 32 channels
+  float v[NP][8];
+  auto load_x = [&](int c) {  // (past the last chunk the loads read 0 or another wave's channels)
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        uint32_t off = xo[p] + static_cast<uint32_t>(32 * c + e) * row_bytes;
+        v[p][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, off, 0, 0));
+      }
+  };
+  // tap t's fragments of chunk c: k-steps 2 c and 2 c + 1 of the tap's C16,
+  // row tiles m0 / 32 and the next
+  const uint32_t a_lane = static_cast<uint32_t>(m0 / 32) * static_cast<uint32_t>(A.KS) * 1024u + 16u * lane;
+  b8 a[T][2][2];
+  auto load_a = [&](int c, auto tc) {
+    constexpr int t = decltype(tc)::value;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int mi = 0; mi < 2; ++mi)
+        a[t][ks][mi] = __builtin_bit_cast(
+            b8, __builtin_amdgcn_raw_buffer_load_b128(
+                    wrs, a_lane + static_cast<uint32_t>((mi * A.KS + t * C16 + 2 * c + ks) * 1024), 0, 0));
+  };
+  f16v acc[2][2] = {};
+  auto each_tap = [&](auto f) {
+    [&]<int... t>(std::integer_sequence<int, t...>) { (f(std::integral_constant<int, t>{}), ...); }
+    (std::make_integer_sequence<int, T>{});
+  };
+  // With few taps registers are left to read an operand ahead and to split
+  // the next chunk's values among the last products (a SIMD has one or two
+  // of these waves: nothing else fills those waits).
+  constexpr bool kDeep = T <= 3 && NP == 5;
+  b8 part[NP][3];
+  auto split = [&](int p) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float x0 = v[p][e];
+      part[p][0][e] = static_cast<__bf16>(x0);
+      const float x1 = x0 - static_cast<float>(part[p][0][e]);
+      part[p][1][e] = static_cast<__bf16>(x1);
+      part[p][2][e] = static_cast<__bf16>(x1 - static_cast<float>(part[p][1][e]));
+    }
+  };
+  b8 x[2][2][3];  // [step % 2][column tile][part]
+  auto read_x = [&](auto step) {  // step: 2 t + ks of the chunk
+    constexpr int t = decltype(step)::value / 2, ks = decltype(step)::value % 2;
+#pragma unroll
+    for (int ni = 0; ni < 2; ++ni)
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        x[ks][ni][k] = *reinterpret_cast<const b8*>(
+            win + ((32 * ni + ln) * A.qs + t * A.tm) * kQPitch + 64 * k + 32 * ks + 16 * g);
+  };
+  auto products = [&](auto step) {
+    constexpr int t = decltype(step)::value / 2, ks = decltype(step)::value % 2;
+#pragma unroll
+    for (int k = 2; k >= 0; --k)
+#pragma unroll
+      for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < 2; ++ni)
+          acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[t][ks][mi], x[ks][ni][k], acc[mi][ni], 0, 0, 0);
+  };
+  auto each_step = [&](auto f) {
+    [&]<int... i>(std::integer_sequence<int, i...>) { (f(std::integral_constant<int, i>{}), ...); }
+    (std::make_integer_sequence<int, 2 * T>{});
+  };
+  load_x(c_lo);
+  each_tap([&](auto t) { load_a(c_lo, t); });
+  if constexpr (kDeep)
+#pragma unroll
+    for (int p = 0; p < NP; ++p) split(p);
+  for (int c = c_lo; c < c_hi; ++c) {
+    // stage this chunk (the wave alone reads and writes its window; its LDS
+    // accesses take effect in order)
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      if constexpr (!kDeep) split(p);
+      if (dst[p] >= 0) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) *reinterpret_cast<b8*>(win + dst[p] + 64 * k) = part[p][k];
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // (sched_barrier: the scheduler would move these loads to the end of the
+    // chunk, where the next one waits for them at once)
+    load_x(c + 1);
+    if constexpr (kDeep) read_x(std::integral_constant<int, 0>{});
+    __builtin_amdgcn_sched_barrier(0);
+    each_step([&](auto sc) {
+      constexpr int i = decltype(sc)::value;
+      if constexpr (!kDeep) read_x(sc);
+      else if constexpr (i + 1 < 2 * T) read_x(std::integral_constant<int, i + 1>{});
+      if constexpr (kDeep) __builtin_amdgcn_sched_barrier(0);
+      products(sc);
+      if constexpr (kDeep && i + 2 >= 2 * T) {
+#pragma unroll
+        for (int p = (i + 1 == 2 * T ? 2 : 0); p < (i + 1 == 2 * T ? NP : 2); ++p) split(p);
+        // one matrix instruction, then VALU work in its shadow
+#pragma unroll
+        for (int k = 0; k < 12; ++k) {
+          __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x2, i + 1 == 2 * T ? 12 : 8, 0);
+        }
+      }
+      if constexpr (i % 2 == 1) load_a(c + 1, std::integral_constant<int, i / 2>{});
+      if constexpr (kDeep || i % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+    });
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  __syncthreads();  // every window is read
+  // wave w keeps tile w = 2 mi + ni; the others' go to LDS ([wave][slot][register][lane])
+  float* red = reinterpret_cast<float*>(convq_lds);
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    if (q != wv)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        red[((wv * 3 + ((q - wv - 1) & 3)) * 16 + r) * 64 + lane] = acc[q >> 1][q & 1][r];
+  f16v own = acc[0][0];
+#pragma unroll
+  for (int q = 1; q < 4; ++q)
+    if (q == wv) own = acc[q >> 1][q & 1];
+  __syncthreads();
+  f16v sum;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    f16v part = own;
+    if (w != wv) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) part[r] = red[((w * 3 + ((wv - w - 1) & 3)) * 16 + r) * 64 + lane];
+    }
+    sum = w == 0 ? part : sum + part;
+  }
+  const int q = n0 + 32 * (wv & 1) + ln;
+  const auto ors = __builtin_amdgcn_make_buffer_rsrc(A.out + b * A.Cout * A.Lout, 0,
+                                                     A.Cout * A.Lout * 4, 0x00020000);
+  const int qpos = q < A.Nq ? q * A.os : INT_MIN / 2;
+#pragma unroll
+  for (int rg = 0; rg < 16; ++rg) {
+    const int ml = 32 * (wv >> 1) + 8 * (rg / 4) + 4 * g + (rg % 4);
+    const int4 rv = rows[ml];
+    const int pos = qpos + rv.y;
+    const bool ok = rv.x >= 0 && pos >= 0 && pos < A.Lout;
+    float s = sum[rg];
+    if (ok && !(fabsf(s) < INFINITY)) {
+      const __bf16* wh = reinterpret_cast<const __bf16*>(A.wp);
+      s = 0.0f;
+      for (int ci = 0; ci < Cin; ++ci)
+        for (int t = 0; t < T; ++t) {
+          const int p = q * A.qs + A.ta + t * A.tm;
+          if (p < 0 || p >= L) continue;
+          const int k = t * Cin + ci, m = m0 + ml;
+          const int64_t unit = (static_cast<int64_t>(m / 32) * A.KS + k / 16) * 64 + (m % 32) + 32 * (k % 16 / 8);
+          s = s + static_cast<float>(wh[unit * 8 + k % 8]) * xb[static_cast<int64_t>(ci) * L + p];
+        }
+    }
+    const uint32_t off = ok ? static_cast<uint32_t>(4 * (rv.x + pos)) : 0x80000000u;
+    const float u = s * __int_as_float(rv.z);
+    const float y = A.bias ? u + __int_as_float(rv.w) : u;
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y), ors, off, 0, 0);
+  }
+}
+
+// Whether 8-bit weights of this geometry are laid out for, and run on,
+// convq_kernel: whole 128-channel rounds for its four waves.
+static bool tap_major(const Geo& g, int w_dt) {
+  return w_dt != KK_F16 && g.Cin % 128 == 0 && g.T <= 7;
+}
+
+template <int T, int NP>
+static int launch_q(const CArgs& a, int W, int64_t batch) {
+  const dim3 grid(static_cast<unsigned>(ceil_div(a.M, 64)), static_cast<unsigned>(ceil_div(a.Nq, 64)),
+                  static_cast<unsigned>(batch));
+  KK_TRY(check_xcd_grid(grid, "convq_kernel"));
+  const int lds = std::max(4 * W * kQPitch, kQExchange);
+  // (a kernel needs the attribute for more than 64 KB of dynamic LDS)
+  KK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(convq_kernel<T, NP>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+  KK_LAUNCH((convq_kernel<T, NP>), grid, dim3(kThreads), static_cast<size_t>(lds), ctx().stream, a, W);
+  return check_launch("convq_kernel");
 }
 
 // The launch shape: MI 32-row tiles a wave, WK waves a column range.
@@ -409,7 +701,31 @@ static int launch_tp(const CArgs& a, const Shape& s, int64_t batch) {
 #undef KK_CONVH_WK
 }
 
+template <int T>
+static int launch_q(const CArgs& a, int W, int64_t batch) {
+  if constexpr (T >= 5) return launch_q<T, 6>(a, W, batch);
+  else return W <= 80 ? launch_q<T, 5>(a, W, batch) : launch_q<T, 8>(a, W, batch);
+}
+
+// tp: the taps a channel spans; 0 for tap-major weights.
 static int launch(const CArgs& a, int tp, int64_t batch) {
+  if (tp == 0) {
+    // the window of 64 columns, up to 16 NP staged rows (five and more taps'
+    // fragments leave registers for 96)
+    const int64_t W = int64_t{63} * a.qs + static_cast<int64_t>(a.T - 1) * a.tm + 1;
+    if (W <= (a.T >= 5 ? 96 : 128)) {
+      switch (a.T) {
+        case 1: return launch_q<1>(a, static_cast<int>(W), batch);
+        case 2: return launch_q<2>(a, static_cast<int>(W), batch);
+        case 3: return launch_q<3>(a, static_cast<int>(W), batch);
+        case 4: return launch_q<4>(a, static_cast<int>(W), batch);
+        case 5: return launch_q<5>(a, static_cast<int>(W), batch);
+        case 6: return launch_q<6>(a, static_cast<int>(W), batch);
+        default: return launch_q<7>(a, static_cast<int>(W), batch);
+      }
+    }
+    return launch_tp<0>(a, pick_shape(a, batch), batch);
+  }
   const Shape s = pick_shape(a, batch);
   if (tp == 2) return launch_tp<2>(a, s, batch);
   if (tp == 4) return launch_tp<4>(a, s, batch);
@@ -428,7 +744,9 @@ static int pack(const Geo& g, void* wp, const kk_tensor* w, const Dequant& dq) {
   p.P = static_cast<int>(g.P); p.T = static_cast<int>(g.T); p.TP = static_cast<int>(g.TP);
   p.M = static_cast<int>(g.M); p.KS = static_cast<int>(g.KS);
   p.transposed = g.transposed;
-  p.units = g.bytes / 16;
+  p.tap_major = tap_major(g, w->dtype) ? 1 : 0;
+  if (p.tap_major) p.KS = static_cast<int>(g.T * g.Cin / 16);  // (no more than g.KS)
+  p.units = g.MT * p.KS * 64;
   const dim3 grid(static_cast<unsigned>(ceil_div(p.units, 256)));
   if (w->dtype == KK_F16) KK_LAUNCH(convh_pack<_Float16>, grid, dim3(256), 0, ctx().stream, p);
   else if (w->dtype == KK_I8) KK_LAUNCH(convh_pack<int8_t>, grid, dim3(256), 0, ctx().stream, p);
@@ -447,9 +765,9 @@ static bool weights_ok(const kk_tensor* w, const Dequant& dq) {
 
 // The launch arguments of a call, or false when the fp16 path does not
 // apply (more than 8 taps, or sizes beyond its 32-bit offsets and grid).
-static bool make_args(CArgs* a, const Geo& g, const kk_tensor* out, const kk_tensor* x,
-                      const Dequant& dq, const kk_tensor* bias, int64_t stride, int64_t dilation,
-                      int64_t pad0, int64_t Nq) {
+static bool make_args(CArgs* a, const Geo& g, bool taps_first, const kk_tensor* out,
+                      const kk_tensor* x, const Dequant& dq, const kk_tensor* bias, int64_t stride,
+                      int64_t dilation, int64_t pad0, int64_t Nq) {
   const int64_t N = x->shape[0], L = x->shape[2], Lout = out->shape[2];
   if (!g.TP || x->dtype != KK_F32 || N > 65535 || g.Cin * L * 4 >= (int64_t{1} << 31) ||
       g.Cout * Lout * 4 >= (int64_t{1} << 31) || g.bytes >= (int64_t{1} << 31) ||
@@ -466,7 +784,8 @@ static bool make_args(CArgs* a, const Geo& g, const kk_tensor* out, const kk_ten
   a->Cin = static_cast<int>(g.Cin); a->L = static_cast<int>(L);
   a->Cout = static_cast<int>(g.Cout); a->Lout = static_cast<int>(Lout);
   a->M = static_cast<int>(g.M); a->Nq = static_cast<int>(Nq); a->P = static_cast<int>(g.P);
-  a->T = static_cast<int>(g.T); a->KS = static_cast<int>(g.KS);
+  a->T = static_cast<int>(g.T);
+  a->KS = static_cast<int>(taps_first ? g.T * g.Cin / 16 : g.KS);
   if (g.transposed) {
     a->qs = 1; a->ta = static_cast<int>(1 - g.T); a->tm = 1;
     a->os = static_cast<int>(g.P); a->oph = static_cast<int>(-pad0);
@@ -522,7 +841,9 @@ bool convh_run(const kk_tensor* out, const kk_tensor* x, const kk_tensor* w, con
   // enough work for the matrix cores
   if (Cin < 8 || g.M * Nq * g.T * Cin < (int64_t{1} << 24)) return false;
   CArgs a;
-  if (!make_args(&a, g, out, x, dq, bias, stride, dilation, pad0, Nq)) return false;
+  const bool taps_first = tap_major(g, w->dtype);
+  const int tp = taps_first ? 0 : static_cast<int>(g.TP);
+  if (!make_args(&a, g, taps_first, out, x, dq, bias, stride, dilation, pad0, Nq)) return false;
   if (packed) {
     a.wp = static_cast<const uint4*>(packed->data);
   } else {
@@ -534,12 +855,12 @@ bool convh_run(const kk_tensor* out, const kk_tensor* x, const kk_tensor* w, con
     *rc = pack(g, wp, w, dq);
     if (*rc == KK_OK) {
       a.wp = static_cast<const uint4*>(wp);
-      *rc = launch(a, static_cast<int>(g.TP), x->shape[0]);
+      *rc = launch(a, tp, x->shape[0]);
     }
     if (ws) kk_free(ws);  // stream order keeps it alive for the kernels above
     return true;
   }
-  *rc = launch(a, static_cast<int>(g.TP), x->shape[0]);
+  *rc = launch(a, tp, x->shape[0]);
   return true;
 }
 

@@ -512,6 +512,60 @@ def test_fp16_weight_conv_small_activations(gpu, oracle, sigma, kind):
     check(got, want, f"{kind} sigma {sigma}")
 
 
+@pytest.mark.parametrize("tr,cin,cout,k,L,pad,dil,stride,wdt,bad", [
+    # every tap count of the 128-channel layout, windows of 64 .. 128 staged rows
+    (0, 128, 192, 1, 700, 0, 1, 1, np.int8, None), (0, 256, 130, 2, 333, 1, 3, 1, np.uint8, None),
+    (0, 512, 512, 3, 129, 1, 1, 1, np.int8, None), (0, 128, 320, 4, 401, 3, 21, 1, np.int8, None),
+    (0, 128, 256, 5, 515, 6, 3, 1, np.int8, None), (0, 128, 200, 6, 450, 5, 1, 1, np.uint8, None),
+    (0, 256, 256, 7, 260, 9, 3, 1, np.int8, None), (0, 128, 256, 3, 801, 1, 1, 2, np.int8, None),
+    # windows that are not staged: wide dilations, strides
+    (0, 128, 256, 3, 900, 40, 40, 1, np.int8, None), (0, 128, 256, 7, 700, 18, 6, 1, np.uint8, None),
+    (0, 128, 300, 3, 1500, 1, 1, 3, np.int8, None), (0, 128, 128, 8, 400, 3, 1, 1, np.int8, None),
+    # phases, and columns past the signal
+    (1, 128, 64, 20, 97, 5, 1, 10, np.int8, None), (1, 256, 48, 12, 130, 3, 1, 6, np.uint8, None),
+    (1, 128, 96, 4, 300, 0, 1, 4, np.int8, None),
+    # an infinity, a NaN (their splits hold NaNs), a huge value
+    (0, 256, 256, 3, 200, 1, 1, 1, np.int8, np.inf), (0, 256, 256, 3, 200, 1, 1, 1, np.int8, np.nan),
+    (0, 256, 256, 3, 200, 1, 1, 1, np.int8, np.float32(1e36)),
+    (0, 128, 256, 3, 900, 40, 40, 1, np.int8, np.inf)])
+def test_8bit_conv_of_128_channel_rounds(gpu, oracle, tr, cin, cout, k, L, pad, dil, stride, wdt, bad):
+    """8-bit weights over a multiple of 128 channels (and its neighbours):
+    packed and not, every tap count, windows at and past what is staged, with
+    a zero point and a bias, against the oracle on the dequantised weight."""
+    r = rng(46)
+    x = r.normal(0, 1, (1, cin, L)).astype(np.float32)
+    lo, hi = (0, 256) if wdt is np.uint8 else (-127, 128)
+    shape = (cin, cout, k) if tr else (cout, cin, k)
+    w = r.integers(lo, hi, shape).astype(wdt)
+    sc, z = np.float32(2.0 ** -9), wdt(121 if wdt is np.uint8 else -3)
+    b = r.normal(0, 0.1, cout).astype(np.float32)
+    if bad is not None:
+        x[0, 5, L // 2] = bad
+        w[:, :, :] = np.where(w == z, z + 1, w)  # (no 0 * inf that another order would not meet)
+    wd = oracle.dequantize(w, np.array(sc), np.array(z))
+    dv = gpu.to_device
+    dw, dz = dv(w), dv(np.array(z))
+    kw = dict(w_scale=dv(np.array(sc)), w_zp=dz)
+    with np.errstate(all="ignore"):
+        if tr:
+            want = oracle.conv_transpose1d(x, wd, b, (pad, pad), stride)
+        else:
+            want = oracle.conv1d(x, wd, b, (pad, pad), stride, dil)
+    for packed in (None, gpu.ops.conv_pack(dw, dz, bool(tr), stride if tr else 1)):
+        if tr:
+            got = gpu.ops.conv_transpose1d(dv(x), dw, dv(b), (pad, pad), stride, packed=packed, **kw).numpy()
+        else:
+            got = gpu.ops.conv1d(dv(x), dw, dv(b), (pad, pad), stride, dil, packed=packed, **kw).numpy()
+        fin = np.isfinite(want)
+        np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+        np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)])
+        if bad is not None and np.isfinite(bad):  # (its outputs dwarf the others)
+            small = fin & (np.abs(want) < 1e30)
+            np.testing.assert_allclose(got[fin & ~small], want[fin & ~small], rtol=1e-5)
+            fin = small
+        check(np.where(fin, got, 0), np.where(fin, want, 0), f"conv {cin}->{cout} k{k} packed={packed is not None}")
+
+
 def decoder_stage(r):
     """The decoder upsample stage's operands (the fixed draws of the stage
     tests and of the bench): int8 ConvTranspose1d(512->256, k20, s10, p5)
