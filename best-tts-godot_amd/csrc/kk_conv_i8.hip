@@ -15,14 +15,14 @@
 // (CinP = Cin rounded up to 64 with zero channels) with sum_k a_k per output
 // channel, once per call.
 // The activations stay as they are, uint8 [N][Cin][L]: each block stages
-// the time window its outputs read, 64 channels at a time, into LDS
-// time-major (channels contiguous, offset to int8 on the way), so each
-// MFMA operand fragment -- 16 channels of one tap at one output row or time
-// step -- is one 16-byte LDS read; the same staged rows give
-// sum_ci b[t][ci] for the epilogue.
-#include <type_traits>
-
+// the time window its outputs read, as many channels at a time as its LDS
+// holds, into LDS time-major (channels contiguous, offset to int8 on the
+// way), so each MFMA operand fragment -- 16 channels of one tap at one output
+// row or time step -- is one 16-byte LDS read; the same fragments give
+// sum_k b_k of an output's receptive field for the epilogue.
+#include <algorithm>
 #include <mutex>
+#include <type_traits>
 #include <unordered_map>
 
 #include "kk_internal.h"
@@ -32,18 +32,11 @@ namespace i8conv {  // named: the kernels keep readable names in profiles
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float f4a __attribute__((ext_vector_type(4)));
+typedef kk_f4u f4u;
 
 constexpr int kTileM = 128;  // output channels per block (2 waves x 64)
 constexpr int kCinAlign = 64;   // channels per chunk: two 32-deep MFMA steps
-constexpr int kRowPitch = 80;   // LDS bytes per 64-channel row (16-byte pad: staggered banks)
-constexpr int kLeafPitch = 136; // LDS floats per output row in the leaf sums' transpose
-
-// LDS of a block: the staged rows and their channel sums, the per-channel
-// epilogue constants; with leaf sums, then the 64-row transpose area.
-__host__ __device__ constexpr int conv_leaf_off(int rows) {
-  return (rows * (kRowPitch + 4) + 2 * kTileM * 4 + 15) & ~15;
-}
-constexpr int kLeafBytes = 64 * kLeafPitch * 4;
 
 // The graph's per-call bias quantisation ahead of a quantised conv:
 // scale = Mul(sa, sw), bias_int32 = Cast(Floor(Div(bias, scale))); sa and sw
@@ -151,7 +144,8 @@ struct ConvI8Args {
   int64_t scale_n;
   int64_t Cout, Cin, CinP, Kw, s, d, L, p0, Lout, Kreal;
   int W4;               // time rows staged per block: the window plus alignment slack
-  int aligned;          // rows start 4-byte aligned (L % 4 == 0): dword loads
+  int SC;               // channels staged at once (a multiple of 64)
+  int area;             // LDS bytes of the staged window / the output area
   // with outf and 128-step tiles: leaf[(n Cout + co) nleaf + t] = the sum of
   // the block's 128 outputs of row co at steps 128 t .. 128 t + 127 in
   // numpy's order, for t < nleaf (the leaves of the rows' whole 8192-blocks)
@@ -159,322 +153,460 @@ struct ConvI8Args {
   int64_t nleaf;
 };
 
-// Block: 128 output channels x TN output steps, 4 waves as 2 (channels) x
-// 2 (time), wave tile 64 x TN/2 as 2 x TN/64 MFMA tiles of 32 x 32.  For each
-// 64-channel chunk the block stages its whole input window -- the
-// ((TN - 1) s + (K - 1) d + 1) time rows every tap reads, each tap shifted by
-// tap * d -- in LDS once, straight from the uint8 activations: a thread
-// loads four time steps of four channels (one dword per channel), swaps the
-// 4 x 4 bytes into four time rows and flips the top bit (u - 128 = u ^ 0x80);
-// positions in the padding hold xz - 128.  The weights' MFMA fragments come
-// from global memory in the order the waves read them (each wave's 4
-// fragments of a (chunk, tap) step are 4 KB contiguous, loaded three steps
-// ahead), so the taps run without LDS weight tiles or barriers.  Lane (r, g)
-// = (lane % 32, lane / 32) holds A[r][16g .. 16g+15] and reads
-// B[16g .. 16g+15][r] of each 32 x 32 x 32 step from LDS; D(i, j) lands in
-// lane j + 32 ((i / 4) % 2), register (i / 8) 4 + i % 4.  The epilogue's
-// per-channel constants and the staged rows' channel sums sit in LDS.
-// TN (128 or 64) output steps per block; a wave covers TN / 2 of them.
-// RES: the scaled fp32 output plus A.resid (its own instantiation: the
-// residual's registers would lower the plain kernel's occupancy).
-template <int TN, bool RES>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) conv_i8_kernel(ConvI8Args A) {
-  constexpr int NI = TN / 64;  // 32-wide MFMA tiles per wave along time
+// Block: TM = 64 WM output channels x TN = 32 NI WN output steps, 4 waves as
+// WM (channels) x WN (time) x WK (shares of the reduction), wave tile 64 x
+// 32 NI as 2 x NI MFMA tiles of 32 x 32.  The block stages its whole input
+// window -- the ((TN - 1) s + (K - 1) d + 1) time rows every tap reads, each
+// tap shifted by tap * d -- for A.SC channels at once (all of them where the
+// window fits the LDS share of three blocks a CU), straight from the uint8
+// activations: a thread loads four time steps of four channels (one dword
+// per channel), swaps the 4 x 4 bytes into four time rows and flips the top
+// bit (u - 128 = u ^ 0x80); positions in the padding hold xz - 128.  Staged
+// 64 channels at a time, each chunk paid a memory round trip with nothing
+// else in flight, which is what the kernel spent most of its time on.
+// The weights' MFMA fragments come from global memory in the order the waves
+// read them (each wave's 4 fragments of a (chunk, tap) step are 4 KB
+// contiguous, loaded R steps ahead), so the taps run without LDS weight
+// tiles or barriers.  Lane (r, g) = (lane % 32, lane / 32) holds
+// A[r][16g .. 16g+15] and reads B[16g .. 16g+15][r] of each 32 x 32 x 32
+// step from LDS; D(i, j) lands in lane j + 32 ((i / 4) % 2), register
+// (i / 8) 4 + i % 4.
+// With WK = 4 the waves take a quarter of the steps each and add their int32
+// tiles through LDS (exact in any order).
+// RES: the scaled fp32 output plus A.resid.  WIDE: the results leave through
+// LDS (aliasing the staged window), 16 bytes a lane, so that a row which
+// starts off a 128-byte line touches five lines a block instead of eight.
+//
+// Bound, a block at a time, by a chain of phases (128 -> 128 k11 over 405841
+// steps, three blocks a CU: window 2 us, products 7 us with the SIMD's matrix
+// core shared by three waves, 2.4 alone, epilogue 4 us), the matrix cores
+// busy 27% of the time and HBM at half its rate.  What shortened the chain:
+// one round trip for the window instead of one per 64 channels and item, the
+// receptive fields' sums from the fragments in the products' shadow (a pass
+// over the staged rows and a barrier before), constants read as vectors.
+// us, before -> after, without / with a residual: 128 -> 128 k11 [1,128,
+// 405841] 125 -> 110 / 172 -> 160, k3 79 -> 71 / 141 -> 121; 256 -> 256 k7
+// [1,256,67641] 69 -> 55 / 72 -> 57, over 7280 13.7 -> 12.7 / 14.3 -> 13.5;
+// 512 -> 512 k3 over 364 14.7 -> 10.3 / 15.5 -> 10.7.
+template <int WM, int WN, int WK, int NI, int R, bool RES, bool WIDE>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(R == 3 ? 3 : 2)))
+conv_i8_kernel(ConvI8Args A) {
+  constexpr int TM = 64 * WM, TN = 32 * NI * WN;
+  constexpr int kPitch = TN + 8;                   // floats a row of the output area
+  constexpr int kPhases = TM * kPitch * 4 > 40960 ? 2 : 1;  // halves (mi) of the tile that pass through it
+  constexpr int kRows = TM / kPhases;              // output rows in the area at a time
+  constexpr int kVec = kRows * TN / 4 / 256;       // float4 a thread of one pass
   extern __shared__ __align__(16) int8_t conv_lds[];
-  int8_t* Bw = conv_lds;                                          // [W4][kRowPitch]
-  int* rs = reinterpret_cast<int*>(conv_lds + A.W4 * kRowPitch);  // [W4] channel sums
-  int* cst = rs + A.W4;                                           // [kTileM] constant term
-  float* scl = reinterpret_cast<float*>(cst + kTileM);            // [kTileM] scale
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int pitch = A.SC + 16;                                    // odd multiple of 16: staggered banks
+  int8_t* Bw = conv_lds;                                          // [W4][pitch]
+  float* ep = reinterpret_cast<float*>(conv_lds);                 // [kRows][kPitch], after the reduction
+  int* cst = reinterpret_cast<int*>(conv_lds + A.area);           // [TM] constant term
+  float* scl = reinterpret_cast<float*>(cst + TM);                // [TM] scale
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 31, g = lane >> 5;
-  const int wm = wv >> 1, wn = wv & 1;
+  const int wm = WM == 2 ? wv >> 1 : 0, wn = WN == 2 ? wv & 1 : 0, wk = WK > 1 ? wv : 0;
   const uint3 tile = xcd_tile();  // neighbouring time tiles on one XCD
-  const int64_t m0 = static_cast<int64_t>(tile.y) * kTileM;
+  const int64_t m0 = static_cast<int64_t>(tile.y) * TM;
   const int64_t nb = static_cast<int64_t>(tile.x) * TN;
   const int64_t b = tile.z;
   const uint8_t* xb = A.x + b * A.Cin * A.L;
-  const int xz = (A.xzp ? static_cast<int>(A.xzp[0]) : 0) - 128;  // offset x zero point
-  const uint32_t padb = static_cast<uint8_t>(static_cast<int8_t>(xz));
-  const uint32_t padw = padb * 0x01010101u;
+  // offset x zero point: the byte of its dword (a scalar load, waited for
+  // where it is used; a byte load would be waited for here)
+  const uintptr_t xzp = A.xzp ? reinterpret_cast<uintptr_t>(A.xzp) : reinterpret_cast<uintptr_t>(A.wsum);
+  const uint32_t xz4 = *reinterpret_cast<const uint32_t*>(xzp & ~uintptr_t{3}) >> (8 * (xzp & 3));
+  const int xz = (A.xzp ? static_cast<int>(xz4 & 255u) : 0) - 128;
+  const uint32_t padw = static_cast<uint8_t>(static_cast<int8_t>(xz)) * 0x01010101u;
   // staged row 0 is source time a0 (padded time nb*s is source time nb*s - p0);
   // the window proper starts sh rows in
   const int64_t a = nb * A.s - A.p0;
-  const int64_t a0 = A.aligned ? (a & ~int64_t{3}) : a;
+  const int64_t a0 = a & ~int64_t{3};  // a dword never straddles time 0
   const int sh = static_cast<int>(a - a0);
-  // v = acc + cst[co] - wz * S, with cst = K wz xz - xz sum(a) (+ bias) and
-  // S = sum of b over the receptive field; the weight zero point is one
-  // value for the tensor (every live row of wzo holds it)
-  const int wz = A.wzo[0];
-  if (tid < kTileM) {
-    const int64_t co = m0 + tid;
-    int c = 0;
-    float sc = 0.0f;
-    if (co < A.Cout) {
-      c = static_cast<int>(A.Kreal) * wz * xz - xz * A.wsum[co];
-      if (A.outf && A.qsa) {
-        c += qbias_channel(A.qsa[0], A.qsw[0], A.qbias[co], &sc);
-      } else if (A.outf) {
-        if (A.bias) c += A.bias[co];
-        sc = A.scale[A.scale_n > 1 ? co : 0];
-      }
-    }
-    cst[tid] = c;
-    scl[tid] = sc;
-  }
   // A fragments straight from the fragment-ordered weights (no LDS): step
-  // st = chunk * Kw + tap of row block m0 / 128 is 8 KB, wave row wm's four
+  // st = chunk * Kw + tap of row block m0 / 128 is 8 KB, a 64-row half's four
   // fragments (ks, mi) 4 KB of it, lane l's 16 bytes of fragment q at
-  // q * 1024 + 16 l.  A ring of three steps' fragments runs three steps
-  // ahead; a load past the block's last step reads 0 (the buffer's range
-  // check) and is never used.
+  // q * 1024 + 16 l.  A ring of R steps' fragments runs R steps ahead; a
+  // load past the block's last step reads 0 (the buffer's range check) and
+  // is never used.
   const int nch = static_cast<int>(A.CinP / kCinAlign), Kw = static_cast<int>(A.Kw);
   const int S = nch * Kw;
   const auto wrs = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<int8_t*>(A.wT) + (m0 / kTileM) * static_cast<int64_t>(S) * 8192, 0, S * 8192,
       0x00020000);
-  const uint32_t w_lane = static_cast<uint32_t>(wm * 4096 + lane * 16);
+  const uint32_t w_lane =
+      static_cast<uint32_t>((wm + static_cast<int>(m0 % kTileM) / 64) * 4096 + lane * 16);
   auto lda = [&](int st, v4i (&f)[4]) {
     const uint32_t off = static_cast<uint32_t>(st) * 8192u + w_lane;
 #pragma unroll
     for (int q = 0; q < 4; ++q)
       f[q] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wrs, off + 1024u * q, 0, 0));
   };
-  // LDS offsets of this lane's B fragments: rows (wn*TN/2 + 32ni + r)*s +
-  // tap*d + sh, columns 16g (+32 per k-step)
+  // LDS offsets of this lane's B fragments: rows (wn 32 NI + 32 ni + r) s +
+  // tap d + sh, columns 16g (+32 per k-step)
   int b_off[NI];
 #pragma unroll
   for (int ni = 0; ni < NI; ++ni)
-    b_off[ni] = ((wn * (TN / 2) + ni * 32 + r) * static_cast<int>(A.s) + sh) * kRowPitch + 16 * g;
-  const int tap_step = static_cast<int>(A.d) * kRowPitch;
+    b_off[ni] = ((wn * 32 * NI + ni * 32 + r) * static_cast<int>(A.s) + sh) * pitch + 16 * g;
+  const int tap_step = static_cast<int>(A.d) * pitch;
   const int ngrp = A.W4 / 4;  // groups of four staged rows
-  const int nitems = static_cast<int>(ceil_div(ngrp, 16)) * 256;
   // 32-bit staging arithmetic (the host checks Cin * L < 2^31)
   const int Cin = static_cast<int>(A.Cin), Li = static_cast<int>(A.L);
   const uint32_t L = static_cast<uint32_t>(A.L);
   const int a0i = static_cast<int>(a0);
-  // A chunk's window: item (tg, cg) = rows 4tg .. 4tg+3 x channels c0 +
-  // 4cg .. 4cg+3.  A wave takes 4 channel groups x 16 consecutive time
-  // groups: one channel of its items is 4 rows x 64 contiguous bytes (its
-  // LDS writes meet 4-way bank conflicts, which cost little).  Then each
-  // staged row's channel sum gains this chunk's share.
-  // The window's loads are buffer loads, issued whatever the position (a
-  // read outside x returns 0), with padding and missing channels chosen by
-  // selects: no branch around a load, which keeps the compiler's wait counts
-  // for the weight ring exact.
-  const auto xrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(xb), 0, Cin * Li,
-                                                     0x00020000);
-  auto stage = [&](int c0) {
-    for (int it = tid; it < nitems; it += 256) {
-      const int cg = (it >> 4) & 15, tg = (it & 15) + 16 * (it >> 8);
-      const int ts = a0i + 4 * tg;
-      const int ci0 = c0 + 4 * cg;
-      uint32_t dw[4];
-      if (A.aligned) {  // a dword is wholly inside the signal or wholly outside
-        const bool in = ts >= 0 && ts < Li;
+  // x of one to three bytes is held in a word; its dword loads go elsewhere
+  const int total = Cin * Li;
+  const bool tiny = total < 4;
+  uint32_t tinyw = 0;
+  if (tiny)
+    for (int q = 0; q < total; ++q) tinyw |= static_cast<uint32_t>(xb[q]) << (8 * q);
+  const uint8_t* xl = tiny ? reinterpret_cast<const uint8_t*>(A.wT) : xb;
+  const uint32_t last4 = static_cast<uint32_t>(tiny ? 0 : total - 4);
+  // Items of a wave: 8 groups of four rows x 8 groups of four channels (its
+  // LDS writes then meet two-way bank conflicts); kU items' loads are in
+  // flight together: six of the first channels (no sums are held yet), fewer
+  // where further channels follow.
+  const int nbt = (ngrp + 7) / 8;
+  const int dq = nbt == 1 ? 4 : nbt == 2 ? 2 : nbt <= 4 ? 1 : 0, dr = 4 - dq * nbt;  // 4 = dq nbt + dr
+  // inner: the items of every staged group lie inside their rows (blocks away
+  // from the signal's ends, channels in whole chunks), so nothing is masked.
+  const bool inner = a0i >= 0 && a0i + 32 * nbt <= Li && Cin % kCinAlign == 0;
+  auto stage_as = [&](int c0, int nc, auto units, auto inner_block) {
+    constexpr int kU = decltype(units)::value;
+    constexpr bool kInner = decltype(inner_block)::value;
+    const int nwi = nbt * (nc / 32);
+    int tb = wv, cb = 0;
+    while (tb >= nbt) { tb -= nbt; ++cb; }
+    for (int w0 = wv; w0 < nwi; w0 += 4 * kU) {
+      uint32_t dw[kU][4];
+      int tgs[kU], cgs[kU];  // (items past the last repeat it, and are not written)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          uint32_t off = static_cast<uint32_t>(ci0 + e) * L + static_cast<uint32_t>(ts);
-          asm volatile("" : "+v"(off));  // keeps the load unconditional
-          const uint32_t ld = __builtin_amdgcn_raw_buffer_load_b32(xrs, off, 0, 0);
-          dw[e] = ci0 + e < Cin ? (in ? (ld ^ 0x80808080u) : padw) : 0u;  // padding channels hold 0
+      for (int u = 0; u < kU; ++u) {
+        const bool live = w0 + 4 * u < nwi;
+        tgs[u] = 8 * (live ? tb : 0) + (lane & 7);
+        cgs[u] = 8 * (live ? cb : 0) + (lane >> 3);
+        tb += dr;
+        cb += dq;
+        if (tb >= nbt) { tb -= nbt; ++cb; }
+        const int ts = a0i + 4 * tgs[u], ci0 = c0 + 4 * cgs[u];
+        uint32_t off = static_cast<uint32_t>(ci0) * L + static_cast<uint32_t>(ts);
+#pragma unroll
+        for (int e = 0; e < 4; ++e, off += L) {
+          // inside x whatever the position: x's last dword where the dword
+          // would pass its end (its bytes then moved down), and where the
+          // position lies outside x (nothing of it kept)
+          const uint32_t offc = kInner || off < last4 ? off : last4;
+          __builtin_memcpy(&dw[u][e], xl + offc, 4);  // one dword load at any alignment
         }
-      } else {
+      }
+      asm volatile("" ::: "memory");  // (no load sinks into the branch that uses it)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          uint32_t off = static_cast<uint32_t>(ci0 + e) * L + static_cast<uint32_t>(ts);
-          asm volatile("" : "+v"(off));
-          uint32_t v = 0;
+      for (int u = 0; u < kU; ++u) {
+        if (w0 + 4 * u >= nwi) continue;  // (wave-uniform)
+        if constexpr (!kInner) {
+          const int ts = a0i + 4 * tgs[u], ci0 = c0 + 4 * cgs[u];
+          // bytes at or past L are padding (keep: the others)
+          const int left = Li - ts;
+          const uint32_t keep = ts < 0 || left <= 0 ? 0u : left >= 4 ? ~0u : (1u << (8 * left)) - 1u;
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int t = ts + q;
-            const uint32_t ld = __builtin_amdgcn_raw_buffer_load_b8(xrs, off + q, 0, 0);
-            v |= ((t >= 0 && t < Li) ? (ld ^ 0x80u) : padb) << (8 * q);
+          for (int e = 0; e < 4; ++e) {
+            const uint32_t off = static_cast<uint32_t>(ci0 + e) * L + static_cast<uint32_t>(ts);
+            const uint32_t offc = off < last4 ? off : last4;
+            const uint32_t v = (tiny ? tinyw : dw[u][e]) >> (8 * ((off - offc) & 3));
+            // (padding channels hold 0: 0x80 once the top bits flip)
+            dw[u][e] = ci0 + e < Cin ? (v & keep) | ((padw ^ 0x80808080u) & ~keep) : 0x80808080u;
           }
-          dw[e] = ci0 + e < Cin ? v : 0u;
         }
+        if (tgs[u] >= ngrp) continue;
+        // 4 x 4 byte transpose (v_perm: bytes 0-3 from the second operand,
+        // 4-7 from the first): word q = the four channels at time 4tg + q
+        const uint32_t t01l = __builtin_amdgcn_perm(dw[u][1], dw[u][0], 0x05010400u);
+        const uint32_t t01h = __builtin_amdgcn_perm(dw[u][1], dw[u][0], 0x07030602u);
+        const uint32_t t23l = __builtin_amdgcn_perm(dw[u][3], dw[u][2], 0x05010400u);
+        const uint32_t t23h = __builtin_amdgcn_perm(dw[u][3], dw[u][2], 0x07030602u);
+        int8_t* dst = Bw + 4 * tgs[u] * pitch + 4 * cgs[u];
+        *reinterpret_cast<uint32_t*>(dst) =
+            __builtin_amdgcn_perm(t23l, t01l, 0x05040100u) ^ 0x80808080u;
+        *reinterpret_cast<uint32_t*>(dst + pitch) =
+            __builtin_amdgcn_perm(t23l, t01l, 0x07060302u) ^ 0x80808080u;
+        *reinterpret_cast<uint32_t*>(dst + 2 * pitch) =
+            __builtin_amdgcn_perm(t23h, t01h, 0x05040100u) ^ 0x80808080u;
+        *reinterpret_cast<uint32_t*>(dst + 3 * pitch) =
+            __builtin_amdgcn_perm(t23h, t01h, 0x07060302u) ^ 0x80808080u;
       }
-      if (tg >= ngrp) continue;
-      // 4 x 4 byte transpose (v_perm: bytes 0-3 from the second operand,
-      // 4-7 from the first): word q = the four channels at time 4tg + q
-      const uint32_t t01l = __builtin_amdgcn_perm(dw[1], dw[0], 0x05010400u);
-      const uint32_t t01h = __builtin_amdgcn_perm(dw[1], dw[0], 0x07030602u);
-      const uint32_t t23l = __builtin_amdgcn_perm(dw[3], dw[2], 0x05010400u);
-      const uint32_t t23h = __builtin_amdgcn_perm(dw[3], dw[2], 0x07030602u);
-      uint32_t* dst = reinterpret_cast<uint32_t*>(Bw + 4 * tg * kRowPitch + 4 * cg);
-      dst[0] = __builtin_amdgcn_perm(t23l, t01l, 0x05040100u);
-      dst[kRowPitch / 4] = __builtin_amdgcn_perm(t23l, t01l, 0x07060302u);
-      dst[2 * kRowPitch / 4] = __builtin_amdgcn_perm(t23h, t01h, 0x05040100u);
-      dst[3 * kRowPitch / 4] = __builtin_amdgcn_perm(t23h, t01h, 0x07060302u);
-    }
-    __syncthreads();
-    for (int row = tid; row < A.W4; row += 256) {
-      const int* p = reinterpret_cast<const int*>(Bw + row * kRowPitch);
-      int sum = c0 == 0 ? 0 : rs[row];
-#pragma unroll
-      for (int k = 0; k < kCinAlign / 4; ++k) sum = __builtin_amdgcn_sdot4(p[k], 0x01010101, sum, false);
-      rs[row] = sum;
     }
   };
+  auto stage = [&](int c0, int nc, auto units) {  // nc channels (a multiple of 64) from c0
+    if (inner) stage_as(c0, nc, units, std::true_type{});
+    else stage_as(c0, nc, units, std::false_type{});
+  };
+  // The first fragments and the channel constants' operands are loaded before
+  // the window (one memory round trip for all of them).
+  v4i f[R][4];
+  // a wave's steps of nc staged channels: lb .. le - 1 of nc / 64 Kw
+  auto first_step = [&](int nc) { return WK > 1 ? wk * (nc / kCinAlign * Kw) / WK : 0; };
+#pragma unroll
+  for (int i = 0; i < R; ++i) lda(first_step(A.SC) + i, f[i]);
+  const int64_t co = std::min<int64_t>(m0 + tid % TM, A.Cout - 1);
+  const float* any = reinterpret_cast<const float*>(A.wsum);
+  const int wsum = A.wsum[co], wz = A.wzo[0];
+  const float qb = (A.qbias ? A.qbias : any)[co], qsa = *(A.qsa ? A.qsa : any), qsw = *(A.qsw ? A.qsw : any);
+  asm volatile("" ::: "memory");
+  stage(0, A.SC, std::integral_constant<int, (R > 3 ? 12 : 6)>{});
   v16i acc[2][NI] = {};
-  // one step's MFMAs: B fragments of the tap from the staged window
-  auto mma = [&](int tap, const v4i (&f)[4]) {
-    const int8_t* Bb = Bw + tap * tap_step;
+  int bs[NI] = {};  // sum_k b_k of this lane's columns, its half (g) of the channels
+  for (int c0 = 0; c0 < static_cast<int>(A.CinP); c0 += A.SC) {
+    const int nc = min(A.SC, static_cast<int>(A.CinP) - c0);
+    const int steps = nc / kCinAlign * Kw, st0 = c0 / kCinAlign * Kw;
+    const int lb = first_step(nc), le = WK > 1 ? (wk + 1) * steps / WK : steps;
+    if (c0 > 0) {
+      __syncthreads();  // every wave is done with the previous window
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      v4i bf[NI];
-#pragma unroll
-      for (int ni = 0; ni < NI; ++ni)
-        bf[ni] = *reinterpret_cast<const v4i*>(Bb + b_off[ni] + 32 * ks);
-#pragma unroll
-      for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < NI; ++ni)
-          acc[mi][ni] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f[2 * ks + mi], bf[ni], acc[mi][ni], 0, 0, 0);
-    }
-  };
-  v4i f0[4], f1[4], f2[4];
-  lda(0, f0);
-  lda(1, f1);
-  lda(2, f2);
-  int tap = 0, c0 = 0;
-  // a chunk's first step stages its window (after every wave is done with
-  // the previous one); the ring slot of step st is st % 3.  Every slot's
-  // refill is issued whether or not its step exists (past the last step it
-  // reads 0): a refill skipped on some path leaves the compiler's wait
-  // counts for the other slots at "all loads", which drains the ring.
-  auto run = [&](int st, v4i (&f)[4]) {
-    if (st < S) {
-      if (tap == 0) {
-        if (st > 0) __syncthreads();
-        stage(c0);
+      for (int i = 0; i < R; ++i) lda(st0 + lb + i, f[i]);
+      stage(c0, nc, std::integral_constant<int, NI == 2 && WK == 1 ? 2 : 4>{});
+    } else if (tid < TM) {
+      // v = acc + cst[co] - wz * S, with cst = K wz xz - xz sum(a) (+ bias) and
+      // S = sum of b over the receptive field; the weight zero point is one
+      // value for the tensor (every live row of wzo holds it)
+      int c = static_cast<int>(A.Kreal) * wz * xz - xz * wsum;
+      float sc = 0.0f;
+      if (A.outf && A.qsa) {
+        c += qbias_channel(qsa, qsw, qb, &sc);
+      } else if (A.outf) {
+        if (A.bias) c += A.bias[co];
+        sc = A.scale[A.scale_n > 1 ? co : 0];
       }
-      mma(tap, f);
-      if (++tap == Kw) {
-        tap = 0;
-        c0 += kCinAlign;
+      cst[tid] = c;
+      scl[tid] = sc;
+    }
+    lds_barrier();
+    int tap = lb % Kw, base = (lb / Kw) * kCinAlign;  // the step's tap, its channels' offset in a row
+    // The ring slot of step i is (i - lb) % R.  Every slot's refill is issued
+    // whether or not its step exists (past the last step it reads another's
+    // or 0): a refill skipped on some path leaves the compiler's wait counts
+    // for the other slots at "all loads", which drains the ring.
+    for (int st = lb; st < le; st += R) {
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        if (st + i < le) {
+          const int8_t* Bb = Bw + tap * tap_step + base;
+#pragma unroll
+          for (int ks = 0; ks < 2; ++ks) {
+            v4i bf[NI];
+#pragma unroll
+            for (int ni = 0; ni < NI; ++ni)
+              bf[ni] = *reinterpret_cast<const v4i*>(Bb + b_off[ni] + 32 * ks);
+            // the sums of b over a column's receptive field (VALU work in the
+            // shadow of the matrix instructions)
+#pragma unroll
+            for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) bs[ni] = __builtin_amdgcn_sdot4(bf[ni][e], 0x01010101, bs[ni], false);
+#pragma unroll
+            for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+              for (int ni = 0; ni < NI; ++ni)
+                acc[mi][ni] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f[i][2 * ks + mi], bf[ni],
+                                                                    acc[mi][ni], 0, 0, 0);
+          }
+          if (++tap == Kw) {
+            tap = 0;
+            base += kCinAlign;
+          }
+        }
+        lda(st0 + st + i + R, f[i]);
       }
     }
-    lda(st + 3, f);
-  };
-  for (int st = 0; st < S; st += 3) {
-    run(st, f0);
-    run(st + 1, f1);
-    run(st + 2, f2);
   }
-  __syncthreads();  // the last chunk's row sums, for the epilogue
-  int zS[NI];  // wz * sum_k b_k of each of this lane's output columns
+  // (the column's other half of the channels is in lane l ^ 32)
 #pragma unroll
   for (int ni = 0; ni < NI; ++ni) {
-    const int j = wn * (TN / 2) + 32 * ni + r;
-    int S = 0;
-    for (int tap = 0; tap < static_cast<int>(A.Kw); ++tap)
-      S += rs[sh + j * static_cast<int>(A.s) + tap * static_cast<int>(A.d)];
-    zS[ni] = wz * S;
+    const auto pr = __builtin_amdgcn_permlane32_swap(bs[ni], bs[ni], false, false);
+    bs[ni] = static_cast<int>(pr[0]) + static_cast<int>(pr[1]);
   }
-  // outputs from the block's corner, 32-bit byte offsets (the host checks
-  // that a batch's output stays below 2 GiB); a block wholly inside the
-  // output skips the per-element bounds checks
+  // the output tile a wave holds: with WK = 4, tile (wk / 2, wk % 2) of the
+  // four after the exchange, else all its 2 x NI
+  constexpr int kMi = WK > 1 ? 1 : 2, kNi = WK > 1 ? 1 : NI;
+  v16i t[kMi][kNi];
+  int zS[kNi];  // -wz * sum_k b_k of each of this lane's output columns
+  int row0 = wm * 64, col0 = wn * 32 * NI;  // its corner in the block's tile
+  if constexpr (WK > 1) {
+    static_assert(WK == 4 && NI == 2, "four waves exchange four 32 x 32 tiles");
+    lds_barrier();  // the window is free to overwrite
+    int* red = reinterpret_cast<int*>(conv_lds);  // [wave][its three other tiles][16][64]
+    int* redz = red + 4 * 3 * 16 * 64;            // [wave][NI][32]
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (q != wk)
+#pragma unroll
+        for (int reg = 0; reg < 16; ++reg)
+          red[((wk * 3 + ((q - wk - 1) & 3)) * 16 + reg) * 64 + lane] = acc[q >> 1][q & 1][reg];
+    if (g == 0) {
+      redz[wk * 64 + r] = bs[0];
+      redz[wk * 64 + 32 + r] = bs[1];
+    }
+    v16i own = acc[0][0];
+#pragma unroll
+    for (int q = 1; q < 4; ++q)
+      if (q == wk) own = acc[q >> 1][q & 1];
+    row0 = 32 * (wk >> 1);
+    col0 = 32 * (wk & 1);
+    lds_barrier();
+    int z = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) z += redz[w * 64 + col0 + r];
+    zS[0] = -wz * z;
+#pragma unroll
+    for (int o = 1; o < 4; ++o) {  // wave w = wk + o keeps tile wk at (wk - w - 1) & 3 = 3 - o
+      const int w = (wk + o) & 3;
+#pragma unroll
+      for (int reg = 0; reg < 16; ++reg) own[reg] += red[((w * 3 + 3 - o) * 16 + reg) * 64 + lane];
+    }
+    t[0][0] = own;
+  } else {
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni) zS[ni] = -wz * bs[ni];
+#pragma unroll
+    for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+      for (int ni = 0; ni < NI; ++ni) t[mi][ni] = acc[mi][ni];
+  }
+  // outputs and residual at 32-bit byte offsets from the block's corner (the
+  // host checks that a batch's output stays below 2 GiB)
   const int64_t o_elem = (b * A.Cout + m0) * A.Lout + nb;
-  char* ob = reinterpret_cast<char*>(A.outf ? static_cast<void*>(A.outf) : static_cast<void*>(A.out)) +
-             4 * o_elem;
+  char* ob = reinterpret_cast<char*>((A.outf ? A.outf : reinterpret_cast<float*>(A.out)) + o_elem);
   const uint32_t lout4 = static_cast<uint32_t>(4 * A.Lout);
-  const bool full = m0 + kTileM <= A.Cout && nb + TN <= A.Lout;
-  const int c_rem = static_cast<int>(A.Cout - m0), l_rem = static_cast<int>(A.Lout - nb);
-  const int lane_c = wm * 64 + 4 * g, lane_j = wn * (TN / 2) + r;
-  const uint32_t lane_off = static_cast<uint32_t>(lane_c) * lout4 + 4u * static_cast<uint32_t>(lane_j);
-  // the residual at the output's element offsets, through a buffer resource
-  // over this batch's [Cout][Lout] (a read past it returns 0: rows past Cout
-  // and columns past Lout of edge blocks are read but never stored)
-  const auto rrs = __builtin_amdgcn_make_buffer_rsrc(
-      RES ? const_cast<float*>(A.resid) + b * A.Cout * A.Lout : nullptr, 0,
-      RES ? static_cast<int>(A.Cout * A.Lout * 4) : 0, 0x00020000);
-  const uint32_t r_off = static_cast<uint32_t>(4 * (m0 * A.Lout + nb)) + lane_off;
+  const bool full = m0 + TM <= A.Cout && nb + TN <= A.Lout;
+  const int c_rem = static_cast<int>(std::min<int64_t>(A.Cout - m0, TM));
+  const int l_rem = static_cast<int>(std::min<int64_t>(A.Lout - nb, TN));
   // This block's outputs are one numpy leaf of each of its rows (the
   // InstanceNorm that reads them sums its rows in numpy's pairwise order,
   // 8192-blocks of 64 leaves of 128 elements): its sum is formed here, in
   // that order, from the values as stored -- accumulator k of 8 sums the
   // elements 8 m + k, m = 0..15, one after another; then ((a0 + a1) + (a2 +
-  // a3)) + ((a4 + a5) + (a6 + a7)).  A half (mi) of the tile, 64 rows x 128
-  // steps, goes through LDS (kLeafPitch floats a row: the two rows a store
-  // instruction writes fall 32 banks apart), where four threads a row each
-  // sum two accumulators from their own addresses and two shuffles form the
-  // tree.
+  // a3)) + ((a4 + a5) + (a6 + a7)): four threads a row each sum two
+  // accumulators and two shuffles form the tree.
   const bool leafy = TN == 128 && A.leaf && static_cast<int64_t>(tile.x) < A.nleaf;
-  float* const lt = reinterpret_cast<float*>(conv_lds + conv_leaf_off(A.W4));  // [64][kLeafPitch]
-  auto epilogue = [&](auto full_tile) {
-    constexpr bool kFull = decltype(full_tile)::value;
+  auto leaf_sums = [&](int ph) {
+    const int e = tid >> 2, q = tid & 3;  // row e of the area, accumulators 2q and 2q + 1
+    const float* src = ep + e * kPitch + 2 * q;
+    float s0 = src[0], s1 = src[1];
 #pragma unroll
-    for (int mi = 0; mi < 2; ++mi) {
-      // the stored values (for the leaf sums), and before them the residual
-      // of this half of the lane's outputs, all its loads issued before the
-      // first store (a load after a store to a possibly aliasing address
-      // would wait for it: one memory round trip per element)
-      float yv[16][NI];
-      if constexpr (RES) {
+    for (int m = 1; m < 16; ++m) {
+      s0 = s0 + src[8 * m];
+      s1 = s1 + src[8 * m + 1];
+    }
+    float p = s0 + s1;
+    p = p + __shfl_xor(p, 1, 64);
+    p = p + __shfl_xor(p, 2, 64);
+    const int cl = (e >> 5) * 64 + 32 * ph + (e & 31);
+    if (q == 0 && cl < c_rem) A.leaf[(b * A.Cout + m0 + cl) * A.nleaf + tile.x] = p;
+  };
+  const int lane_c = row0 + 4 * g, lane_j = col0 + r;  // this lane's first row and column
+  if constexpr (!WIDE) {
+    // The values leave from the matrix layout, four bytes a lane, each wave
+    // on its own; a half's residual loads all go out before its first store
+    // (a load after a store waits for it: one counter, in order).
+    const auto rrs = __builtin_amdgcn_make_buffer_rsrc(
+        RES ? const_cast<float*>(A.resid) + b * A.Cout * A.Lout : nullptr, 0,
+        RES ? static_cast<int>(A.Cout * A.Lout * 4) : 0, 0x00020000);
+    const uint32_t lane_off = static_cast<uint32_t>(lane_c) * lout4 + 4u * static_cast<uint32_t>(lane_j);
+    const uint32_t r_off = static_cast<uint32_t>(4 * (m0 * A.Lout + nb)) + lane_off;
+    if (leafy) lds_barrier();  // (the sums pass through the window's area)
+    auto store = [&](auto full_tile) {
+      constexpr bool kFull = decltype(full_tile)::value;
 #pragma unroll
-        for (int reg = 0; reg < 16; ++reg) {
-          const int cr = 32 * mi + 8 * (reg / 4) + (reg % 4);
-          const uint32_t roff = r_off + static_cast<uint32_t>(cr) * lout4;
+      for (int mi = 0; mi < kMi; ++mi) {
+        float yv[16][kNi];
 #pragma unroll
-          for (int ni = 0; ni < NI; ++ni)
+        for (int reg = 0; reg < 16; ++reg)
+#pragma unroll
+          for (int ni = 0; RES && ni < kNi; ++ni)  // (past the batch's end a load reads 0)
             yv[reg][ni] = __builtin_bit_cast(
-                float, __builtin_amdgcn_raw_buffer_load_b32(rrs, roff + 128u * ni, 0, 0));
+                float, __builtin_amdgcn_raw_buffer_load_b32(
+                           rrs, r_off + static_cast<uint32_t>(32 * mi + 8 * (reg / 4) + reg % 4) * lout4 + 128u * ni, 0, 0));
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const v4i c = *reinterpret_cast<const v4i*>(cst + lane_c + 32 * mi + 8 * q);
+          const f4a sc = *reinterpret_cast<const f4a*>(scl + lane_c + 32 * mi + 8 * q);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const int reg = 4 * q + k, cr = 32 * mi + 8 * q + k;
+            if (!kFull && lane_c + cr >= c_rem) continue;
+#pragma unroll
+            for (int ni = 0; ni < kNi; ++ni) {
+              if (!kFull && lane_j + 32 * ni >= l_rem) continue;
+              const int v = t[mi][ni][reg] + c[k] + zS[ni];
+              const float y = static_cast<float>(v) * sc[k];
+              yv[reg][ni] = RES ? y + yv[reg][ni] : A.outf ? y : __builtin_bit_cast(float, v);
+              *reinterpret_cast<float*>(ob + (lane_off + static_cast<uint32_t>(cr) * lout4 + 128u * ni)) = yv[reg][ni];
+            }
+          }
         }
-      }
+        if constexpr (TN == 128) {
+          if (leafy) {  // block-uniform: every wave meets the barriers
 #pragma unroll
-      for (int reg = 0; reg < 16; ++reg) {
-        const int cr = 32 * mi + 8 * (reg / 4) + (reg % 4);  // constant once unrolled
-        const int cl = lane_c + cr;
-        if (!kFull && cl >= c_rem) continue;
-        const int c = cst[cl];
-        const float sc = scl[cl];
-        const uint32_t roff = lane_off + static_cast<uint32_t>(cr) * lout4;
+            for (int reg = 0; reg < 16; ++reg)
 #pragma unroll
-        for (int ni = 0; ni < NI; ++ni) {
-          if (!kFull && lane_j + 32 * ni >= l_rem) continue;
-          const int v = acc[mi][ni][reg] + c - zS[ni];
-          char* dst = ob + (roff + 128u * ni);
-          if constexpr (RES) {
-            yv[reg][ni] = static_cast<float>(v) * sc + yv[reg][ni];
-            *reinterpret_cast<float*>(dst) = yv[reg][ni];
-          } else if (A.outf) {
-            yv[reg][ni] = static_cast<float>(v) * sc;
-            *reinterpret_cast<float*>(dst) = yv[reg][ni];
-          } else {
-            *reinterpret_cast<int*>(dst) = v;
+              for (int ni = 0; ni < kNi; ++ni)
+                ep[(wm * 32 + 8 * (reg / 4) + 4 * g + reg % 4) * kPitch + lane_j + 32 * ni] = yv[reg][ni];
+            lds_barrier();
+            leaf_sums(mi);
+            if (mi == 0) lds_barrier();  // (the next half reuses the area)
           }
         }
       }
-      if constexpr (TN == 128) {
-        if (leafy) {  // block-uniform: every wave meets the barriers
+    };
+    if (full) store(std::true_type{});
+    else store(std::false_type{});
+    return;
+  }
+  lds_barrier();  // the window (or the exchanged tiles) may be overwritten
+  // a thread's float4 k of half ph: rows tid / (TN / 4) + kStep k of the area
+  constexpr int kStep = 256 / (TN / 4);
+  const int e0 = tid / (TN / 4), c4 = tid % (TN / 4);
+  const uint32_t off0 = static_cast<uint32_t>(e0) * lout4 + 16u * c4;
+  // row e of the output area in half ph: its channel in the block
+  auto chan = [&](int e, int ph) { return kPhases == 2 ? (e >> 5) * 64 + 32 * ph + (e & 31) : e; };
 #pragma unroll
-          for (int reg = 0; reg < 16; ++reg) {
-            const int rl = wm * 32 + 8 * (reg / 4) + 4 * g + (reg % 4);
+  for (int ph = 0; ph < kPhases; ++ph) {
 #pragma unroll
-            for (int ni = 0; ni < NI; ++ni)
-              lt[rl * kLeafPitch + wn * 64 + 32 * ni + r] = yv[reg][ni];
+    for (int mi = 0; mi < kMi; ++mi) {
+      if (kPhases == 2 && mi != ph) continue;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        // rows 8q + 4g .. + 3 of the 32 x 32 tile: registers 4q .. 4q + 3
+        const int cl = lane_c + 32 * mi + 8 * q;
+        const int e = kPhases == 2 ? wm * 32 + 8 * q + 4 * g : cl;
+        const v4i c = *reinterpret_cast<const v4i*>(cst + cl);
+        const f4a sc = *reinterpret_cast<const f4a*>(scl + cl);
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int ni = 0; ni < kNi; ++ni) {
+            const int v = t[mi][ni][4 * q + k] + c[k] + zS[ni];
+            ep[(e + k) * kPitch + lane_j + 32 * ni] =
+                A.outf ? static_cast<float>(v) * sc[k] : __builtin_bit_cast(float, v);
           }
-          __syncthreads();
-          const int rl = tid >> 2, q = tid & 3;  // row rl, accumulators 2q and 2q + 1
-          const float* src = lt + rl * kLeafPitch + 2 * q;
-          float a0 = src[0], a1 = src[1];
-#pragma unroll
-          for (int m = 1; m < 16; ++m) {
-            a0 = a0 + src[8 * m];
-            a1 = a1 + src[8 * m + 1];
-          }
-          float p = a0 + a1;
-          p = p + __shfl_xor(p, 1, 64);
-          p = p + __shfl_xor(p, 2, 64);
-          const int cl = (rl >> 5) * 64 + 32 * mi + (rl & 31);
-          if (q == 0 && cl < c_rem) A.leaf[(b * A.Cout + m0 + cl) * A.nleaf + tile.x] = p;
-          if (mi == 0) __syncthreads();  // (the next half reuses the area)
-        }
       }
     }
-  };
-  if (full) epilogue(std::true_type{});
-  else epilogue(std::false_type{});
+    lds_barrier();
+    if (full) {
+#pragma unroll
+      for (int k = 0; k < kVec; ++k)
+        *reinterpret_cast<f4u*>(ob + (off0 + static_cast<uint32_t>(chan(kStep * k, ph)) * lout4)) =
+            *reinterpret_cast<const f4a*>(ep + (e0 + kStep * k) * kPitch + 4 * c4);
+    } else {
+      for (int k = tid; k < kRows * TN; k += 256) {
+        const int e = k / TN, col = k % TN, cl = chan(e, ph);
+        if (cl >= c_rem || col >= l_rem) continue;
+        *reinterpret_cast<float*>(ob + (static_cast<uint32_t>(cl) * lout4 + 4u * col)) = ep[e * kPitch + col];
+      }
+    }
+    if constexpr (TN == 128) {
+      if (leafy) leaf_sums(ph);
+    }
+    if (ph + 1 < kPhases) lds_barrier();  // (the next half reuses the area)
+  }
 }
 
 }  // namespace i8conv
@@ -489,32 +621,48 @@ static int64_t conv_rows(int64_t tn, int64_t stride, int64_t dilation, int64_t K
   return ceil_div(conv_window(tn, stride, dilation, K) + 3, 4) * 4;
 }
 
-// LDS of a block: the staged rows and their channel sums, the per-channel
+// LDS of a block that stages sc channels: the rows (with four bytes to spare
+// each, which hold the widest window taken where it was), the per-channel
 // epilogue constants.
-static size_t conv_lds(int64_t rows) {
-  return static_cast<size_t>(rows * (kRowPitch + 4) + 2 * kTileM * 4);
+static int64_t conv_lds(int64_t rows, int64_t sc = kCinAlign) {
+  return rows * (sc + 16 + 4) + 2 * kTileM * 4;
 }
+constexpr int64_t kConvLds = 65536;
 
-// The time tile (128, else 64) whose block fits 64 KB of LDS; 0 if neither does.
+// The time tile (128, else 64) whose block fits 64 KB of LDS with 64 channels
+// staged; 0 if neither does.
 static int conv_tile_n(int64_t stride, int64_t dilation, int64_t K) {
   for (int tn : {128, 64})
-    if (conv_lds(conv_rows(tn, stride, dilation, K)) <= 65536) return tn;
+    if (conv_lds(conv_rows(tn, stride, dilation, K)) <= kConvLds) return tn;
   return 0;
 }
 
-// The launch's time tile: 128 when its blocks still give every CU two (the
-// kernel is latency-bound and three blocks share a CU), else 64 for twice
-// the blocks.  Measured on the 128-id graph (whose convolutions run at
-// 240 .. 431,000 steps): 128 everywhere 39.6 ms, 64 everywhere 38.4 ms, and
-// 64 everywhere 7% slower on [1,128,431000] alone.
-static int conv_launch_tile(int64_t stride, int64_t dilation, int64_t K, int64_t N,
-                            int64_t CoutP, int64_t Lout) {
+// Whether leaf sums can be formed: the window of a 128-step tile and 64 rows
+// of its outputs side by side in 64 KB.
+static bool conv_leaves_fit(int64_t stride, int64_t dilation, int64_t K) {
+  return ceil_div(conv_lds(conv_rows(128, stride, dilation, K)), 16) * 16 + 64 * 136 * 4 <= kConvLds;
+}
+
+// The launch's block.  128 x 128 outputs when such blocks still give every
+// CU two (three share a CU); else 128 x 64 where those give every other CU
+// one (256 -> 256 k3 over 7280 steps, 228 blocks: 10.6 us against 12.0 for
+// 64 x 64; k7 over 14560, 456 blocks: 19.0 against 25.2); else 64 x 64, its
+// waves sharing the reduction, for short rows, whose few blocks are bound by
+// the chain of steps of each (512 -> 512 k3 over 364, 24 blocks: 10.7 us
+// against 13.2), and up to a block a CU for reductions of more than 32 steps
+// of 64 (256 -> 256 k11 over 7280: 15.6 against 17.6).
+struct ConvShape {
+  int tm, tn;
+};
+static ConvShape conv_launch_shape(int64_t stride, int64_t dilation, int64_t K, int64_t N,
+                                   int64_t CinP, int64_t CoutP, int64_t Lout) {
   const int tn = conv_tile_n(stride, dilation, K);
   const int64_t cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
-  if (tn == 128 && N * (CoutP / kTileM) * ceil_div(Lout, 128) < 2 * cus &&
-      conv_lds(conv_rows(64, stride, dilation, K)) <= 65536)
-    return 64;
-  return tn;
+  if (tn == 128 && (N * (CoutP / kTileM) * ceil_div(Lout, 128) >= 2 * cus ||
+                    conv_lds(conv_rows(64, stride, dilation, K)) > kConvLds))
+    return {128, 128};
+  const int64_t blocks = N * (CoutP / kTileM) * ceil_div(Lout, 64);
+  return {2 * blocks < cus || (blocks < cus && CinP / kCinAlign * K > 32) ? 64 : 128, 64};
 }
 
 // The allocation-free entry point's workspace: a file-scope device array of
@@ -620,6 +768,14 @@ static int check_conv_integer(const kk_tensor* out, const kk_tensor* x, const kk
   return KK_OK;
 }
 
+static int conv_launch(void (*kernel)(ConvI8Args), const dim3& grid, size_t lds, const ConvI8Args& A) {
+  if (lds > 65536)  // (the widest windows; a kernel needs the attribute for more)
+    KK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+  KK_LAUNCH(kernel, grid, dim3(256), lds, ctx().stream, A);
+  return check_launch("conv_i8_kernel");
+}
+
 // Every entry point: `outf` set gives the scaled fp32 form; `fixed_ws`, when
 // given, is the workspace (conv_ws_layout(...).total bytes, checked by the
 // caller) instead of one from the pool.
@@ -686,28 +842,44 @@ static int conv_integer_run(const kk_tensor* out, const kk_tensor* x, const kk_t
     A.Cout = Cout; A.Cin = Cin; A.CinP = CinP; A.Kw = Kw; A.s = stride; A.d = dilation;
     A.L = L; A.p0 = pad0; A.Lout = Lout; A.Kreal = Cin * Kw;
     A.resid = resid ? static_cast<const float*>(resid->data) : nullptr;
-    A.aligned = (L % 4 == 0) && (reinterpret_cast<uintptr_t>(x->data) % 4 == 0);
     // leaf sums need the 128-step tiles (checked to fit by the caller)
-    const int tn = leaves ? 128 : conv_launch_tile(stride, dilation, Kw, N, CoutP, Lout);
+    const ConvShape sh = leaves ? ConvShape{128, 128}
+                                : conv_launch_shape(stride, dilation, Kw, N, CinP, CoutP, Lout);
     if (leaves) {
       A.leaf = static_cast<float*>(leaves->data);
       A.nleaf = (Lout / 8192) * 64;
     }
-    A.W4 = static_cast<int>(conv_rows(tn, stride, dilation, Kw));
-    const dim3 grid(static_cast<unsigned>(ceil_div(Lout, tn)),
-                    static_cast<unsigned>(CoutP / kTileM), static_cast<unsigned>(N));
+    A.W4 = static_cast<int>(conv_rows(sh.tn, stride, dilation, Kw));
+    // Channels staged at once: all of them if three blocks a CU (two of the
+    // smaller tiles, whose blocks are few) keep their LDS, else equal shares.
+    const int64_t lds_max = sh.tn == 128 ? 53248 : kConvLds;
+    int64_t parts = 1;
+    while (parts < CinP / kCinAlign &&
+           conv_lds(A.W4, ceil_div(CinP / kCinAlign, parts) * kCinAlign) > lds_max)
+      ++parts;
+    A.SC = static_cast<int>(ceil_div(CinP / kCinAlign, parts) * kCinAlign);
+    // the window, or after it the outputs (64 x 136 or 128 x 72 floats; with
+    // the reduction shared, the waves' 12 exchanged tiles of 4 KB)
+    const int out_area = sh.tm == 64 ? 49152 + 1024 : sh.tn == 64 ? 128 * 72 * 4 : 64 * 136 * 4;
+    A.area = static_cast<int>(std::max<int64_t>(A.W4 * int64_t{A.SC + 16}, out_area));
+    const dim3 grid(static_cast<unsigned>(ceil_div(Lout, sh.tn)),
+                    static_cast<unsigned>(ceil_div(Cout, sh.tm)), static_cast<unsigned>(N));
     rc = check_xcd_grid(grid, "ConvInteger");
     if (rc == KK_OK) {
-      const size_t lds = A.leaf ? static_cast<size_t>(conv_leaf_off(A.W4) + kLeafBytes)
-                                : conv_lds(A.W4);
-      if (A.resid) {
-        if (tn == 128) KK_LAUNCH((conv_i8_kernel<128, true>), grid, dim3(256), lds, st, A);
-        else KK_LAUNCH((conv_i8_kernel<64, true>), grid, dim3(256), lds, st, A);
-      } else {
-        if (tn == 128) KK_LAUNCH((conv_i8_kernel<128, false>), grid, dim3(256), lds, st, A);
-        else KK_LAUNCH((conv_i8_kernel<64, false>), grid, dim3(256), lds, st, A);
-      }
-      rc = check_launch("conv_i8_kernel");
+      const size_t lds = static_cast<size_t>(A.area + 2 * 4 * sh.tm);
+#define KK_CONV_LAUNCH(...) rc = A.resid ? conv_launch(conv_i8_kernel<__VA_ARGS__, true, false>, grid, lds, A) \
+                                         : conv_launch(conv_i8_kernel<__VA_ARGS__, false, false>, grid, lds, A)
+      // Rows of odd length into an output that the last-level cache does not
+      // hold: 16-byte stores through LDS ([1,128,405841] k11 114.4 -> 109.6
+      // us, with leaf sums 113.7 -> 107.3; into 69 MB, [1,256,67641] k7, they
+      // cost 2.6 us).  With a residual they never paid.
+      const bool beyond_llc = N * Cout * Lout * 4 > (int64_t{128} << 20);
+      if (sh.tn == 128 && !A.resid && Lout % 2 != 0 && beyond_llc)
+        rc = conv_launch(conv_i8_kernel<2, 2, 1, 2, 3, false, true>, grid, lds, A);
+      else if (sh.tn == 128) KK_CONV_LAUNCH(2, 2, 1, 2, 3);
+      else if (sh.tm == 128) KK_CONV_LAUNCH(2, 2, 1, 1, 3);
+      else KK_CONV_LAUNCH(1, 1, 4, 2, 6);
+#undef KK_CONV_LAUNCH
     }
   }
   if (own_ws) kk_free(ws);  // stream order keeps the workspace alive for the kernels
@@ -974,8 +1146,7 @@ int kk_conv_integer_scaled_qbias_packed_leaves(
     if (leaves->dtype != KK_F32 || !is_contiguous(leaves) || numel(leaves) != rows * nleaf)
       return set_error(KK_E_ARG, "%s: leaves must be %lld contiguous fp32 values", who,
                        (long long)(rows * nleaf));
-    if (conv_leaf_off(static_cast<int>(conv_rows(128, stride, dilation, w->shape[2]))) +
-            kLeafBytes > 65536)
+    if (!conv_leaves_fit(stride, dilation, w->shape[2]))
       return set_error(KK_E_UNSUPPORTED, "%s: the 128-step tile's window does not fit LDS", who);
   }
   if (empty) return KK_OK;

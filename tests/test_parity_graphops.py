@@ -291,6 +291,27 @@ def brute_conv_integer(x, w, xzp, wzp, pad, dil):
     return out[None]
 
 
+@pytest.mark.parametrize("n,cin,L,pad,dil,skip", [
+    (1, 1, 1, 1, 1, 0), (1, 1, 3, 2, 1, 1), (1, 3, 1, 1, 1, 2), (1, 1, 4, 1, 1, 1), (1, 1, 5, 7, 3, 3),
+    (2, 3, 127, 3, 3, 0), (2, 65, 129, 1, 1, 1), (1, 64, 130, 25, 5, 0), (1, 67, 131, 0, 1, 3),
+    (1, 64, 132, 1, 1, 2), (3, 128, 255, 5, 5, 1)])
+def test_conv_integer_rows_at_any_alignment(gpu, n, cin, L, pad, dil, skip):
+    """Rows of odd lengths, and activations `skip` bytes off a dword: whole
+    dwords are loaded wherever a row starts, padding falls inside a dword,
+    and the last row ends with the tensor.  Exact, against brute force."""
+    r = rng(29)
+    x = r.integers(0, 256, (n, cin, L)).astype(np.uint8)
+    w = r.integers(0, 256, (34, cin, 3)).astype(np.uint8)
+    xz, wz = np.array(17, np.uint8), np.array(201, np.uint8)
+    flat = gpu.to_device(np.concatenate([np.zeros(skip, np.uint8), x.ravel()]))
+    dx = flat.slice_axis(0, skip, skip + x.size).reshape(x.shape)
+    assert dx.ptr % 4 == skip % 4
+    got = gpu.ops.conv_integer(dx, gpu.to_device(w), gpu.to_device(xz), gpu.to_device(wz), (pad, pad),
+                               1, dil).numpy()
+    want = np.concatenate([brute_conv_integer(x[i:i + 1], w, xz, wz, pad, dil) for i in range(n)])
+    assert_bitexact(got, want.astype(np.int32), f"ConvInteger L={L} skip={skip}")
+
+
 def test_conv_integer_exact_beyond_2_24(gpu, oracle):
     """Sums above 2^24: the device is exact int32 (int8 matrix cores), while
     the reference convolves the shifted integers in float32 and rounds
