@@ -650,9 +650,7 @@ static int launch_q(const CArgs& a, int W, int64_t batch) {
                   static_cast<unsigned>(batch));
   KK_TRY(check_xcd_grid(grid, "convq_kernel"));
   const int lds = std::max(4 * W * kQPitch, kQExchange);
-  // (a kernel needs the attribute for more than 64 KB of dynamic LDS)
-  KK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(convq_kernel<T, NP>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+  if (lds > 65536) KK_TRY(allow_large_lds(reinterpret_cast<const void*>(convq_kernel<T, NP>)));
   KK_LAUNCH((convq_kernel<T, NP>), grid, dim3(kThreads), static_cast<size_t>(lds), ctx().stream, a, W);
   return check_launch("convq_kernel");
 }

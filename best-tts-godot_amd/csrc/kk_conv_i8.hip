@@ -769,9 +769,7 @@ static int check_conv_integer(const kk_tensor* out, const kk_tensor* x, const kk
 }
 
 static int conv_launch(void (*kernel)(ConvI8Args), const dim3& grid, size_t lds, const ConvI8Args& A) {
-  if (lds > 65536)  // (the widest windows; a kernel needs the attribute for more)
-    KK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+  if (lds > 65536) KK_TRY(allow_large_lds(reinterpret_cast<const void*>(kernel)));
   KK_LAUNCH(kernel, grid, dim3(256), lds, ctx().stream, A);
   return check_launch("conv_i8_kernel");
 }

@@ -487,6 +487,14 @@ int zp_shift(Dequant* d, const kk_tensor* zp, int64_t count, const char* who);
 
 
 
+// More than 64 KB of dynamic LDS: a kernel needs the attribute (always the
+// same value, so that threads launching one kernel do not undercut each other).
+constexpr int kDynLdsMax = 155648;
+inline int allow_large_lds(const void* kernel) {
+  KK_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kDynLdsMax));
+  return KK_OK;
+}
+
 // A workgroup barrier that orders LDS only: global loads and stores stay
 // in flight across it, where __syncthreads would wait for them.
 __device__ __forceinline__ void lds_barrier() {
