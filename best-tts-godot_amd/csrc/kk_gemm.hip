@@ -376,6 +376,10 @@ struct GemmArgs {
   int splits;
   float* part;
   const void* bpack;   // B packed by kk_gemm_pack (the bf16 matrix-core path), or NULL
+  // bytes from one batch item's scale / zero point to the next's (0: shared);
+  // with per_item, tiles and splits are chosen as for one item
+  int64_t scale_bytes, zp_bytes;
+  bool per_item;
 };
 
 // A kinds: 0 = K-contiguous quads of TA, 1 = scalar gather.
@@ -400,6 +404,9 @@ __global__ void __launch_bounds__(kNT) gemm_kernel(GemmArgs G) {
     else out[m * som + n * son] = alpha == 1.0f ? v : v * alpha;
   };
   const Dequant none{};  // fp32 activations: no per-row dequantisation
+  Dequant dq = G.dq;     // this item's
+  if (dq.scale) dq.scale = static_cast<const char*>(dq.scale) + bz * G.scale_bytes;
+  if (dq.zp) dq.zp = static_cast<const char*>(dq.zp) + bz * G.zp_bytes;
   // this split's K-steps
   const int64_t nk_all = ceil_div(K, kBK), chunk = ceil_div(nk_all, splits);
   const int64_t kt0 = split * chunk, kt1 = std::min<int64_t>(nk_all, kt0 + chunk);
@@ -410,13 +417,13 @@ __global__ void __launch_bounds__(kNT) gemm_kernel(GemmArgs G) {
   auto getB = [&](int64_t k, int64_t n) -> float {
     if (k >= K || n >= N) return 0.0f;
     const float q = load_as_f32(G.b, G.b_dt, ob + k * G.b_si + n * G.b_sj);
-    return G.dq.active ? dequant_value(q, G.dq, n) : q;
+    return dq.active ? dequant_value(q, dq, n) : q;
   };
   if constexpr (AK == 0 && BK == 0) {
     AQuad<C, TA> la;
     la.init(static_cast<const TA*>(G.a) + oa, G.a_si, M, K, m0, none);
     BQuad<C, TB> lb;
-    lb.init(static_cast<const TB*>(G.b) + ob, G.b_si, N, K, n0, G.dq);
+    lb.init(static_cast<const TB*>(G.b) + ob, G.b_si, N, K, n0, dq);
     gemm_run<C>(la, lb, store, M, N, K, m0, n0, kt0, kt1);
   } else if constexpr (AK == 0) {
     AQuad<C, TA> la;
@@ -430,7 +437,7 @@ __global__ void __launch_bounds__(kNT) gemm_kernel(GemmArgs G) {
     }
   } else if constexpr (BK == 0) {
     BQuad<C, TB> lb;
-    lb.init(static_cast<const TB*>(G.b) + ob, G.b_si, N, K, n0, G.dq);
+    lb.init(static_cast<const TB*>(G.b) + ob, G.b_si, N, K, n0, dq);
     if (G.a_si == 1) {
       AScalar<C, decltype(getA), false> la{getA, m0};
       gemm_run<C>(la, lb, store, M, N, K, m0, n0, kt0, kt1);
@@ -786,7 +793,7 @@ static int conv_common(const kk_tensor* out, const kk_tensor* x, const kk_tensor
 // (the fp32 matrix cores); else 8-bit and fp16 weights may take the bf16
 // matrix cores, which scale the exact sum instead.
 static int launch_gemm(const GemmArgs& args, int64_t batch, bool weights_rounded = false) {
-  if (args.N <= kSkinnyN && args.K <= kSkinnyK && args.M * batch >= 4096) {
+  if (!args.per_item && args.N <= kSkinnyN && args.K <= kSkinnyK && args.M * batch >= 4096) {
     const int64_t rows = args.M * batch;
     const unsigned grid = static_cast<unsigned>(std::min<int64_t>(ceil_div(rows, 256), 1 << 16));
     KK_LAUNCH(gemm_skinny_kernel, dim3(grid), dim3(256), 0, ctx().stream, args, batch);
@@ -801,7 +808,7 @@ static int launch_gemm(const GemmArgs& args, int64_t batch, bool weights_rounded
                     args.alpha, args.only_if, args.bpack, &st))
       return st;
   }
-  const TileSize ts = pick_tile(args.M, args.N, batch);
+  const TileSize ts = pick_tile(args.M, args.N, args.per_item ? 1 : batch);
   dim3 grid = grid_of(ts, args.M, args.N, batch);
   KK_TRY(check_grid(grid, batch));
   // Split K when the tiles leave CUs idle and the K loop is long (each
@@ -810,7 +817,7 @@ static int launch_gemm(const GemmArgs& args, int64_t batch, bool weights_rounded
   GemmArgs args_s = args;
   {
     const int64_t cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
-    const int64_t blocks = static_cast<int64_t>(grid.x) * grid.y * grid.z;
+    const int64_t blocks = static_cast<int64_t>(grid.x) * grid.y * (args.per_item ? 1 : grid.z);
     const int64_t nk = ceil_div(args.K, kBK);
     int64_t S = 1;
     while (S < 8 && blocks * S < 2 * cus && nk / (2 * S) >= 4 &&
@@ -970,6 +977,22 @@ int gemm(const kk_tensor* out, const kk_tensor* a, const kk_tensor* w, const kk_
   if (G.M == 0 || G.N == 0 || batch == 0) return KK_OK;
   if (G.K == 0) return kk_fill(out, 0.0);
   return launch_gemm(G, batch, weights_rounded);
+}
+
+int gemm_items(const kk_tensor* out, const kk_tensor* a, const kk_tensor* w, const kk_tensor* w_scale,
+               const kk_tensor* w_zp, int64_t scale_bytes, int64_t zp_bytes) {
+  const char* who = "gemm_items";
+  GemmArgs G{};
+  int64_t batch = 0;
+  KK_TRY(setup_gemm(&G, out, a, w, &batch, who));
+  KK_TRY(make_dequant(&G.dq, w, w_scale, w_zp, G.N, who));
+  G.alpha = 1.0f;
+  G.scale_bytes = scale_bytes;
+  G.zp_bytes = zp_bytes;
+  G.per_item = true;
+  if (G.M == 0 || G.N == 0 || batch == 0) return KK_OK;
+  if (G.K == 0) return kk_fill(out, 0.0);
+  return launch_gemm(G, batch, true);
 }
 
 }  // namespace kk

@@ -274,7 +274,7 @@ __global__ void __launch_bounds__(kDqlSmallThreads) dql_small(const float* __res
 // multiplies), the sigmoid's division is one Newton step, the zero point's
 // sum of h stays in the VALU (its LDS shuffles were 0.5 us a step where
 // R's zero point is not 0), and R is packed through LDS in words at set-up.
-// Bidirectional, 640 -> 256, the whole call: 130 steps 254 -> 189 us.
+// Bidirectional, 640 -> 256, the whole call: 130 steps 254 -> 183 us.
 constexpr int kLstmThreads = 1024;
 constexpr int kLstmMaxH = kLstmThreads / 4;
 // Steps per chunk of the input projections: a chunk (4 rows of 4H floats,
@@ -884,7 +884,9 @@ int kk_lstm(const kk_tensor* ys, const kk_tensor* yh, const kk_tensor* yc, const
       KK_TRY(f32_contig(t, "state"));
       if (numel(t) != ndir * batch * H) return set_error(KK_E_ARG, "kk_lstm: state shape");
     }
-  // Input projections xw[d] = x @ deq(W[d]) on the MFMA GEMM; the recurrence
+  // Input projections xw[d] = x @ deq(W[d]), every direction in one launch
+  // (and one that adds the splits: at 130 steps a direction's two took 14
+  // us, waiting on loads with a third of the CUs idle); the recurrence
   // adds wb[d] + rb[d] (summed first, as op_lstm does) to each step's row as
   // it reads it, which two elementwise passes a direction did before.
   void* xw = nullptr;
@@ -892,25 +894,23 @@ int kk_lstm(const kk_tensor* ys, const kk_tensor* yh, const kk_tensor* yc, const
   const int64_t xw_bytes = ((sizeof(float) * std::max<int64_t>(xw_n, 1) + 255) / 256) * 256;
   KK_TRY(kk_alloc(static_cast<size_t>(xw_bytes), &xw));
   int rc = KK_OK;
-  for (int64_t d = 0; d < ndir && rc == KK_OK && seq * batch > 0; ++d) {
+  if (seq * batch > 0) {
     kk_tensor a{}, wd{}, o{}, sc{}, zpt{};
     a.data = x->data; a.dtype = KK_F32; a.rank = 2;
     a.shape[0] = seq * batch; a.shape[1] = in; a.strides[0] = in; a.strides[1] = 1;
-    wd.data = static_cast<int8_t*>(w->data) + d * in * 4 * H; wd.dtype = KK_I8; wd.rank = 2;
-    wd.shape[0] = in; wd.shape[1] = 4 * H; wd.strides[0] = 4 * H; wd.strides[1] = 1;
-    o.data = static_cast<float*>(xw) + d * seq * batch * 4 * H; o.dtype = KK_F32; o.rank = 2;
-    o.shape[0] = seq * batch; o.shape[1] = 4 * H; o.strides[0] = 4 * H; o.strides[1] = 1;
-    sc.data = static_cast<char*>(w_scale->data) + (nws > 1 ? d * dtype_size(w_scale->dtype) : 0);
-    sc.dtype = w_scale->dtype; sc.rank = 0;
-    const kk_tensor* zptr = nullptr;
-    if (w_zp) {
-      zpt.data = static_cast<char*>(w_zp->data) + (numel(w_zp) > 1 ? d * dtype_size(w_zp->dtype) : 0);
-      zpt.dtype = w_zp->dtype; zpt.rank = 0;
-      zptr = &zpt;
-    }
+    auto per_dir = [&](kk_tensor* t, void* data, int dtype, int64_t rows) {
+      t->data = data; t->dtype = dtype; t->rank = 3;
+      t->shape[0] = ndir; t->shape[1] = rows; t->shape[2] = 4 * H;
+      t->strides[0] = rows * 4 * H; t->strides[1] = 4 * H; t->strides[2] = 1;
+    };
+    per_dir(&wd, w->data, KK_I8, in);
+    per_dir(&o, xw, KK_F32, seq * batch);
+    sc.data = w_scale->data; sc.dtype = w_scale->dtype; sc.rank = 0;
+    if (w_zp) { zpt.data = w_zp->data; zpt.dtype = w_zp->dtype; zpt.rank = 0; }
     // the recurrence amplifies the projection's rounding: keep numpy's
     // (each dequantised weight rounded to fp32, exact fp32 products)
-    rc = gemm(&o, &a, &wd, &sc, zptr, 1.0f, true);
+    rc = gemm_items(&o, &a, &wd, &sc, w_zp ? &zpt : nullptr, nws > 1 ? dtype_size(w_scale->dtype) : 0,
+                    w_zp && numel(w_zp) > 1 ? dtype_size(w_zp->dtype) : 0);
   }
   if (rc == KK_OK) {
     LstmArgs A{};

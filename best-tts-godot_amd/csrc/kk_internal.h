@@ -444,6 +444,12 @@ int matmul_shape(const kk_tensor* out, const kk_tensor* a, const kk_tensor* w, B
 int gemm(const kk_tensor* out, const kk_tensor* a, const kk_tensor* w, const kk_tensor* w_scale,
          const kk_tensor* w_zp, float alpha, bool weights_rounded,
          const kk_tensor* packed = nullptr);
+// out[i] = a @ deq(w[i]) in one launch, each item with its own per-tensor scale
+// and zero point (scale_bytes, zp_bytes after the one before; 0: shared), on
+// the fp32 matrix cores with numpy's rounding of each weight.  Tiles and
+// splits are those of one item alone, so the results are too.
+int gemm_items(const kk_tensor* out, const kk_tensor* a, const kk_tensor* w, const kk_tensor* w_scale,
+               const kk_tensor* w_zp, int64_t scale_bytes, int64_t zp_bytes);
 // out = A @ dequant(B) on the bf16 matrix cores (kk_gemm_dq.hip) when the
 // operands fit: fp32 A with K contiguous, int8/uint8 B (zero point of the
 // same type) or fp16 B with N contiguous.  Returns false, launching nothing,
