@@ -106,59 +106,41 @@ __global__ void __launch_bounds__(kThreads) fir_kernel(const float* __restrict__
   }
 }
 
-// The FIR on the matrix cores, for kMfmaMinTaps .. kMfmaTaps taps (the split
-// copies of the taps take 54 KB of LDS at 1023; below 256 taps forming them
-// costs more than the sum: 128 taps over 1,060,000 samples 12.2 us, 10.4 on
-// the VALU, 513 taps 19.1 and 29.4).  Outputs in tiles of
-// 32 x 32, y[o + 32 i + r] = sum_s T[r][s] x[o + 32 i + s] with the Toeplitz
-// matrix T[r][s] = h[s - r] (0 outside the filter): taps + 31 terms of which
-// taps count, 3% more at 1023 taps.  Samples and taps are split into three
-// bf16 parts (round to nearest, exact: 3 x 8 significant bits) and the six
-// products of parts above 2^-26 of the whole run on
-// v_mfma_f32_32x32x16_bf16 (2.5 PF/s dense, so 417 TF/s of fp32-accurate work
-// against 79 on the VALU); the sum of the leading products and that of the
-// other five are kept apart until the end.  Its 66 steps round less than the
-// chain of 1023 fused multiply-adds: the notch filter's relative error
-// against 64 bits is 2.1e-7 (6.8e-8 with the sum shared by four waves)
-// where that chain's is 5.7e-7, 1.2e-7 against 4.0e-7 at 513 taps and 2.3e-7
-// against 7.0e-7 at 1536.  Measured, 1023 taps: 2,029,200 samples 67.4 ->
-// 31.5 us (PCM16 65 -> 30), 400,000 33.8 -> 12.9, 2400 32.1 -> 8.3; bound by
-// LDS reads and their latency (nine fragments for twelve matrix
-// instructions, one wave a SIMD), the products alone taking 10.5 us.
+// The FIR on the fp32 matrix cores, for kMfmaMinTaps taps and more.  Outputs in
+// tiles of 16 x 16, y[o + 16 i + r] = sum_s T[r][s] x[o + 16 i + s] with the
+// Toeplitz matrix T[r][s] = h[s - r] (0 outside the filter): taps + 15 terms
+// of which taps count, 1.5% more at 1023 taps.  v_mfma_f32_16x16x4_f32 adds
+// its four terms one after another, each a fused multiply-add, so an output
+// is the chain of the kernel above, bit for bit (the zeros before and after
+// its taps leave it as it is), at twice the VALU's fp32 rate.  (On the bf16
+// matrix cores, samples and taps split in three, it took 31 us; its sums are
+// closer to 64 bits, but another rounding than the chain's puts 0.23% of the
+// PCM16 samples on another step.)
 //
-// LDS: the taps in eight copies shifted by 0 .. 7 (row r of T reads copy
-// r % 8, so every operand fragment is one aligned 16-byte read), and the
-// block's window of x, in units of eight bf16 dealt round over four regions,
-// so the 32 columns of a fragment -- four units apart in time -- read
-// consecutive units.
+// Lane (n, g) = (lane % 16, lane / 16) holds row / column n of k = g, i.e.
+// the terms s = 4 j + g of steps j, so the window is kept as four sequences of
+// every fourth sample and a lane reads four steps at once; column n's unit of
+// four is n after column 0's.  The taps likewise, in four copies shifted by 0
+// .. 3 units' quarters, so that row r's reads are aligned too; the sixteen
+// sequences start on different banks.
 //
-// A wave takes NC tiles and one of WK shares of the sum; with WK = 4 the four
-// waves' partial tiles are added through LDS in wave order.  Where an output
-// is not finite (an infinity or NaN in its tile's window, or a sample above
-// bf16's range), it is formed again as the kernel above does.
-constexpr int kMfmaMinTaps = 256, kMfmaTaps = 1536;
-typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
-typedef float f16v __attribute__((ext_vector_type(16)));
+// Bound by the matrix cores (2,029,200 samples x 1023 taps: 27.7 us at their
+// rate).  A wave takes NC tiles, which share the taps' reads.  Measured, 1023
+// taps: 2,029,200 samples 67.4 -> 40.0 us (PCM16 65.1 -> 38.8), 1,060,000
+// 52.7 -> 29.5, 400,000 33.8 -> 14.2, 2400 32.1 -> 10.3; 64 taps over
+// 1,060,000 7.1 either way, over 24,000 5.2 -> 3.8.
+constexpr int kMfmaMinTaps = 32;
+typedef float fir_f4 __attribute__((ext_vector_type(4)));
 
-__host__ __device__ constexpr int fir_steps(int taps, int wk) {  // of 16 terms, a multiple of wk
-  return ((taps + 31 + 15) / 16 + wk - 1) / wk * wk;
+__host__ __device__ constexpr int fir_units(int taps) { return (taps + 15 + 15) / 16; }  // of four steps
+// 16-byte units of a sequence of taps (= 1 mod 16) and of samples (= 4 mod 16:
+// the window's writes fall on all banks)
+__host__ __device__ constexpr int fir_tap_pitch(int units) { return (units + 15) / 16 * 16 + 1; }
+__host__ __device__ constexpr int fir_win_pitch(int tile, int units) {
+  return (tile / 16 + units - 4 + 15) / 16 * 16 + 4;
 }
-// units a copy of the taps takes: -3 .. 2 steps - 1; = 4 mod 16 (the copies
-// of a row octet fall on different banks)
-__host__ __device__ constexpr int fir_tap_pitch(int steps) { return (2 * steps + 3 - 4 + 15) / 16 * 16 + 4; }
-// units of a region of the window (a quarter of the window's)
-__host__ __device__ constexpr int fir_win_pitch(int tile, int steps) { return (tile / 8 + 2 * steps + 3) / 4; }
-__host__ __device__ constexpr int fir_lds(int tile, int steps, int wk) {
-  const int w = 3 * 4 * fir_win_pitch(tile, steps) * 16, red = wk > 1 ? wk * tile * 4 : 0;
-  return 3 * 8 * fir_tap_pitch(steps) * 16 + (w > red ? w : red);
-}
-
-// v = p[0] + p[1] + p[2] (up to 2^-26 of v), each a bf16
-__device__ __forceinline__ void split3(float v, __bf16 (&p)[3]) {
-  p[0] = static_cast<__bf16>(v);
-  const float r1 = v - static_cast<float>(p[0]);
-  p[1] = static_cast<__bf16>(r1);
-  p[2] = static_cast<__bf16>(r1 - static_cast<float>(p[1]));
+__host__ __device__ constexpr int fir_lds(int tile, int units) {
+  return 16 * (16 * fir_tap_pitch(units) + 4 * fir_win_pitch(tile, units));
 }
 
 // one output from its own samples, taps in order
@@ -173,147 +155,93 @@ __device__ __attribute__((noinline)) float fir_direct(const float* x, int64_t n,
   return acc;
 }
 
-template <int NC, int WK, bool PCM>
+template <int NC, bool PCM>
 __global__ void __launch_bounds__(kThreads) fir_mfma_kernel(const float* __restrict__ x, int64_t n,
                                                             const float* __restrict__ h, int taps,
                                                             int center, float* __restrict__ y,
                                                             int16_t* __restrict__ pcm, float gain) {
-  constexpr int kOut = 1024 * NC * (4 / WK);  // outputs per block
+  constexpr int kOut = 256 * NC * 4;  // outputs per block
   extern __shared__ __align__(16) unsigned char fir_mem[];
-  const int steps = fir_steps(taps, WK), VP = fir_tap_pitch(steps), XP = fir_win_pitch(kOut, steps);
-  bf8* ht = reinterpret_cast<bf8*>(fir_mem);  // [part][copy][VP]
-  bf8* xt = ht + 3 * 8 * VP;                  // [part][unit % 4][XP]
+  const int units = fir_units(taps), VP = fir_tap_pitch(units), XP = fir_win_pitch(kOut, units);
+  float* ht = reinterpret_cast<float*>(fir_mem);  // [s % 4][copy][4 VP]
+  float* xt = ht + 16 * 4 * VP;                   // [s % 4][4 XP]
   const int64_t i0 = static_cast<int64_t>(blockIdx.x) * kOut;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // the window: unit u holds samples i0 - center + 8 u ..
-  for (int u = tid; u < 4 * XP; u += kThreads) {
-    bf8 q[3];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      int64_t s = i0 - center + 8 * u + e;
-      s = s < 0 ? 0 : (s >= n ? n - 1 : s);
-      __bf16 p[3];
-      split3(x[s], p);
-#pragma unroll
-      for (int k = 0; k < 3; ++k) q[k][e] = p[k];
-    }
-#pragma unroll
-    for (int k = 0; k < 3; ++k) xt[(k * 4 + (u & 3)) * XP + (u >> 2)] = q[k];
+  // the window: samples i0 - center + t
+  const int span = kOut + 16 * units;
+#pragma unroll 4
+  for (int t = tid; t < span; t += kThreads) {
+    int64_t s = i0 - center + t;
+    s = s < 0 ? 0 : (s >= n ? n - 1 : s);
+    xt[(t & 3) * 4 * XP + (t >> 2)] = x[s];
   }
-  // the taps: copy c, unit v holds h[8 (v - 3) - c + 0 .. 7]
-  for (int it = tid; it < 8 * VP; it += kThreads) {
-    const int c = it & 7, v = it >> 3, k0 = 8 * (v - 3) - c;
-    bf8 q[3];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int k = k0 + e;
-      __bf16 p[3];
-      split3(k >= 0 && k < taps ? h[k] : 0.0f, p);
-#pragma unroll
-      for (int t = 0; t < 3; ++t) q[t][e] = p[t];
-    }
-#pragma unroll
-    for (int t = 0; t < 3; ++t) ht[(t * 8 + c) * VP + v] = q[t];
+  // copy c of residue q: place m holds h[4 (m - 4 - c) + q]
+#pragma unroll 4
+  for (int it = tid; it < 16 * 4 * (units + 1); it += kThreads) {
+    const int a = it & 15, m = it >> 4, q = a >> 2, c = a & 3;
+    const int k = 4 * (m - 4 - c) + q;
+    ht[a * 4 * VP + m] = k >= 0 && k < taps ? h[k] : 0.0f;
   }
   __syncthreads();
-  const int r = lane & 31, g = lane >> 5;
-  const int kp = wv % WK, o_w = (wv / WK) * 1024 * NC;  // this wave's share of the sum, its outputs
-  const int per = steps / WK, st0 = kp * per;
-  // lane (r, g) of step st: taps unit 2 st + g - r / 8 (+ 3) of copy r % 8;
-  // window unit o_w / 8 + 128 c + 2 st + g + 4 r of tile c
-  const bf8* ha = ht + (r & 7) * VP + g - (r >> 3) + 3;
-  auto xaddr = [&](int st, int c) {
-    const int u0 = 2 * st + g;
-    return xt + (u0 & 3) * XP + (u0 >> 2) + o_w / 32 + 32 * c + r;
-  };
-  f16v big[NC] = {}, small[NC] = {};
-  bf8 a[2][3], b[2][NC][3];
-  auto fetch = [&](int st, bf8 (&fa)[3], bf8 (&fb)[NC][3]) {
+  const int r = lane & 15, g = lane >> 4;
+  const int o_w = wv * 256 * NC;
+  // row r's term s = 4 j + g is h[4 (j - c) + q], q = (g - r) mod 4
+  const int q = (g - r) & 3, c = (r - g + q) >> 2;  // c = 0 .. 4
+  const fir_f4* ha = reinterpret_cast<const fir_f4*>(ht + (q * 4 + (c & 3)) * 4 * VP) + 1 - (c >> 2);
+  const fir_f4* xa = reinterpret_cast<const fir_f4*>(xt + g * 4 * XP) + o_w / 16 + r;
+  fir_f4 acc[NC] = {};
+  fir_f4 a[2], b[2][NC];
+  auto fetch = [&](int u, int slot) {
+    a[slot] = ha[u];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) fa[k] = ha[k * 8 * VP + 2 * st];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const bf8* p = xaddr(st, c);
-#pragma unroll
-      for (int k = 0; k < 3; ++k) fb[c][k] = p[k * 4 * XP];
-    }
+    for (int t = 0; t < NC; ++t) b[slot][t] = xa[16 * t + u];
   };
-  auto mma = [&](const bf8 (&fa)[3], const bf8 (&fb)[NC][3]) {
-#define KK_FIR_MMA(D, P, Q) \
-  _Pragma("unroll") for (int c = 0; c < NC; ++c) D[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[P], fb[c][Q], D[c], 0, 0, 0)
-    KK_FIR_MMA(small, 2, 0);
-    KK_FIR_MMA(big, 0, 0);
-    KK_FIR_MMA(small, 0, 2);
-    KK_FIR_MMA(small, 1, 1);
-    KK_FIR_MMA(small, 1, 0);
-    KK_FIR_MMA(small, 0, 1);
-#undef KK_FIR_MMA
+  auto mma = [&](int slot) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int t = 0; t < NC; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[slot][e], b[slot][t][e], acc[t], 0, 0, 0);
   };
-  fetch(st0, a[0], b[0]);
-  for (int st = 0; st < per; st += 2) {  // (fetches past the share read its last step again)
-    fetch(st0 + min(st + 1, per - 1), a[1], b[1]);
-    mma(a[0], b[0]);
-    if (st + 1 < per) {
-      fetch(st0 + min(st + 2, per - 1), a[0], b[0]);
-      mma(a[1], b[1]);
+  fetch(0, 0);
+  for (int u = 0; u < units; u += 2) {  // (fetches past the last unit read it again)
+    fetch(min(u + 1, units - 1), 1);
+    mma(0);
+    if (u + 1 < units) {
+      fetch(min(u + 2, units - 1), 0);
+      mma(1);
     }
   }
-  // D(i, j): lane j + 32 ((i / 4) % 2), register (i / 8) 4 + i % 4: four
-  // consecutive outputs a register quad
-  auto put4 = [&](int64_t o, float4 v4) {
-    if (o >= n) return;
-    float v[4] = {v4.x, v4.y, v4.z, v4.w};
+  // D: column lane % 16, rows 4 (lane / 16) + 0 .. 3: four consecutive outputs a lane
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
-      if (!(fabsf(v[t]) < INFINITY) && o + t < n) v[t] = fir_direct(x, n, h, taps, o + t - center);
+  for (int t = 0; t < NC; ++t) {
+    const int64_t o = i0 + o_w + 256 * t + 16 * r + 4 * g;
+    if (o >= n) continue;
+    float v[4] = {acc[t][0], acc[t][1], acc[t][2], acc[t][3]};
+    // not finite: an infinity or NaN beside the output's own samples may have
+    // met a zero of T
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (!(fabsf(v[e]) < INFINITY) && o + e < n) v[e] = fir_direct(x, n, h, taps, o + e - center);
     if (o + 4 <= n) {
       if (PCM) {
         uint32_t w[2];
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-          w[t] = static_cast<uint16_t>(to_pcm16(v[2 * t], gain)) |
-                 (static_cast<uint32_t>(static_cast<uint16_t>(to_pcm16(v[2 * t + 1], gain))) << 16);
+        for (int e = 0; e < 2; ++e)
+          w[e] = static_cast<uint16_t>(to_pcm16(v[2 * e], gain)) |
+                 (static_cast<uint32_t>(static_cast<uint16_t>(to_pcm16(v[2 * e + 1], gain))) << 16);
         *reinterpret_cast<uint2*>(pcm + o) = make_uint2(w[0], w[1]);
       } else {
-        *reinterpret_cast<float4*>(y + o) = make_float4(v[0], v[1], v[2], v[3]);
+        st_stream4(y + o, make_float4(v[0], v[1], v[2], v[3]));
       }
     } else {
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-        if (o + t < n) {
-          if (PCM) pcm[o + t] = to_pcm16(v[t], gain);
-          else y[o + t] = v[t];
+      for (int e = 0; e < 4; ++e)
+        if (o + e < n) {
+          if (PCM) pcm[o + e] = to_pcm16(v[e], gain);
+          else y[o + e] = v[e];
         }
-    }
-  };
-  if constexpr (WK == 1) {
-#pragma unroll
-    for (int c = 0; c < NC; ++c)
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        put4(i0 + o_w + 1024 * c + 32 * r + 8 * q + 4 * g,
-             make_float4(big[c][4 * q] + small[c][4 * q], big[c][4 * q + 1] + small[c][4 * q + 1],
-                         big[c][4 * q + 2] + small[c][4 * q + 2], big[c][4 * q + 3] + small[c][4 * q + 3]));
-  } else {
-    __syncthreads();  // every wave is done with the window
-    float4* red = reinterpret_cast<float4*>(xt);  // [wave][outputs / 4]
-#pragma unroll
-    for (int c = 0; c < NC; ++c)
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        red[kp * (kOut / 4) + o_w / 4 + 256 * c + 8 * r + 2 * q + g] =
-            make_float4(big[c][4 * q] + small[c][4 * q], big[c][4 * q + 1] + small[c][4 * q + 1],
-                        big[c][4 * q + 2] + small[c][4 * q + 2], big[c][4 * q + 3] + small[c][4 * q + 3]);
-    __syncthreads();
-    for (int t = tid; t < kOut / 4; t += kThreads) {
-      float4 v = red[t];
-#pragma unroll
-      for (int w = 1; w < WK; ++w) {
-        const float4 p = red[w * (kOut / 4) + t];
-        v = make_float4(v.x + p.x, v.y + p.y, v.z + p.z, v.w + p.w);
-      }
-      put4(i0 + 4 * t, v);
     }
   }
 }
@@ -375,18 +303,15 @@ static int check_taps(const kk_tensor* taps, int* center, const char* who) {
   return KK_OK;
 }
 
-template <int NC, int WK, bool PCM>
+template <int NC, bool PCM>
 static int launch_mfma(const float* x, int64_t n, const float* h, int taps, int center, float* y,
                        int16_t* pcm, float gain) {
-  constexpr int kOut = 1024 * NC * (4 / WK);
+  constexpr int kOut = 256 * NC * 4;
   const int64_t blocks = ceil_div(n, kOut);
   if (blocks > 0x7fffffff) return set_error(KK_E_UNSUPPORTED, "FIR: waveform too long");
-  const size_t lds = static_cast<size_t>(fir_lds(kOut, fir_steps(taps, WK), WK));
-  // above 64 KB of dynamic LDS a kernel needs the attribute (per device: set
-  // on each call, a host-side store)
-  KK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(fir_mfma_kernel<NC, WK, PCM>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-  KK_LAUNCH((fir_mfma_kernel<NC, WK, PCM>), dim3(static_cast<unsigned>(blocks)), dim3(kThreads), lds,
+  const size_t lds = static_cast<size_t>(fir_lds(kOut, fir_units(taps)));
+  if (lds > 65536) KK_TRY(allow_large_lds(reinterpret_cast<const void*>(fir_mfma_kernel<NC, PCM>)));
+  KK_LAUNCH((fir_mfma_kernel<NC, PCM>), dim3(static_cast<unsigned>(blocks)), dim3(kThreads), lds,
             ctx().stream, x, n, h, taps, center, y, pcm, gain);
   return check_launch("fir_mfma_kernel");
 }
@@ -397,19 +322,22 @@ static int launch_fir(const kk_tensor* x, const kk_tensor* taps, int center, flo
   const float* xp = static_cast<const float*>(x->data);
   const float* hp = static_cast<const float*>(taps->data);
   const int t = static_cast<int>(numel(taps));
-  if (t >= kMfmaMinTaps && t <= kMfmaTaps) {
-    // 8192 outputs a block, one block a CU (1,500,000 samples 28.9 us) where
-    // its rounds over the CUs are at least two thirds full: it takes as long
-    // at 1,060,000 (27.7 us) and twice as long at 2,154,000 (52 us).  Else
-    // 1024 outputs a block, the waves sharing the sum (1,040,000 samples 23.6
-    // us, 2400 8.3 us).
+  if (t >= kMfmaMinTaps) {
+    // Tiles a wave: the blocks go round the CUs whole, and a block of one,
+    // two or four tiles a wave takes 5.5, 5.1 x 2 or 4.9 x 4 us (1023 taps):
+    // 1,060,000 samples 29.5, 31.4 and 38.3 us, 1,500,000 35.3, 32.5, 39.4,
+    // 2,029,200 45.4, 40.9, 40.6, 2,154,000 48.9, 50.9, 53.9.
     const int64_t cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
-    const int64_t b8 = ceil_div(n, 8192), rounds = ceil_div(b8, cus);
-    if (3 * b8 >= 2 * rounds * cus)
-      return pcm ? launch_mfma<2, 1, true>(xp, n, hp, t, center, y, pcm, gain)
-                 : launch_mfma<2, 1, false>(xp, n, hp, t, center, y, pcm, gain);
-    return pcm ? launch_mfma<1, 4, true>(xp, n, hp, t, center, y, pcm, gain)
-               : launch_mfma<1, 4, false>(xp, n, hp, t, center, y, pcm, gain);
+    auto rounds = [&](int64_t tiles) { return ceil_div(ceil_div(n, 1024 * tiles), cus); };
+    const int64_t c1 = 55 * rounds(1), c2 = 102 * rounds(2), c4 = 196 * rounds(4);
+    auto run = [&](auto nc) {
+      constexpr int kNc = decltype(nc)::value;
+      return pcm ? launch_mfma<kNc, true>(xp, n, hp, t, center, y, pcm, gain)
+                 : launch_mfma<kNc, false>(xp, n, hp, t, center, y, pcm, gain);
+    };
+    if (c4 <= c2 && c4 <= c1) return run(std::integral_constant<int, 4>{});
+    if (c2 <= c1) return run(std::integral_constant<int, 2>{});
+    return run(std::integral_constant<int, 1>{});
   }
   const int64_t blocks = ceil_div(n, kTile);
   if (blocks > 0x7fffffff) return set_error(KK_E_UNSUPPORTED, "FIR: waveform too long");

@@ -43,19 +43,20 @@ def test_fir(gpu, oracle, n, t, c):
 
 
 @pytest.mark.parametrize("n,t,c", [
-    (1, 256, -1), (1023, 256, 0), (1024, 257, 64), (1027, 271, 5), (5000, 1536, 1535), (5000, 1537, 3),
-    (3 * 1024 + 2, 993, 0), (5000, 255, 7), (1500001, 300, 11), (171 * 8192 + 5, 1024, 1023)])
+    (1, 32, -1), (1023, 33, 0), (1024, 49, 48), (1027, 271, 5), (5000, 1536, 1535), (5000, 4096, 3),
+    (3 * 1024 + 2, 993, 0), (255, 31, 7), (256 * 4096, 300, 11), (256 * 4096 - 4097, 1023, 1022),
+    (1500001, 64, 0), (2029200, 36, 35)])
 def test_fir_matrix_core_tiles(gpu, oracle, n, t, c):
     """The matrix-core FIR at the edges of its tiles, of its sum's steps and
-    of its range of taps, the bar as above; and a window's infinity, NaN or
-    sample above bf16's largest reaches the outputs that read it, no other."""
+    of its range of taps, the bar as above; and an infinity or NaN reaches
+    the outputs that read it, no other."""
     r = rng(43)
     x = r.normal(0, 0.3, n).astype(np.float32)
     h = r.normal(0, 0.1, t).astype(np.float32)
     cc = (t - 1) // 2 if c < 0 else c
-    for special in (None, np.inf, np.nan, np.float32(3.4e38)):
+    for special in (None, np.inf, np.nan):
         if special is not None:
-            if n > 10000 or not 256 <= t <= 1536:  # (the other kernel pads its last taps)
+            if n > 10000 or t < 32:  # (the other kernel pads its last taps)
                 break
             x[n // 2] = special
         got = gpu.ops.fir(gpu.to_device(x), gpu.to_device(h), c).numpy()
