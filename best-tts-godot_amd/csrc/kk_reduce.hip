@@ -1839,7 +1839,8 @@ struct RedArgs {
   int64_t nout, nred;
 };
 
-__global__ void reduce_generic_kernel(float* __restrict__ out, const float* __restrict__ x,
+constexpr int kRedBatch = 48;
+__global__ void __launch_bounds__(256) reduce_generic_kernel(float* __restrict__ out, const float* __restrict__ x,
                                       RedArgs R, int op) {
   for (int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; t < R.nout;
        t += static_cast<int64_t>(gridDim.x) * blockDim.x) {
@@ -1852,26 +1853,55 @@ __global__ void reduce_generic_kernel(float* __restrict__ out, const float* __re
     float m = -INFINITY;
     bool nan = false;
     if (R.rr == 1) {
-      // One reduced axis: sixteen independent loads in flight, then added
-      // (or compared) in order.
-      const int64_t st = R.rst[0];
-      int64_t j = 0;
-      for (; j + 16 <= R.nred; j += 16) {
-        float v[16];
+      // One reduced axis: its terms are added (or compared) in order, one
+      // thread an output, so the time is that of the loads' round trips:
+      // kRedBatch loads are in flight while the batch before is added (16 at
+      // a time, each waited for, before: [1,3380,512] over its middle axis 60
+      // -> 48 us, 512 rows of 3380 of a view 364 -> 37).
+      const int64_t st = R.rst[0], last = R.nred - 1;
+      float v[kRedBatch], w[kRedBatch];
+      auto load = [&](int64_t j, float (&d)[kRedBatch]) {  // (past the end: the last term again)
+        if (j + kRedBatch <= R.nred) {
+          const float* p = x + base + j * st;
+          if (st == 1) {  // a row of a view: a line a lane, 16 bytes of it at a time
 #pragma unroll
-        for (int u = 0; u < 16; ++u) v[u] = x[base + (j + u) * st];
+            for (int u = 0; u < kRedBatch; u += 4) {
+              const kk_f4u q = *reinterpret_cast<const kk_f4u*>(p + u);
 #pragma unroll
-        for (int u = 0; u < 16; ++u) {
-          s += v[u];
-          nan |= __builtin_isnan(v[u]);
-          m = fmaxf(m, v[u]);
+              for (int e = 0; e < 4; ++e) d[u + e] = q[e];
+            }
+          } else {
+#pragma unroll
+            for (int u = 0; u < kRedBatch; ++u, p += st) d[u] = *p;
+          }
+        } else {
+#pragma unroll
+          for (int u = 0; u < kRedBatch; ++u) d[u] = x[base + min(j + u, last) * st];
         }
-      }
-      for (; j < R.nred; ++j) {
-        const float v = x[base + j * st];
-        s += v;
-        nan |= __builtin_isnan(v);
-        m = fmaxf(m, v);
+      };
+      auto add = [&](int64_t j, const float (&d)[kRedBatch]) {
+        const int n = static_cast<int>(R.nred - j < kRedBatch ? R.nred - j : kRedBatch);
+        if (op == KK_REDUCE_MAX) {
+#pragma unroll
+          for (int u = 0; u < kRedBatch; ++u) {  // (a repeated term changes nothing)
+            nan |= __builtin_isnan(d[u]);
+            m = fmaxf(m, d[u]);
+          }
+        } else if (n == kRedBatch) {
+#pragma unroll
+          for (int u = 0; u < kRedBatch; ++u) s += d[u];
+        } else {
+#pragma unroll
+          for (int u = 0; u < kRedBatch; ++u)
+            if (u < n) s += d[u];
+        }
+      };
+      if (R.nred > 0) load(0, v);
+      for (int64_t j = 0; j < R.nred; j += 2 * kRedBatch) {
+        load(j + kRedBatch, w);
+        add(j, v);
+        load(j + 2 * kRedBatch, v);
+        if (j + kRedBatch < R.nred) add(j + kRedBatch, w);
       }
     }
     for (int64_t j = 0; j < R.nred && R.rr != 1; ++j) {
@@ -2685,8 +2715,10 @@ int kk_reduce(int op, const kk_tensor* out, const kk_tensor* x, uint32_t axes_ma
                     static_cast<const float*>(x->data), nout, nred, op);
     return check_launch("reduce_rows_kernel");
   }
-  const unsigned grid = static_cast<unsigned>(std::min<int64_t>(ceil_div(nout, 256), 65535));
-  KK_LAUNCH(reduce_generic_kernel, dim3(grid), dim3(256), 0, ctx().stream,
+  // few outputs: a wave a block, over more CUs
+  const int64_t threads = nout <= 64 * 256 ? 64 : 256;
+  const unsigned grid = static_cast<unsigned>(std::min<int64_t>(ceil_div(nout, threads), 65535));
+  KK_LAUNCH(reduce_generic_kernel, dim3(grid), dim3(static_cast<unsigned>(threads)), 0, ctx().stream,
                      static_cast<float*>(out->data), static_cast<const float*>(x->data), R, op);
   return check_launch("reduce_generic_kernel");
 }

@@ -230,3 +230,25 @@ def test_reduce(gpu, oracle, op, shape, axes, keep):
         assert_bitexact(got, oenv["y"], f"{op} {shape} {axes}")
     else:
         assert_close(got, oenv["y"], RTOL, ATOL, floor_rel=1e-6, what=f"{op} {shape} {axes}")
+
+
+@pytest.mark.parametrize("op", ["ReduceMean", "ReduceSum", "ReduceMax"])
+@pytest.mark.parametrize("rows,n,cols", [(1, 1, 5), (2, 47, 70), (1, 48, 512), (3, 49, 64), (1, 96, 65),
+                                         (1, 97, 3), (2, 145, 33), (1, 3380, 512), (300, 50, 64)])
+def test_reduce_strided_axis(gpu, op, rows, n, cols):
+    """One axis that is not the last, around the batches its terms are loaded
+    in: numpy adds such an axis in order, in fp32 (its maximum keeps NaN)."""
+    r = rng(47)
+    x = r.normal(0, 1, (rows, n, cols)).astype(np.float32)
+    if op == "ReduceMax":
+        x[0, n // 2, 1] = np.nan
+    got = gpu.ops.reduce(op, gpu.to_device(x), [1]).numpy()
+    if op == "ReduceMax":
+        want = x.max(axis=1, keepdims=True)
+    else:
+        want = np.zeros((rows, 1, cols), np.float32)
+        for k in range(n):
+            want[:, 0] += x[:, k]
+        if op == "ReduceMean":
+            want = want / np.float32(n)
+    assert_bitexact(got, want, f"{op} [{rows},{n},{cols}]")
