@@ -1065,19 +1065,24 @@ __device__ __forceinline__ float np_block_sum(F f, int m, NpScratch& S) {
   return s;
 }
 
-// Loads elements [0, n) of `src` into the padded LDS row `dst`.
-__device__ __forceinline__ void np_load_row(float* dst, const float* __restrict__ src, int64_t n,
-                                            bool vec) {
-  if (vec) {
-    for (int64_t e = 4 * threadIdx.x; e < n; e += 4 * kNpThreads) {
-      const float4 v = ld_stream4(src + e);
-      *reinterpret_cast<float4*>(dst + np_pad(static_cast<int>(e))) = v;
+// Loads elements [0, n) of `src`, at any float's address, into the padded LDS
+// row `dst`: four 16-byte loads a thread in flight (a load at a time, each
+// waited for, made a row of 7280 four round trips, one of odd length fifteen).
+__device__ __forceinline__ void np_load_row(float* dst, const float* __restrict__ src, int n) {
+  const int n4 = n & ~3, tid = static_cast<int>(threadIdx.x);
+  for (int e0 = 4 * tid; e0 < n4; e0 += 16 * kNpThreads) {
+    kk_f4u v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)  // (past the row's last float4 it is read again)
+      v[u] = *reinterpret_cast<const kk_f4u*>(src + min(e0 + 4 * kNpThreads * u, n4 - 4));
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int e = e0 + 4 * kNpThreads * u;
+      if (e < n4) *reinterpret_cast<float4*>(dst + np_pad(e)) = make_float4(v[u][0], v[u][1], v[u][2], v[u][3]);
     }
-  } else {
-    for (int64_t e = threadIdx.x; e < n; e += kNpThreads) dst[np_pad(static_cast<int>(e))] = ld_stream(src + e);
   }
+  if (tid < n - n4) dst[np_pad(n4 + tid)] = src[n4 + tid];
 }
-
 
 // numpy's pairwise tree over a row's last, partial 8192-block of m
 // elements (0 < m < 8192; nleaf = 0 when the row has none): its leaves
@@ -1196,7 +1201,7 @@ __global__ void __launch_bounds__(kNpThreads) np_rows_kernel(float* __restrict__
   const int64_t row = blockIdx.x;
   const float* xr = x + row * n;
   np_plan_to_lds(tail, P);
-  np_load_row(np_lds, xr, n, vec);
+  np_load_row(np_lds, xr, n);
   __syncthreads();
   const float sum = np_row_sum(np_lds, n, [](float v) { return v; }, S, tail, P);
   if (mode < 2) {
@@ -2240,7 +2245,11 @@ static int instnorm_quant_run(const kk_tensor* q, const kk_tensor* y_scale, cons
   // aligned; the rows held in LDS take 16-byte loads only when T % 4 == 0
   const bool vec = aligned16(x->data) && (reinterpret_cast<uintptr_t>(q->data) % 4 == 0);
   const bool rows_vec = vec && T % 4 == 0;
-  const int64_t per_block = kRowBlock * (vec ? 4 : 1) * 8;
+  // Eight passes a thread, fewer where that leaves fewer than 2048 blocks: each
+  // pass is a round trip ([1,256,7280]: one block a row took seven).
+  int64_t passes = 8;
+  while (passes > 1 && rows * ceil_div(T, kRowBlock * (vec ? 4 : 1) * passes) < 2048) passes /= 2;
+  const int64_t per_block = kRowBlock * (vec ? 4 : 1) * passes;
   const int64_t gx = std::max<int64_t>(1, std::min<int64_t>(ceil_div(T, per_block), 1 << 16));
   const bool long_rows = T > kNpRowMax;
   if (long_rows && rows > kRowCounters)
