@@ -49,7 +49,6 @@ MFMA_PEAKS = {
     "bf16x3": ("bf16 MFMA, activations in 3 bf16 parts (v_mfma_f32_32x32x16_bf16 x3)", 2500.0 / 3),
     "bf16x6": ("bf16 MFMA, activations in 3 bf16 parts, fp16 weights in 2 "
                "(v_mfma_f32_32x32x16_bf16 x6)", 2500.0 / 6),
-    "f16x2": ("fp16 MFMA, activations in 2 fp16 parts (v_mfma_f32_32x32x16_f16 x2)", 1250.0),
     "i8": ("int8 MFMA (v_mfma_i32_32x32x32_i8)", INT8_PEAK_TOPS),
 }
 
@@ -403,7 +402,7 @@ def run_gpu(args):
         pk = kk.ops.conv_pack(wq, None, False, 1)
         rec = per_op(name, lambda i: B.call("kk_conv1d_packed", o[i].desc(), x[i].desc(), wq.desc(),
                                             pk.desc(), sc.desc(), None, None, 1, dil, pad, pad),
-                     flops=2 * cout * cin * k * lout, sets=4, mfma="f16x2")
+                     flops=2 * cout * cin * k * lout, sets=4, mfma="bf16x3")
         # the per-call form (kk_conv1d): the layout made for every call
         fe = lambda i: B.call("kk_conv1d", o[i].desc(), x[i].desc(), wq.desc(), sc.desc(), None,
                               None, 1, dil, pad, pad, 1)
@@ -432,7 +431,7 @@ def run_gpu(args):
     pkt = kk.ops.conv_pack(wt, None, True, 10)
     rec = per_op("convT_i8_512x256_k20_s10", lambda i: B.call(
         "kk_conv_transpose1d_packed", ot[i].desc(), xt[i].desc(), wt.desc(), pkt.desc(), sct.desc(),
-        None, None, 10, 5, 5, 0), flops=2 * 512 * 256 * 2400 * 20 // 10, sets=4, mfma="f16x2")
+        None, None, 10, 5, 5, 0), flops=2 * 512 * 256 * 2400 * 20 // 10, sets=4, mfma="bf16x3")
     fe = lambda i: B.call("kk_conv_transpose1d", ot[i].desc(), xt[i].desc(), wt.desc(), sct.desc(),
                           None, None, 10, 1, 5, 5, 1, 0)
     rec["per_call_us"] = round(B.time_eager(fe, 4, 20) * 1e3, 3)

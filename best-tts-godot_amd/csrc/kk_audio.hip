@@ -4,13 +4,12 @@
 //
 // FIR: y[i] = sum_k h[k] x[clamp(i - center + k, 0, n - 1)], each output's
 // taps accumulated in order (k = 0, 1, ...) in fp32 with one fused
-// multiply-add per tap.  A block of 256 threads computes 2048 consecutive
-// outputs: it stages the input window they read (2048 + taps - 1 samples,
-// edges clamped) in LDS once; each thread keeps a 16-sample register window
-// over its 8 consecutive outputs and slides it 8 taps at a time (two 16-byte
-// LDS reads per 64 FMAs), the taps coming from the scalar cache (the same
-// address in every lane).  1023 taps over 2.15M samples are 2.2 G FMAs:
-// bound by the VALU's fp32 FMA rate, not by HBM (17 MB in and out).
+// multiply-add per tap: on the fp32 matrix cores (fir_mfma_kernel), and with
+// fewer than 32 taps, where that product would be half padding, on the VALU
+// (fir_kernel: a block of 256 threads computes 2048 consecutive outputs from
+// a window staged in LDS; each thread keeps a 16-sample register window over
+// its 8 outputs and slides it 8 taps at a time, the taps coming from the
+// scalar cache).
 //
 // PCM16: round(clamp(x * gain, -1, 1) * 32767) as int16, written as the
 // little-endian byte stream the reference reads back (two bytes per
@@ -27,8 +26,9 @@ namespace audio {  // named: the kernels keep readable names in profiles
 constexpr int kThreads = 256;
 constexpr int kPerThread = 8;                        // consecutive outputs per thread
 constexpr int kTile = kThreads * kPerThread;         // outputs per block
-constexpr int kMaxTaps = 4096;                       // window: kTile + taps rounded up + slack
-constexpr int kWindow = kTile + kMaxTaps + 16;
+constexpr int kMaxTaps = 4096;
+constexpr int kMfmaMinTaps = 32;                     // from here on the matrix cores
+constexpr int kWindow = kTile + kMfmaMinTaps + 16;   // fir_kernel's: outputs, taps rounded up, slack
 
 __device__ __forceinline__ int16_t to_pcm16(float v, float gain) {
   const float c = fminf(fmaxf(v * gain, -1.0f), 1.0f);
@@ -129,7 +129,6 @@ __global__ void __launch_bounds__(kThreads) fir_kernel(const float* __restrict__
 // taps: 2,029,200 samples 67.4 -> 40.0 us (PCM16 65.1 -> 38.8), 1,060,000
 // 52.7 -> 29.5, 400,000 33.8 -> 14.2, 2400 32.1 -> 10.3; 64 taps over
 // 1,060,000 7.1 either way, over 24,000 5.2 -> 3.8.
-constexpr int kMfmaMinTaps = 32;
 typedef float fir_f4 __attribute__((ext_vector_type(4)));
 
 __host__ __device__ constexpr int fir_units(int taps) { return (taps + 15 + 15) / 16; }  // of four steps

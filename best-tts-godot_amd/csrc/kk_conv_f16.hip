@@ -1,5 +1,6 @@
 // Conv1d and ConvTranspose1d with fp16 or 8-bit weights on the fp16 matrix
-// cores (v_mfma_f32_32x32x16_f16), fp32 results, in one launch.
+// cores (v_mfma_f32_32x32x16_f16), fp32 results, in one launch (8-bit weights
+// over multiples of 128 channels: convq_kernel below, on the bf16 ones).
 //
 // Exact operands.  An fp16 weight is exact in fp16, and so is an 8-bit
 // weight less its zero point (|q - zp| <= 255); the 8-bit weights' scale,

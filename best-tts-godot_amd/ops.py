@@ -256,7 +256,7 @@ def gemm_pack(w, w_zp=None):
 def conv_pack(w, w_zp=None, transposed=False, stride=1):
     """The packed form of a constant Conv (transposed=False, any stride) or
     ConvTranspose (transposed=True, this stride) weight: fp16, or int8/uint8
-    with its int8/uint8 zero point, laid out once for the fp16 matrix cores
+    with its int8/uint8 zero point, laid out once for the 16-bit matrix cores
     (uint8 bytes on the device), for conv1d / conv_transpose1d(packed=...)."""
     w = w.contiguous()
     cin, cout = (w.shape[0], w.shape[1]) if transposed else (w.shape[1], w.shape[0])

@@ -255,7 +255,7 @@ int kk_conv_transpose1d(const kk_tensor* out, const kk_tensor* x,
                         const kk_tensor* w_zp, const kk_tensor* bias,
                         int stride, int dilation, int pad0, int pad1,
                         int group, int output_padding);
-/* Constant Conv / ConvTranspose weights laid out once for the fp16 matrix
+/* Constant Conv / ConvTranspose weights laid out once for the 16-bit matrix
  * cores: the same convolutions as kk_conv1d / kk_conv_transpose1d (the
  * Conv :637-640 and ConvTranspose :646-651 branches over op_conv1d,
  * ref_runtime.py:58-103), whose weights the reference dequantizes on every
