@@ -403,7 +403,7 @@ __global__ void __launch_bounds__(kThreads) convh_kernel(CArgs A) {
 // scaling (bf16 has fp32's exponents).  The reduction runs tap-major (k =
 // t' Cin + ci): no padded taps, and an operand is eight channels at one time.
 //
-// A block owns 64 rows x 64 columns; its four waves take a quarter of the
+// A block owns 64 rows x 32 NI columns; its four waves take a quarter of the
 // channels each and own nothing in common until they add their tiles.  A wave
 // stages the time window its columns read, 32 channels at a time, in its own
 // LDS (time-major, the three parts side by side, 208 bytes a row: the 32
@@ -427,7 +427,7 @@ typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 constexpr int kQPitch = 208;  // bytes a staged row: three parts of 32 channels, 16 to spare
 constexpr int kQExchange = 4 * 3 * 16 * 64 * 4;  // bytes the waves' tiles take
 
-template <int T, int NP>
+template <int T, int NP, int NI>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(T == 7 ? 1 : 2, 2)))
 convq_kernel(CArgs A, int W) {
   extern __shared__ __align__(16) unsigned char convq_lds[];
@@ -437,7 +437,7 @@ convq_kernel(CArgs A, int W) {
   const int ln = lane & 31, g = lane >> 5;
   const uint3 tile = xcd_tile();  // row tiles fastest: a column range's blocks share an XCD
   const int m0 = __builtin_amdgcn_readfirstlane(static_cast<int>(tile.x)) * 64;
-  const int n0 = __builtin_amdgcn_readfirstlane(static_cast<int>(tile.y)) * 64;
+  const int n0 = __builtin_amdgcn_readfirstlane(static_cast<int>(tile.y)) * 32 * NI;
   const int64_t b = __builtin_amdgcn_readfirstlane(static_cast<int>(tile.z));
   const int Cin = A.Cin, L = A.L, C16 = Cin / 16;
   const float* xb = A.x + b * Cin * L;
@@ -496,7 +496,7 @@ convq_kernel(CArgs A, int W) {
             b8, __builtin_amdgcn_raw_buffer_load_b128(
                     wrs, a_lane + static_cast<uint32_t>((mi * A.KS + t * C16 + 2 * c + ks) * 1024), 0, 0));
   };
-  f16v acc[2][2] = {};
+  f16v acc[2][NI] = {};
   auto each_tap = [&](auto f) {
     [&]<int... t>(std::integer_sequence<int, t...>) { (f(std::integral_constant<int, t>{}), ...); }
     (std::make_integer_sequence<int, T>{});
@@ -504,7 +504,7 @@ convq_kernel(CArgs A, int W) {
   // With few taps registers are left to read an operand ahead and to split
   // the next chunk's values among the last products (a SIMD has one or two
   // of these waves: nothing else fills those waits).
-  constexpr bool kDeep = T <= 3 && NP == 5;
+  constexpr bool kDeep = T <= 3 && NP <= 5;
   b8 part[NP][3];
   auto split = [&](int p) {
 #pragma unroll
@@ -516,11 +516,11 @@ convq_kernel(CArgs A, int W) {
       part[p][2][e] = static_cast<__bf16>(x1 - static_cast<float>(part[p][1][e]));
     }
   };
-  b8 x[2][2][3];  // [step % 2][column tile][part]
+  b8 x[2][NI][3];  // [step % 2][column tile][part]
   auto read_x = [&](auto step) {  // step: 2 t + ks of the chunk
     constexpr int t = decltype(step)::value / 2, ks = decltype(step)::value % 2;
 #pragma unroll
-    for (int ni = 0; ni < 2; ++ni)
+    for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
       for (int k = 0; k < 3; ++k)
         x[ks][ni][k] = *reinterpret_cast<const b8*>(
@@ -533,7 +533,7 @@ convq_kernel(CArgs A, int W) {
 #pragma unroll
       for (int mi = 0; mi < 2; ++mi)
 #pragma unroll
-        for (int ni = 0; ni < 2; ++ni)
+        for (int ni = 0; ni < NI; ++ni)
           acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[t][ks][mi], x[ks][ni][k], acc[mi][ni], 0, 0, 0);
   };
   auto each_step = [&](auto f) {
@@ -574,7 +574,7 @@ convq_kernel(CArgs A, int W) {
         for (int p = (i + 1 == 2 * T ? 2 : 0); p < (i + 1 == 2 * T ? NP : 2); ++p) split(p);
         // one matrix instruction, then VALU work in its shadow
 #pragma unroll
-        for (int k = 0; k < 12; ++k) {
+        for (int k = 0; k < 6 * NI; ++k) {
           __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
           __builtin_amdgcn_sched_group_barrier(0x2, i + 1 == 2 * T ? 12 : 8, 0);
         }
@@ -586,36 +586,38 @@ convq_kernel(CArgs A, int W) {
     __builtin_amdgcn_wave_barrier();
   }
   __syncthreads();  // every window is read
-  // wave w keeps tile w = 2 mi + ni; the others' go to LDS ([wave][slot][register][lane])
+  // wave w keeps tile w = NI mi + ni; the others' go to LDS ([slot][register][lane])
+  constexpr int kTiles = 2 * NI;
   float* red = reinterpret_cast<float*>(convq_lds);
+  auto slot = [](int w, int q) { return NI == 2 ? w * 3 + ((q - w - 1) & 3) : w * 2 + q; };
 #pragma unroll
-  for (int q = 0; q < 4; ++q)
+  for (int q = 0; q < kTiles; ++q)
     if (q != wv)
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        red[((wv * 3 + ((q - wv - 1) & 3)) * 16 + r) * 64 + lane] = acc[q >> 1][q & 1][r];
+      for (int r = 0; r < 16; ++r) red[(slot(wv, q) * 16 + r) * 64 + lane] = acc[q / NI][q % NI][r];
   f16v own = acc[0][0];
 #pragma unroll
-  for (int q = 1; q < 4; ++q)
-    if (q == wv) own = acc[q >> 1][q & 1];
+  for (int q = 1; q < kTiles; ++q)
+    if (q == wv) own = acc[q / NI][q % NI];
   __syncthreads();
+  if (wv >= kTiles) return;
   f16v sum;
 #pragma unroll
   for (int w = 0; w < 4; ++w) {
     f16v part = own;
     if (w != wv) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) part[r] = red[((w * 3 + ((wv - w - 1) & 3)) * 16 + r) * 64 + lane];
+      for (int r = 0; r < 16; ++r) part[r] = red[(slot(w, wv) * 16 + r) * 64 + lane];
     }
     sum = w == 0 ? part : sum + part;
   }
-  const int q = n0 + 32 * (wv & 1) + ln;
+  const int q = n0 + 32 * (wv % NI) + ln;
   const auto ors = __builtin_amdgcn_make_buffer_rsrc(A.out + b * A.Cout * A.Lout, 0,
                                                      A.Cout * A.Lout * 4, 0x00020000);
   const int qpos = q < A.Nq ? q * A.os : INT_MIN / 2;
 #pragma unroll
   for (int rg = 0; rg < 16; ++rg) {
-    const int ml = 32 * (wv >> 1) + 8 * (rg / 4) + 4 * g + (rg % 4);
+    const int ml = 32 * (wv / NI) + 8 * (rg / 4) + 4 * g + (rg % 4);
     const int4 rv = rows[ml];
     const int pos = qpos + rv.y;
     const bool ok = rv.x >= 0 && pos >= 0 && pos < A.Lout;
@@ -645,14 +647,14 @@ static bool tap_major(const Geo& g, int w_dt) {
   return w_dt != KK_F16 && g.Cin % 128 == 0 && g.T <= 7;
 }
 
-template <int T, int NP>
+template <int T, int NP, int NI>
 static int launch_q(const CArgs& a, int W, int64_t batch) {
-  const dim3 grid(static_cast<unsigned>(ceil_div(a.M, 64)), static_cast<unsigned>(ceil_div(a.Nq, 64)),
+  const dim3 grid(static_cast<unsigned>(ceil_div(a.M, 64)), static_cast<unsigned>(ceil_div(a.Nq, 32 * NI)),
                   static_cast<unsigned>(batch));
   KK_TRY(check_xcd_grid(grid, "convq_kernel"));
-  const int lds = std::max(4 * W * kQPitch, kQExchange);
-  if (lds > 65536) KK_TRY(allow_large_lds(reinterpret_cast<const void*>(convq_kernel<T, NP>)));
-  KK_LAUNCH((convq_kernel<T, NP>), grid, dim3(kThreads), static_cast<size_t>(lds), ctx().stream, a, W);
+  const int lds = std::max(4 * W * kQPitch, NI == 2 ? kQExchange : kQExchange * 2 / 3);
+  if (lds > 65536) KK_TRY(allow_large_lds(reinterpret_cast<const void*>(convq_kernel<T, NP, NI>)));
+  KK_LAUNCH((convq_kernel<T, NP, NI>), grid, dim3(kThreads), static_cast<size_t>(lds), ctx().stream, a, W);
   return check_launch("convq_kernel");
 }
 
@@ -702,8 +704,21 @@ static int launch_tp(const CArgs& a, const Shape& s, int64_t batch) {
 
 template <int T>
 static int launch_q(const CArgs& a, int W, int64_t batch) {
-  if constexpr (T >= 5) return launch_q<T, 6>(a, W, batch);
-  else return W <= 80 ? launch_q<T, 5>(a, W, batch) : launch_q<T, 8>(a, W, batch);
+  // 32 columns a block where 64 leave half the CUs without one (us, 64 -> 32:
+  // 512 -> 512 k3 over 40 steps, 8 blocks, 14.2 -> 10.1; 128 -> 130 k5 over
+  // 2400, 114 blocks, 10.3 -> 7.8; 256 -> 256 k3 over 2400, 152 blocks, 11.1
+  // either way; ConvTranspose1d 512 -> 256 k20 over 240, 160 blocks, 13.7 ->
+  // 15.2), in windows of up to 16 NP rows
+  const int64_t cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
+  const int W32 = W - 32 * a.qs;
+  const bool narrow = ceil_div(a.M, 64) * ceil_div(a.Nq, 64) * batch * 2 <= cus;
+  if constexpr (T >= 5) {
+    return narrow && W32 <= 64 ? launch_q<T, 4, 1>(a, W32, batch) : launch_q<T, 6, 2>(a, W, batch);
+  } else {
+    if (narrow && W32 <= 48) return launch_q<T, 3, 1>(a, W32, batch);
+    if (narrow && W32 <= 80) return launch_q<T, 5, 1>(a, W32, batch);
+    return W <= 80 ? launch_q<T, 5, 2>(a, W, batch) : launch_q<T, 8, 2>(a, W, batch);
+  }
 }
 
 // tp: the taps a channel spans; 0 for tap-major weights.

@@ -518,6 +518,11 @@ def test_fp16_weight_conv_small_activations(gpu, oracle, sigma, kind):
     (0, 512, 512, 3, 129, 1, 1, 1, np.int8, None), (0, 128, 320, 4, 401, 3, 21, 1, np.int8, None),
     (0, 128, 256, 5, 515, 6, 3, 1, np.int8, None), (0, 128, 200, 6, 450, 5, 1, 1, np.uint8, None),
     (0, 256, 256, 7, 260, 9, 3, 1, np.int8, None), (0, 128, 256, 3, 801, 1, 1, 2, np.int8, None),
+    # enough blocks for 64 columns each
+    (0, 128, 512, 1, 1100, 0, 1, 1, np.int8, None), (0, 128, 512, 2, 1100, 1, 3, 1, np.int8, None),
+    (0, 128, 512, 4, 1100, 3, 21, 1, np.int8, None), (0, 128, 512, 5, 1100, 6, 3, 1, np.uint8, None),
+    (0, 128, 512, 6, 1100, 5, 1, 1, np.int8, None), (0, 128, 512, 7, 1103, 9, 3, 1, np.int8, None),
+    (0, 256, 512, 3, 1100, 1, 1, 1, np.int8, np.inf),
     # windows that are not staged: wide dilations, strides
     (0, 128, 256, 3, 900, 40, 40, 1, np.int8, None), (0, 128, 256, 7, 700, 18, 6, 1, np.uint8, None),
     (0, 128, 300, 3, 1500, 1, 1, 3, np.int8, None), (0, 128, 128, 8, 400, 3, 1, 1, np.int8, None),
