@@ -789,11 +789,30 @@ static int conv_common(const kk_tensor* out, const kk_tensor* x, const kk_tensor
   return KK_OK;
 }
 
+// What gemm_skinny_kernel takes: few columns, a short K, many rows.
+static bool gemm_skinny(const GemmArgs& args, int64_t batch) {
+  return args.N <= kSkinnyN && args.K <= kSkinnyK && args.M * batch >= 4096;
+}
+
+// Into how many ranges K is split: when `blocks` tiles leave CUs idle and the
+// K loop is long (each K-step waits on its loads), with the partials of
+// `batch` items in the context scratch.
+static int64_t gemm_splits(const GemmArgs& args, int64_t blocks, int64_t batch) {
+  const int64_t cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
+  const int64_t nk = ceil_div(args.K, kBK);
+  int64_t S = 1;
+  while (S < 8 && blocks * S < 2 * cus && nk / (2 * S) >= 4 &&
+         static_cast<size_t>(batch * 2 * S * args.M * args.N) * 4 <= kScratchBytes &&
+         batch * 2 * S <= 65535)
+    S *= 2;
+  return S;
+}
+
 // weights_rounded: keep numpy's per-weight rounding of (q - zp) * scale
 // (the fp32 matrix cores); else 8-bit and fp16 weights may take the bf16
 // matrix cores, which scale the exact sum instead.
 static int launch_gemm(const GemmArgs& args, int64_t batch, bool weights_rounded = false) {
-  if (!args.per_item && args.N <= kSkinnyN && args.K <= kSkinnyK && args.M * batch >= 4096) {
+  if (!args.per_item && gemm_skinny(args, batch)) {
     const int64_t rows = args.M * batch;
     const unsigned grid = static_cast<unsigned>(std::min<int64_t>(ceil_div(rows, 256), 1 << 16));
     KK_LAUNCH(gemm_skinny_kernel, dim3(grid), dim3(256), 0, ctx().stream, args, batch);
@@ -811,19 +830,12 @@ static int launch_gemm(const GemmArgs& args, int64_t batch, bool weights_rounded
   const TileSize ts = pick_tile(args.M, args.N, args.per_item ? 1 : batch);
   dim3 grid = grid_of(ts, args.M, args.N, batch);
   KK_TRY(check_grid(grid, batch));
-  // Split K when the tiles leave CUs idle and the K loop is long (each
-  // K-step waits on its loads): partials in the context scratch, summed in
-  // split order by a second kernel.
+  // K's ranges, summed in order by a second kernel (per_item: the caller has
+  // checked that the scratch holds every item's)
   GemmArgs args_s = args;
   {
-    const int64_t cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
     const int64_t blocks = static_cast<int64_t>(grid.x) * grid.y * (args.per_item ? 1 : grid.z);
-    const int64_t nk = ceil_div(args.K, kBK);
-    int64_t S = 1;
-    while (S < 8 && blocks * S < 2 * cus && nk / (2 * S) >= 4 &&
-           static_cast<size_t>(batch * 2 * S * args.M * args.N) * 4 <= kScratchBytes &&
-           batch * 2 * S <= 65535)
-      S *= 2;
+    const int64_t S = gemm_splits(args, blocks, args.per_item ? 1 : batch);
     if (S > 1) {
       args_s.splits = static_cast<int>(S);
       args_s.part = static_cast<float*>(ctx().scratch);
@@ -992,7 +1004,35 @@ int gemm_items(const kk_tensor* out, const kk_tensor* a, const kk_tensor* w, con
   G.per_item = true;
   if (G.M == 0 || G.N == 0 || batch == 0) return KK_OK;
   if (G.K == 0) return kk_fill(out, 0.0);
-  return launch_gemm(G, batch, true);
+  // One launch where that gives each item what it gets alone: not the kernel
+  // of few columns, whose rule counts rows, and not where the scratch holds
+  // one item's K ranges but not all ([1100, 640] x [640, 1024]: two ranges an
+  // item, 9 MB each).
+  const dim3 grid = grid_of(pick_tile(G.M, G.N, 1), G.M, G.N, 1);
+  const int64_t S = gemm_splits(G, static_cast<int64_t>(grid.x) * grid.y, 1);
+  const bool fits = static_cast<size_t>(batch * S * G.M * G.N) * 4 <= kScratchBytes && batch * S <= 65535;
+  if (!gemm_skinny(G, 1) && (S == 1 || fits)) return launch_gemm(G, batch, true);
+  for (int64_t i = 0; i < batch; ++i) {
+    kk_tensor oi{}, wi{}, si = *w_scale, zi{};
+    auto item = [i](kk_tensor* t, const kk_tensor* all) {
+      t->data = static_cast<char*>(all->data) + i * all->strides[0] * dtype_size(all->dtype);
+      t->dtype = all->dtype;
+      t->rank = 2;
+      for (int d = 0; d < 2; ++d) {
+        t->shape[d] = all->shape[d + 1];
+        t->strides[d] = all->strides[d + 1];
+      }
+    };
+    item(&oi, out);
+    item(&wi, w);
+    si.data = static_cast<char*>(si.data) + i * scale_bytes;
+    if (w_zp) {
+      zi = *w_zp;
+      zi.data = static_cast<char*>(zi.data) + i * zp_bytes;
+    }
+    KK_TRY(gemm(&oi, a, &wi, &si, w_zp ? &zi : nullptr, 1.0f, true));
+  }
+  return KK_OK;
 }
 
 }  // namespace kk

@@ -444,10 +444,11 @@ int matmul_shape(const kk_tensor* out, const kk_tensor* a, const kk_tensor* w, B
 int gemm(const kk_tensor* out, const kk_tensor* a, const kk_tensor* w, const kk_tensor* w_scale,
          const kk_tensor* w_zp, float alpha, bool weights_rounded,
          const kk_tensor* packed = nullptr);
-// out[i] = a @ deq(w[i]) in one launch, each item with its own per-tensor scale
-// and zero point (scale_bytes, zp_bytes after the one before; 0: shared), on
-// the fp32 matrix cores with numpy's rounding of each weight.  Tiles and
-// splits are those of one item alone, so the results are too.
+// out[i] = a @ deq(w[i]) (out and w of rank 3, a of rank 2), each item with its
+// own per-tensor scale and zero point (scale_bytes, zp_bytes after the one
+// before; 0: shared), with numpy's rounding of each weight.  Kernel, tiles and
+// splits are those of one item alone, so the results are too; all items go in
+// one launch where that allows it.
 int gemm_items(const kk_tensor* out, const kk_tensor* a, const kk_tensor* w, const kk_tensor* w_scale,
                const kk_tensor* w_zp, int64_t scale_bytes, int64_t zp_bytes);
 // out = A @ dequant(B) on the bf16 matrix cores (kk_gemm_dq.hip) when the

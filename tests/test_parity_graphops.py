@@ -408,6 +408,34 @@ def test_lstm_hidden_sizes(gpu, oracle, H, seq, batch, bias, zp):
         assert_close(g, wv, 1e-4, floor_rel=1e-5, what=f"LSTM {name} H={H}")
 
 
+@pytest.mark.parametrize("seq,inp,H", [(130, 640, 256), (1024, 640, 256), (1025, 640, 256),
+                                       (1984, 512, 256), (1985, 512, 256), (2100, 512, 128), (4096, 24, 1)])
+def test_lstm_directions_as_if_alone(gpu, seq, inp, H):
+    """Each direction of a bidirectional call has the bits of a call of its
+    own (the backward one: on reversed x), whatever the split of its input
+    projection: at seq 1025 .. 1984 the scratch holds one direction's K
+    ranges only, and H = 1 takes the kernel of few columns."""
+    r = rng(43)
+    x = r.normal(0, 1, (seq, 1, inp)).astype(np.float32)
+    w = r.integers(-127, 128, (2, inp, 4 * H)).astype(np.int8)
+    rr = r.integers(-127, 128, (2, H, 4 * H)).astype(np.int8)
+    b = r.normal(0, 0.05, (2, 8 * H)).astype(np.float32)
+    h0, c0 = (r.normal(0, 0.5, (2, 1, H)).astype(np.float32) for _ in range(2))
+    ws, rs = (r.uniform(0.002, 0.006, 2).astype(np.float32) for _ in range(2))
+    wz, rz = np.array([3, -2], np.int8), np.array([0, 1], np.int8)
+
+    def call(ins, direction):
+        return node(gpu, "DynamicQuantizeLSTM", ins, {"hidden_size": H, "direction": direction}, nout=3)
+    both = call([x, w, rr, b, None, h0, c0, None, ws, wz, rs, rz], "bidirectional")
+    for d in range(2):
+        s = slice(d, d + 1)
+        xd = x[::-1].copy() if d else x
+        one = call([xd, w[s], rr[s], b[s], None, h0[s], c0[s], None, ws[s], wz[s], rs[s], rz[s]], "forward")
+        y = one[0][::-1] if d else one[0]
+        for got, want, name in zip((both[0][:, s], both[1][s], both[2][s]), (y, one[1], one[2]), ("Y", "Y_h", "Y_c")):
+            assert_bitexact(got, want, f"LSTM {name} direction {d}, {seq} steps")
+
+
 @pytest.mark.parametrize("batch,slen,n,step,onesided", [(1, 3005, 20, 5, 1), (2, 999, 16, 3, 0),
                                                          (1, 1400003, 20, 5, 1)])
 def test_stft(gpu, oracle, batch, slen, n, step, onesided):
