@@ -397,10 +397,13 @@ __global__ void __launch_bounds__(kThreads) convh_kernel(CArgs A) {
 
 // ------------------------------------- 8-bit weights, channels in 128s
 // The same implicit GEMM on the bf16 matrix cores (v_mfma_f32_32x32x16_bf16):
-// an 8-bit weight less its zero point is exact in bf16, and an activation is
-// split exactly into three bf16 parts by rounding (8 + 8 + 8 significant
-// bits), so three products per weight give exact fp32 products with no
-// scaling (bf16 has fp32's exponents).  The reduction runs tap-major (k =
+// an 8-bit weight less its zero point is exact in bf16, and an activation
+// times 2^24 is split exactly into three bf16 parts by rounding (8 + 8 + 8
+// significant bits), so three products per weight give exact fp32 products.
+// The factor keeps the lower parts of the smallest floats out of bf16's
+// subnormals (unscaled, activations below 2^-110 lost bits, and all but eight
+// at 1e-38); the sums leave it in the epilogue.  It costs a multiplication a
+// staged value (512 -> 512 k3 over 2400 steps 22.7 -> 23.0 us).  The reduction runs tap-major (k =
 // t' Cin + ci): no padded taps, and an operand is eight channels at one time.
 //
 // A block owns 64 rows x 32 NI columns; its four waves take a quarter of the
@@ -414,8 +417,9 @@ __global__ void __launch_bounds__(kThreads) convh_kernel(CArgs A) {
 // weight fragments are in flight in registers.  Then each wave keeps one
 // 32 x 32 tile of the 64 x 64 and adds the other waves' in wave order.
 //
-// An output that is not finite (an infinity or NaN in reach, or a sample
-// above bf16's range) is summed again with scalar fp32 products.
+// An output that is not finite (an infinity or NaN in reach, a sample above
+// 2^104 or a sum that 2^24 takes beyond fp32's range) is summed again with
+// scalar fp32 products.
 //
 // Bound by each wave's chain (a chunk: window, products) at one or two waves
 // a SIMD.  us, the kernel above -> this one: Conv1d 512 -> 512 k3 over 2400
@@ -509,7 +513,7 @@ convq_kernel(CArgs A, int W) {
   auto split = [&](int p) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const float x0 = v[p][e];
+      const float x0 = v[p][e] * 0x1p24f;
       part[p][0][e] = static_cast<__bf16>(x0);
       const float x1 = x0 - static_cast<float>(part[p][0][e]);
       part[p][1][e] = static_cast<__bf16>(x1);
@@ -621,7 +625,7 @@ convq_kernel(CArgs A, int W) {
     const int4 rv = rows[ml];
     const int pos = qpos + rv.y;
     const bool ok = rv.x >= 0 && pos >= 0 && pos < A.Lout;
-    float s = sum[rg];
+    float s = sum[rg] * 0x1p-24f;
     if (ok && !(fabsf(s) < INFINITY)) {
       const __bf16* wh = reinterpret_cast<const __bf16*>(A.wp);
       s = 0.0f;

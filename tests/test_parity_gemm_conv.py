@@ -571,6 +571,28 @@ def test_8bit_conv_of_128_channel_rounds(gpu, oracle, tr, cin, cout, k, L, pad, 
         check(np.where(fin, got, 0), np.where(fin, want, 0), f"conv {cin}->{cout} k{k} packed={packed is not None}")
 
 
+@pytest.mark.parametrize("sigma", [1e-30, 1e-34, 1e-36, 1e-38, 1e30])
+@pytest.mark.parametrize("tr", [0, 1])
+def test_8bit_conv_of_128_channel_rounds_keeps_every_float(gpu, sigma, tr):
+    """Activations down to fp32's subnormals, and far above audio's, at the
+    error of unit-scale ones: exact products summed in fp32, K = 384 (at most
+    sqrt(K) 2^-24 = 1.2e-6 of the result's norm), against 64 bits."""
+    r = rng(48)
+    x = (r.normal(0, 1, (2, 128, 700)) * sigma).astype(np.float32)
+    w = r.integers(-127, 128, (128, 128, 3)).astype(np.int8)
+    if tr:  # stride 1: the convolution with the taps turned round and the channels swapped
+        got = gpu.ops.conv_transpose1d(gpu.to_device(x), gpu.to_device(w), None, (1, 1), 1,
+                                       w_scale=gpu.to_device(np.array(np.float32(1)))).numpy()
+        w = w.transpose(1, 0, 2)[:, :, ::-1]
+    else:
+        got = gpu.ops.conv1d(gpu.to_device(x), gpu.to_device(w), None, (1, 1),
+                             w_scale=gpu.to_device(np.array(np.float32(1)))).numpy()
+    xp = np.pad(x.astype(np.float64) / sigma, ((0, 0), (0, 0), (1, 1)))
+    want = sum(w[None, :, :, t].astype(np.float64) @ xp[:, :, t:t + 700] for t in range(3))
+    err = np.linalg.norm(got.astype(np.float64) / sigma - want) / np.linalg.norm(want)
+    assert err < 1.2e-6, f"sigma {sigma}: relative error {err:.2e}"
+
+
 def decoder_stage(r):
     """The decoder upsample stage's operands (the fixed draws of the stage
     tests and of the bench): int8 ConvTranspose1d(512->256, k20, s10, p5)
