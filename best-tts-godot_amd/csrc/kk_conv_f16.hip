@@ -160,8 +160,25 @@ __device__ __forceinline__ int scale_exp(unsigned mbits) {
   return min(120, 10 - e);
 }
 
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+constexpr float kSplitScale = 0x1p24f;
+
+// Eight activations times kSplitScale as three bf16 parts each.
+__device__ __forceinline__ void split3(const float (&v)[8], b8 (&part)[3]) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float x0 = v[e] * kSplitScale;
+    part[0][e] = static_cast<__bf16>(x0);
+    const float x1 = x0 - static_cast<float>(part[0][e]);
+    part[1][e] = static_cast<__bf16>(x1);
+    part[2][e] = static_cast<__bf16>(x1 - static_cast<float>(part[1][e]));
+  }
+}
+
 // TP = 0: weights laid out for convq_kernel (tap-major bf16), for the strides
-// and dilations whose window that kernel does not hold.
+// and dilations whose window that kernel does not hold: its three products a
+// weight, no scale (as fp16 operands, each weight fragment converted for two
+// products, 512 -> 512 k4 over 2400 steps took 45 us; so 38; the fp16 layout 34).
 template <int TP, int MI, int WK, int R>
 __global__ void __launch_bounds__(kThreads) convh_kernel(CArgs A) {
   constexpr int NPO = TP ? TP : 1;
@@ -261,6 +278,16 @@ __global__ void __launch_bounds__(kThreads) convh_kernel(CArgs A) {
   int kcur = 0, have = 0, bad = 0;
   // one slice: the column's running scale, the split, the products
   auto mma = [&](float (&v)[8], const uint4 (&f)[MI]) {
+    if constexpr (TP == 0) {  // bf16: three exact parts, as convq_kernel forms them, and no scale
+      b8 part[3];
+      split3(v, part);
+#pragma unroll
+      for (int k = 2; k >= 0; --k)
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi)
+          acc[mi] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(b8, f[mi]), part[k], acc[mi], 0, 0, 0);
+      return;
+    }
     unsigned mx = 0;
 #pragma unroll
     for (int e = 0; e < 8; ++e) mx = max(mx, __float_as_uint(v[e]) & 0x7fffffffu);
@@ -293,15 +320,7 @@ __global__ void __launch_bounds__(kThreads) convh_kernel(CArgs A) {
     }
 #pragma unroll
     for (int mi = 0; mi < MI; ++mi) {
-      h8 a = __builtin_bit_cast(h8, f[mi]);
-      if constexpr (TP == 0) {  // bf16 -> fp16, exact for these integers
-        const uint32_t w[4] = {f[mi].x, f[mi].y, f[mi].z, f[mi].w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          a[2 * e] = static_cast<_Float16>(__uint_as_float(w[e] << 16));
-          a[2 * e + 1] = static_cast<_Float16>(__uint_as_float(w[e] & 0xffff0000u));
-        }
-      }
+      const h8 a = __builtin_bit_cast(h8, f[mi]);
       acc[mi] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, hi, acc[mi], 0, 0, 0);
       acc[mi] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, lo, acc[mi], 0, 0, 0);
     }
@@ -317,7 +336,7 @@ __global__ void __launch_bounds__(kThreads) convh_kernel(CArgs A) {
       fetch(s0 + i + u + R, bv[u], av[u]);
     }
   }
-  const float uns = ldexpf(1.0f, -kcur);  // exact: a power of two
+  const float uns = TP ? ldexpf(1.0f, -kcur) : 1.0f / kSplitScale;  // exact: a power of two
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -344,6 +363,12 @@ __global__ void __launch_bounds__(kThreads) convh_kernel(CArgs A) {
         for (int r = 0; r < 16; ++r) acc[i][r] += src[(i * 16 + r) * 64];
       bad |= red_bad[(k * WN + wn) * 64 + lane];
     }
+  }
+  if constexpr (TP == 0) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) bad |= !(fabsf(acc[i][r]) < INFINITY);
   }
   // D(i, j) of a 32x32 tile: lane j + 32 ((i / 4) % 2), register (i / 8) 4 + i % 4.
   // Stores through a buffer resource over this item's output: an offset
@@ -427,12 +452,11 @@ __global__ void __launch_bounds__(kThreads) convh_kernel(CArgs A) {
 // over 2400 15.8 -> 11.2; 512 -> 512 k7 over 7000 135 -> 99; ConvTranspose1d
 // 512 -> 256 k20 s10 over 240 16.5 -> 13.7, over 700 28.9 -> 22.1.  No further
 // from 64 bits (2.0e-7 -> 1.9e-7 relative for the first).
-typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 constexpr int kQPitch = 208;  // bytes a staged row: three parts of 32 channels, 16 to spare
 constexpr int kQExchange = 4 * 3 * 16 * 64 * 4;  // bytes the waves' tiles take
 
 template <int T, int NP, int NI>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(T == 7 ? 1 : 2, 2)))
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(T == 7 && NI == 2 ? 1 : 2, 2)))
 convq_kernel(CArgs A, int W) {
   extern __shared__ __align__(16) unsigned char convq_lds[];
   __shared__ int4 rows[64];  // output row offset, phase offset, scale, bias
@@ -510,16 +534,7 @@ convq_kernel(CArgs A, int W) {
   // of these waves: nothing else fills those waits).
   constexpr bool kDeep = T <= 3 && NP <= 5;
   b8 part[NP][3];
-  auto split = [&](int p) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float x0 = v[p][e] * 0x1p24f;
-      part[p][0][e] = static_cast<__bf16>(x0);
-      const float x1 = x0 - static_cast<float>(part[p][0][e]);
-      part[p][1][e] = static_cast<__bf16>(x1);
-      part[p][2][e] = static_cast<__bf16>(x1 - static_cast<float>(part[p][1][e]));
-    }
-  };
+  auto split = [&](int p) { split3(v[p], part[p]); };
   b8 x[2][NI][3];  // [step % 2][column tile][part]
   auto read_x = [&](auto step) {  // step: 2 t + ks of the chunk
     constexpr int t = decltype(step)::value / 2, ks = decltype(step)::value % 2;
@@ -625,7 +640,7 @@ convq_kernel(CArgs A, int W) {
     const int4 rv = rows[ml];
     const int pos = qpos + rv.y;
     const bool ok = rv.x >= 0 && pos >= 0 && pos < A.Lout;
-    float s = sum[rg] * 0x1p-24f;
+    float s = sum[rg] * (1.0f / kSplitScale);
     if (ok && !(fabsf(s) < INFINITY)) {
       const __bf16* wh = reinterpret_cast<const __bf16*>(A.wp);
       s = 0.0f;
@@ -645,10 +660,16 @@ convq_kernel(CArgs A, int W) {
   }
 }
 
-// Whether 8-bit weights of this geometry are laid out for, and run on,
-// convq_kernel: whole 128-channel rounds for its four waves.
+// Whether 8-bit weights of this geometry are laid out for convq_kernel: whole
+// 128-channel rounds for its four waves, and not two taps of 128 channels, of
+// which the fp16 layout pads none and a wave has one chunk, with nothing to
+// overlap (128 -> 128 k2 over 9000 steps 11.0 us there, 11.7 here; over 17,000
+// 14.3 and 17.0).  From 256 channels two taps gain more often than they lose
+// (256 -> 128 stride 6 over 2400 steps 19.5 and 15.6, over 1600 13.8 and 15.0;
+// 256 -> 256 over 5000 14.4 and 14.6, over 17,000 35.1 and 31.1; 512 -> 256
+// stride 8 over 1000 30.3 and 23.6, over 8000 144 and 156).
 static bool tap_major(const Geo& g, int w_dt) {
-  return w_dt != KK_F16 && g.Cin % 128 == 0 && g.T <= 7;
+  return w_dt != KK_F16 && g.Cin % 128 == 0 && g.T <= 7 && !(g.T == 2 && g.Cin < 256);
 }
 
 template <int T, int NP, int NI>
@@ -706,43 +727,66 @@ static int launch_tp(const CArgs& a, const Shape& s, int64_t batch) {
 #undef KK_CONVH_WK
 }
 
+// Runs convq_kernel if a block's window fits; the rule is of one to seven taps
+// T, the window W of 64 columns (W32 of 32) and the blocks of 64.  Measured
+// over 128 to 1024 channels, 300 to 17,000 steps, strides 1 to 4 and dilations
+// 1 to 70 against the fp16 layout (1.0 = that kernel's time):
+//  - 32 columns a block where 64 leave half the CUs without one (512 -> 512 k3
+//    over 40 steps, 8 blocks: 14.2 us with 64, 10.1 with 32; 256 -> 256 k3 over
+//    2400, 152 blocks: 11.1 either way), where 64 need more than 96 staged
+//    rows, which cost more than the columns save (512 -> 512 k5 stride 2 0.44 -
+//    0.54, k7 dilation 9 0.63 - 0.73; through convh_kernel<0> 0.67 - 1.03), and
+//    with seven taps, whose fragments leave a SIMD one wave of 64 columns, from
+//    a block a CU on (256 -> 256 over 5000 steps, 316 blocks, 0.69 against
+//    0.86; over 2400, 152 blocks, 0.71 against 0.66).
+//  - one tap: a window is read once, so staging pays only for few blocks (512
+//    -> 512 over 9000 steps 0.67 staged, 0.65 not; 128 channels 0.90 and 0.85).
+//  - wider windows: convh_kernel<0> (0.67 - 1.06; 0.98 - 1.15 with two and four
+//    taps, of which the fp16 layout pads none).
 template <int T>
-static int launch_q(const CArgs& a, int W, int64_t batch) {
-  // 32 columns a block where 64 leave half the CUs without one (us, 64 -> 32:
-  // 512 -> 512 k3 over 40 steps, 8 blocks, 14.2 -> 10.1; 128 -> 130 k5 over
-  // 2400, 114 blocks, 10.3 -> 7.8; 256 -> 256 k3 over 2400, 152 blocks, 11.1
-  // either way; ConvTranspose1d 512 -> 256 k20 over 240, 160 blocks, 13.7 ->
-  // 15.2), in windows of up to 16 NP rows
+static bool launch_q(const CArgs& a, int64_t W, int64_t batch, int* rc) {
   const int64_t cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
-  const int W32 = W - 32 * a.qs;
-  const bool narrow = ceil_div(a.M, 64) * ceil_div(a.Nq, 64) * batch * 2 <= cus;
-  if constexpr (T >= 5) {
-    return narrow && W32 <= 64 ? launch_q<T, 4, 1>(a, W32, batch) : launch_q<T, 6, 2>(a, W, batch);
+  const int64_t W32 = W - int64_t{32} * a.qs;
+  const int64_t blocks = ceil_div(a.M, 64) * ceil_div(a.Nq, 64) * batch;
+  const bool narrow = blocks * 2 <= cus;
+  if (W32 > 128) return false;
+  const int w = static_cast<int>(std::min<int64_t>(W, 128)), w32 = static_cast<int>(W32);
+  if constexpr (T == 1) {
+    if (!narrow || W32 > 48) return false;
+    *rc = launch_q<T, 3, 1>(a, w32, batch);
+  } else if constexpr (T <= 4) {
+    if (narrow && W32 <= 48) *rc = launch_q<T, 3, 1>(a, w32, batch);
+    else if (narrow && W32 <= 80) *rc = launch_q<T, 5, 1>(a, w32, batch);
+    else if (W <= 80) *rc = launch_q<T, 5, 2>(a, w, batch);
+    else if (W <= 96) *rc = launch_q<T, 6, 2>(a, w, batch);
+    else if (W32 <= 80) *rc = launch_q<T, 5, 1>(a, w32, batch);
+    else if (T == 4) *rc = launch_q<4, 8, 1>(a, w32, batch);
+    else return false;
   } else {
-    if (narrow && W32 <= 48) return launch_q<T, 3, 1>(a, W32, batch);
-    if (narrow && W32 <= 80) return launch_q<T, 5, 1>(a, W32, batch);
-    return W <= 80 ? launch_q<T, 5, 2>(a, W, batch) : launch_q<T, 8, 2>(a, W, batch);
+    if (!narrow && (T < 7 || blocks <= cus) && W <= 96) *rc = launch_q<T, 6, 2>(a, w, batch);
+    else if (W32 <= 64) *rc = launch_q<T, 4, 1>(a, w32, batch);
+    else if (W32 <= 96) *rc = launch_q<T, 6, 1>(a, w32, batch);
+    else return false;
   }
+  return true;
 }
 
 // tp: the taps a channel spans; 0 for tap-major weights.
 static int launch(const CArgs& a, int tp, int64_t batch) {
   if (tp == 0) {
-    // the window of 64 columns, up to 16 NP staged rows (five and more taps'
-    // fragments leave registers for 96)
     const int64_t W = int64_t{63} * a.qs + static_cast<int64_t>(a.T - 1) * a.tm + 1;
-    if (W <= (a.T >= 5 ? 96 : 128)) {
-      switch (a.T) {
-        case 1: return launch_q<1>(a, static_cast<int>(W), batch);
-        case 2: return launch_q<2>(a, static_cast<int>(W), batch);
-        case 3: return launch_q<3>(a, static_cast<int>(W), batch);
-        case 4: return launch_q<4>(a, static_cast<int>(W), batch);
-        case 5: return launch_q<5>(a, static_cast<int>(W), batch);
-        case 6: return launch_q<6>(a, static_cast<int>(W), batch);
-        default: return launch_q<7>(a, static_cast<int>(W), batch);
-      }
+    int rc = KK_OK;
+    bool ran = false;
+    switch (a.T) {
+      case 1: ran = launch_q<1>(a, W, batch, &rc); break;
+      case 2: ran = launch_q<2>(a, W, batch, &rc); break;
+      case 3: ran = launch_q<3>(a, W, batch, &rc); break;
+      case 4: ran = launch_q<4>(a, W, batch, &rc); break;
+      case 5: ran = launch_q<5>(a, W, batch, &rc); break;
+      case 6: ran = launch_q<6>(a, W, batch, &rc); break;
+      default: ran = launch_q<7>(a, W, batch, &rc); break;
     }
-    return launch_tp<0>(a, pick_shape(a, batch), batch);
+    return ran ? rc : launch_tp<0>(a, pick_shape(a, batch), batch);
   }
   const Shape s = pick_shape(a, batch);
   if (tp == 2) return launch_tp<2>(a, s, batch);

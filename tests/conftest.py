@@ -1,6 +1,8 @@
+import ctypes
 import importlib
 import os
 import sys
+import time
 
 import numpy as np
 import pytest
@@ -44,6 +46,26 @@ def gpu(kk):
 
 def rng(seed=0):
     return np.random.default_rng(seed)
+
+
+def graph_us(kk, fn, inner=8):
+    """The least time of one call of `fn`, in microseconds, among recorded
+    calls replayed."""
+    fn()
+    kk.sync()
+    kk._lib.call("kk_graph_begin")
+    for _ in range(inner):
+        fn()
+    g = ctypes.c_int(-1)
+    kk._lib.call("kk_graph_end", ctypes.byref(g))
+    best = float("inf")
+    for _ in range(10):
+        t = time.perf_counter()
+        kk._lib.call("kk_graph_launch", g.value)
+        kk.sync()
+        best = min(best, (time.perf_counter() - t) / inner * 1e6)
+    kk._lib.call("kk_graph_destroy", g.value)
+    return best
 
 
 def assert_close(got, want, rtol, atol=0.0, floor_rel=0.0, what=""):

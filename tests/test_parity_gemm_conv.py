@@ -11,7 +11,7 @@ max|ref| stays below 1e-4."""
 import numpy as np
 import pytest
 
-from conftest import assert_bitexact, assert_close, rng
+from conftest import graph_us, assert_bitexact, assert_close, rng
 
 pytestmark = pytest.mark.gpu
 RTOL, FLOOR = 1e-4, 1e-5
@@ -591,6 +591,57 @@ def test_8bit_conv_of_128_channel_rounds_keeps_every_float(gpu, sigma, tr):
     want = sum(w[None, :, :, t].astype(np.float64) @ xp[:, :, t:t + 700] for t in range(3))
     err = np.linalg.norm(got.astype(np.float64) / sigma - want) / np.linalg.norm(want)
     assert err < 1.2e-6, f"sigma {sigma}: relative error {err:.2e}"
+
+
+# (taps, dilation, stride): each way a block's window can fit, at its limits
+WINDOWS = [(1, 1, 1), (1, 1, 2), (2, 16, 1), (2, 17, 1), (2, 32, 1), (2, 33, 1), (2, 48, 1), (2, 49, 1),
+           (3, 8, 1), (3, 9, 1), (3, 16, 1), (3, 17, 1), (3, 24, 1), (3, 25, 1), (3, 1, 2), (3, 1, 3),
+           (4, 5, 1), (4, 11, 1), (4, 16, 1), (4, 17, 1), (4, 32, 1), (4, 33, 1), (4, 1, 4),
+           (5, 8, 1), (5, 9, 1), (5, 16, 1), (5, 17, 1), (6, 6, 1), (6, 7, 1), (6, 12, 1), (6, 13, 1),
+           (7, 5, 1), (7, 6, 1), (7, 10, 1), (7, 11, 1), (7, 1, 2), (7, 1, 4)]
+
+
+@pytest.mark.parametrize("k,dil,stride", WINDOWS)
+def test_8bit_conv_of_128_channel_rounds_windows(gpu, k, dil, stride):
+    """Every window rule at its limits, for few blocks and for many, two batch
+    items, against 64 bits: exact products summed in fp32 (sqrt(K) 2^-24 of
+    the result's norm, K = 256 k)."""
+    r = rng(49)
+    dv = gpu.to_device
+    for cout, L in ((96, 301), (512, 1130 * stride)):
+        x = r.normal(0, 1, (2, 256, L)).astype(np.float32)
+        w = r.integers(0, 256, (cout, 256, k)).astype(np.uint8)
+        sc, z, pad = np.float32(2.0 ** -8), np.uint8(117), dil * (k - 1) // 2 + 1
+        xp = np.pad(x.astype(np.float64), ((0, 0), (0, 0), (pad, pad)))
+        lo = (L + 2 * pad - dil * (k - 1) - 1) // stride + 1
+        wd = (w.astype(np.float64) - 117) * 2.0 ** -8
+        want = sum(np.matmul(wd[:, :, t], xp[:, :, t * dil:t * dil + stride * (lo - 1) + 1:stride]) for t in range(k))
+        dw, kw = dv(w), dict(w_scale=dv(np.array(sc)), w_zp=dv(np.array(z)))
+        for packed in (None, gpu.ops.conv_pack(dw, kw["w_zp"], False, stride)):
+            got = gpu.ops.conv1d(dv(x), dw, None, (pad, pad), stride, dil, packed=packed, **kw).numpy()
+            for n in range(2):
+                err = np.linalg.norm(got[n] - want[n]) / np.linalg.norm(want[n])
+                assert err < np.sqrt(256 * k) * 2.0 ** -24, f"cout {cout} item {n}: relative error {err:.2e}"
+
+
+@pytest.mark.parametrize("cin,cout,k,dil,L", [(1024, 256, 7, 9, 9000), (512, 512, 2, 70, 2400), (512, 512, 4, 33, 2400)])
+def test_8bit_conv_of_wide_windows_time(gpu, cin, cout, k, dil, L):
+    """Windows past what a block of 64 columns stages take no longer than the
+    same convolution on fp16 weights (0.7 to 1.15 of it measured; 1.25 leaves
+    room for the clock's noise)."""
+    r = rng(50)
+    dv, pad = gpu.to_device, dil * (k - 1) // 2
+    x = dv(r.normal(0, 1, (1, cin, L)).astype(np.float32))
+    w8 = r.integers(-127, 128, (cout, cin, k)).astype(np.int8)
+    sc = dv(np.array(np.float32(2.0 ** -8)))
+    out = gpu.DeviceTensor.empty((1, cout, L + 2 * pad - dil * (k - 1)), np.float32)
+    us = []
+    for w, scale in ((dv(w8), sc), (dv(w8.astype(np.float16)), None)):
+        pk = gpu.ops.conv_pack(w, None, False, 1)
+        us.append(graph_us(gpu, lambda: gpu._lib.call(
+            "kk_conv1d_packed", out.desc(), x.desc(), w.desc(), pk.desc(), scale.desc() if scale else None,
+            None, None, 1, dil, pad, pad)))
+    assert us[0] <= 1.25 * us[1], f"{us[0]:.1f} us on 8-bit weights, {us[1]:.1f} on fp16"
 
 
 def decoder_stage(r):
