@@ -453,13 +453,14 @@ __global__ void __launch_bounds__(kThreads) convh_kernel(CArgs A) {
 // 512 -> 256 k20 s10 over 240 16.5 -> 13.7, over 700 28.9 -> 22.1.  No further
 // from 64 bits (2.0e-7 -> 1.9e-7 relative for the first).
 constexpr int kQPitch = 208;  // bytes a staged row: three parts of 32 channels, 16 to spare
+constexpr int kQRows = 64 * 16;  // bytes of the 64 rows' constants (static LDS)
 constexpr int kQExchange = 4 * 3 * 16 * 64 * 4;  // bytes the waves' tiles take
 
 template <int T, int NP, int NI>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(T == 7 && NI == 2 ? 1 : 2, 2)))
 convq_kernel(CArgs A, int W) {
   extern __shared__ __align__(16) unsigned char convq_lds[];
-  __shared__ int4 rows[64];  // output row offset, phase offset, scale, bias
+  __shared__ int4 rows[kQRows / sizeof(int4)];  // output row offset, phase offset, scale, bias
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ln = lane & 31, g = lane >> 5;
@@ -666,7 +667,7 @@ convq_kernel(CArgs A, int W) {
 // overlap (128 -> 128 k2 over 9000 steps 11.0 us there, 11.7 here; over 17,000
 // 14.3 and 17.0).  From 256 channels two taps gain more often than they lose
 // (256 -> 128 stride 6 over 2400 steps 19.5 and 15.6, over 1600 13.8 and 15.0;
-// 256 -> 256 over 5000 14.4 and 14.6, over 17,000 35.1 and 31.1; 512 -> 256
+// 256 -> 256 over 5000 13.9 and 14.8, over 17,000 35.1 and 31.1; 512 -> 256
 // stride 8 over 1000 30.3 and 23.6, over 8000 144 and 156).
 static bool tap_major(const Geo& g, int w_dt) {
   return w_dt != KK_F16 && g.Cin % 128 == 0 && g.T <= 7 && !(g.T == 2 && g.Cin < 256);
@@ -678,7 +679,7 @@ static int launch_q(const CArgs& a, int W, int64_t batch) {
                   static_cast<unsigned>(batch));
   KK_TRY(check_xcd_grid(grid, "convq_kernel"));
   const int lds = std::max(4 * W * kQPitch, NI == 2 ? kQExchange : kQExchange * 2 / 3);
-  if (lds > 65536) KK_TRY(allow_large_lds(reinterpret_cast<const void*>(convq_kernel<T, NP, NI>)));
+  if (lds + kQRows > 65536) KK_TRY(allow_large_lds(reinterpret_cast<const void*>(convq_kernel<T, NP, NI>)));
   KK_LAUNCH((convq_kernel<T, NP, NI>), grid, dim3(kThreads), static_cast<size_t>(lds), ctx().stream, a, W);
   return check_launch("convq_kernel");
 }
@@ -734,11 +735,11 @@ static int launch_tp(const CArgs& a, const Shape& s, int64_t batch) {
 //  - 32 columns a block where 64 leave half the CUs without one (512 -> 512 k3
 //    over 40 steps, 8 blocks: 14.2 us with 64, 10.1 with 32; 256 -> 256 k3 over
 //    2400, 152 blocks: 11.1 either way), where 64 need more than 96 staged
-//    rows, which cost more than the columns save (512 -> 512 k5 stride 2 0.44 -
-//    0.54, k7 dilation 9 0.63 - 0.73; through convh_kernel<0> 0.67 - 1.03), and
+//    rows, which cost more than the columns save (512 -> 512 k5 stride 2 0.46 -
+//    0.55, k7 dilation 9 0.63 - 0.73; through convh_kernel<0> 0.67 - 1.03), and
 //    with seven taps, whose fragments leave a SIMD one wave of 64 columns, from
-//    a block a CU on (256 -> 256 over 5000 steps, 316 blocks, 0.69 against
-//    0.86; over 2400, 152 blocks, 0.71 against 0.66).
+//    a block a CU on (256 -> 256 over 5000 steps, 316 blocks, 0.73 against
+//    0.89; over 2400, 152 blocks, 0.71 against 0.65).
 //  - one tap: a window is read once, so staging pays only for few blocks (512
 //    -> 512 over 9000 steps 0.67 staged, 0.65 not; 128 channels 0.90 and 0.85).
 //  - wider windows: convh_kernel<0> (0.67 - 1.06; 0.98 - 1.15 with two and four

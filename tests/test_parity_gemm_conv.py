@@ -595,6 +595,7 @@ def test_8bit_conv_of_128_channel_rounds_keeps_every_float(gpu, sigma, tr):
 
 # (taps, dilation, stride): each way a block's window can fit, at its limits
 WINDOWS = [(1, 1, 1), (1, 1, 2), (2, 16, 1), (2, 17, 1), (2, 32, 1), (2, 33, 1), (2, 48, 1), (2, 49, 1),
+           (2, 14, 1), (2, 46, 1), (3, 7, 1), (3, 23, 1),  # 78 rows: past 64 KB of LDS with the row constants
            (3, 8, 1), (3, 9, 1), (3, 16, 1), (3, 17, 1), (3, 24, 1), (3, 25, 1), (3, 1, 2), (3, 1, 3),
            (4, 5, 1), (4, 11, 1), (4, 16, 1), (4, 17, 1), (4, 32, 1), (4, 33, 1), (4, 1, 4),
            (5, 8, 1), (5, 9, 1), (5, 16, 1), (5, 17, 1), (6, 6, 1), (6, 7, 1), (6, 12, 1), (6, 13, 1),
