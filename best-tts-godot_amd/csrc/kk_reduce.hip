@@ -1844,7 +1844,7 @@ struct RedArgs {
   int64_t nout, nred;
 };
 
-constexpr int kRedBatch = 48;
+template <bool ONE>  // one reduced axis, or any number
 __global__ void __launch_bounds__(256) reduce_generic_kernel(float* __restrict__ out, const float* __restrict__ x,
                                       RedArgs R, int op) {
   for (int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; t < R.nout;
@@ -1857,68 +1857,40 @@ __global__ void __launch_bounds__(256) reduce_generic_kernel(float* __restrict__
     float s = 0.0f;  // numpy sums a non-contiguous axis in order, in fp32
     float m = -INFINITY;
     bool nan = false;
-    if (R.rr == 1) {
-      // One reduced axis: its terms are added (or compared) in order, one
-      // thread an output, so the time is that of the loads' round trips:
-      // kRedBatch loads are in flight while the batch before is added (16 at
-      // a time, each waited for, before: [1,3380,512] over its middle axis 60
-      // -> 48 us, 512 rows of 3380 of a view 364 -> 37).
-      const int64_t st = R.rst[0], last = R.nred - 1;
-      float v[kRedBatch], w[kRedBatch];
-      auto load = [&](int64_t j, float (&d)[kRedBatch]) {  // (past the end: the last term again)
-        if (j + kRedBatch <= R.nred) {
-          const float* p = x + base + j * st;
-          if (st == 1) {  // a row of a view: a line a lane, 16 bytes of it at a time
+    if (ONE) {
+      // One reduced axis: sixteen independent loads in flight, then added
+      // (or compared) in order.
+      const int64_t st = R.rst[0];
+      int64_t j = 0;
+      for (; j + 16 <= R.nred; j += 16) {
+        float v[16];
 #pragma unroll
-            for (int u = 0; u < kRedBatch; u += 4) {
-              const kk_f4u q = *reinterpret_cast<const kk_f4u*>(p + u);
+        for (int u = 0; u < 16; ++u) v[u] = x[base + (j + u) * st];
 #pragma unroll
-              for (int e = 0; e < 4; ++e) d[u + e] = q[e];
-            }
-          } else {
-#pragma unroll
-            for (int u = 0; u < kRedBatch; ++u, p += st) d[u] = *p;
-          }
-        } else {
-#pragma unroll
-          for (int u = 0; u < kRedBatch; ++u) d[u] = x[base + min(j + u, last) * st];
+        for (int u = 0; u < 16; ++u) {
+          s += v[u];
+          nan |= __builtin_isnan(v[u]);
+          m = fmaxf(m, v[u]);
         }
-      };
-      auto add = [&](int64_t j, const float (&d)[kRedBatch]) {
-        const int n = static_cast<int>(R.nred - j < kRedBatch ? R.nred - j : kRedBatch);
-        if (op == KK_REDUCE_MAX) {
-#pragma unroll
-          for (int u = 0; u < kRedBatch; ++u) {  // (a repeated term changes nothing)
-            nan |= __builtin_isnan(d[u]);
-            m = fmaxf(m, d[u]);
-          }
-        } else if (n == kRedBatch) {
-#pragma unroll
-          for (int u = 0; u < kRedBatch; ++u) s += d[u];
-        } else {
-#pragma unroll
-          for (int u = 0; u < kRedBatch; ++u)
-            if (u < n) s += d[u];
+      }
+      for (; j < R.nred; ++j) {
+        const float v = x[base + j * st];
+        s += v;
+        nan |= __builtin_isnan(v);
+        m = fmaxf(m, v);
+      }
+    } else {
+      for (int64_t j = 0; j < R.nred; ++j) {
+        int64_t rj = j, off = base;
+        for (int d = R.rr - 1; d >= 0; --d) {
+          off += (rj % R.rdims[d]) * R.rst[d];
+          rj /= R.rdims[d];
         }
-      };
-      if (R.nred > 0) load(0, v);
-      for (int64_t j = 0; j < R.nred; j += 2 * kRedBatch) {
-        load(j + kRedBatch, w);
-        add(j, v);
-        load(j + 2 * kRedBatch, v);
-        if (j + kRedBatch < R.nred) add(j + kRedBatch, w);
+        const float v = x[off];
+        s += v;
+        nan |= __builtin_isnan(v);
+        m = fmaxf(m, v);
       }
-    }
-    for (int64_t j = 0; j < R.nred && R.rr != 1; ++j) {
-      int64_t rj = j, off = base;
-      for (int d = R.rr - 1; d >= 0; --d) {
-        off += (rj % R.rdims[d]) * R.rst[d];
-        rj /= R.rdims[d];
-      }
-      const float v = x[off];
-      s += v;
-      nan |= __builtin_isnan(v);
-      m = fmaxf(m, v);
     }
     float v;
     if (op == KK_REDUCE_MAX) v = nan ? NAN : m;
@@ -1926,6 +1898,98 @@ __global__ void __launch_bounds__(256) reduce_generic_kernel(float* __restrict__
     else v = s;
     out[t] = v;
   }
+}
+
+// One reduced axis of many terms.  They are added (or compared) in order, one
+// thread an output, so the time is that of the loads' round trips: kRedBatch
+// loads are in flight while the batch before is added, and a unit stride's
+// (UNIT: rows of a view, a line a lane) are 16 bytes wide.  Where it is taken
+// (us, sixteen loads at a time, each waited for, as above -> so, sums):
+//  - unit stride from 48 terms: 4096 x 48 3.8 -> 3.0, 512 x 3380 95 -> 19,
+//    262,144 x 96 85 -> 19 (16 terms: 1.0 to 1.1 times);
+//  - other strides from 192 terms below 65,536 outputs: 200 x 512 6.6 -> 5.0,
+//    3380 x 512 57 -> 32, 3380 x 16,384 88 -> 33 (128 x 512 4.7 -> 4.8, its
+//    maximum 4.6 -> 5.5; 400 x 65,536 17.2 -> 17.6).
+constexpr int kRedBatch = 48;
+template <bool UNIT, bool MAX>
+__global__ void __launch_bounds__(64) reduce_long_kernel(float* __restrict__ out, const float* __restrict__ x,
+                                                         RedArgs R, bool mean) {
+  const int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+  if (t >= R.nout) return;
+  int64_t rem = t, base = 0;
+  for (int d = R.kr - 1; d >= 0; --d) {
+    base += (rem % R.kdims[d]) * R.kst[d];
+    rem /= R.kdims[d];
+  }
+  const int64_t st = UNIT ? 1 : R.rst[0];
+  float s = 0.0f, m = -INFINITY;
+  bool nan = false;
+  auto load = [&](int64_t batch, float (&d)[kRedBatch]) {
+    const float* p = x + base + batch * kRedBatch * st;
+    if constexpr (UNIT) {  // a row of a view: a line a lane, 16 bytes of it at a time
+#pragma unroll
+      for (int u = 0; u < kRedBatch; u += 4) {
+        const kk_f4u q = *reinterpret_cast<const kk_f4u*>(p + u);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) d[u + e] = q[e];
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < kRedBatch; ++u, p += st) d[u] = *p;
+    }
+  };
+  auto add = [&](const float (&d)[kRedBatch]) {
+    if constexpr (MAX) {
+#pragma unroll
+      for (int u = 0; u < kRedBatch; ++u) {
+        nan |= __builtin_isnan(d[u]);
+        m = fmaxf(m, d[u]);
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < kRedBatch; ++u) s += d[u];
+    }
+  };
+  const int64_t full = R.nred / kRedBatch;  // whole batches
+  float v[kRedBatch], w[kRedBatch];
+  if (full > 0) {
+    load(0, v);
+    int64_t b = 0;
+    // (no condition inside, which would leave the waits at "all loads"; the
+    // barriers keep the scheduler from moving a batch's loads to its sums)
+    for (; b + 2 < full; b += 2) {
+      load(b + 1, w);
+      __builtin_amdgcn_sched_barrier(0);
+      add(v);
+      __builtin_amdgcn_sched_barrier(0);
+      load(b + 2, v);
+      __builtin_amdgcn_sched_barrier(0);
+      add(w);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (b + 1 < full) load(b + 1, w);
+    __builtin_amdgcn_sched_barrier(0);
+    add(v);
+    if (b + 1 < full) add(w);
+  }
+  // the rest, sixteen at a time (past the end: the last term again, not added)
+  for (int64_t j = full * kRedBatch; j < R.nred; j += 16) {
+    float q[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) q[u] = x[base + min(j + u, R.nred - 1) * st];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      if (j + u >= R.nred) continue;
+      s += q[u];
+      nan |= __builtin_isnan(q[u]);
+      m = fmaxf(m, q[u]);
+    }
+  }
+  float r;
+  if (MAX) r = nan ? NAN : m;
+  else if (mean) r = s / static_cast<float>(R.nred);
+  else r = s;
+  out[t] = r;
 }
 
 // ------------------------------------------------------------- launching
@@ -2724,11 +2788,29 @@ int kk_reduce(int op, const kk_tensor* out, const kk_tensor* x, uint32_t axes_ma
                     static_cast<const float*>(x->data), nout, nred, op);
     return check_launch("reduce_rows_kernel");
   }
+  const bool unit = R.rst[0] == 1;
+  if (R.rr == 1 && (unit ? nred >= kRedBatch : nred >= 4 * kRedBatch && nout < 65536) &&
+      ceil_div(nout, 64) <= 0x7fffffff) {
+    auto run = [&](auto unit_stride, auto max) {
+      KK_LAUNCH((reduce_long_kernel<decltype(unit_stride)::value, decltype(max)::value>),
+                dim3(static_cast<unsigned>(ceil_div(nout, 64))), dim3(64), 0, ctx().stream,
+                static_cast<float*>(out->data), static_cast<const float*>(x->data), R, op == KK_REDUCE_MEAN);
+    };
+    const std::true_type yes;
+    const std::false_type no;
+    if (unit) op == KK_REDUCE_MAX ? run(yes, yes) : run(yes, no);
+    else op == KK_REDUCE_MAX ? run(no, yes) : run(no, no);
+    return check_launch("reduce_long_kernel");
+  }
   // few outputs: a wave a block, over more CUs
   const int64_t threads = nout <= 64 * 256 ? 64 : 256;
   const unsigned grid = static_cast<unsigned>(std::min<int64_t>(ceil_div(nout, threads), 65535));
-  KK_LAUNCH(reduce_generic_kernel, dim3(grid), dim3(static_cast<unsigned>(threads)), 0, ctx().stream,
-                     static_cast<float*>(out->data), static_cast<const float*>(x->data), R, op);
+  if (R.rr == 1)
+    KK_LAUNCH(reduce_generic_kernel<true>, dim3(grid), dim3(static_cast<unsigned>(threads)), 0, ctx().stream,
+              static_cast<float*>(out->data), static_cast<const float*>(x->data), R, op);
+  else
+    KK_LAUNCH(reduce_generic_kernel<false>, dim3(grid), dim3(static_cast<unsigned>(threads)), 0, ctx().stream,
+              static_cast<float*>(out->data), static_cast<const float*>(x->data), R, op);
   return check_launch("reduce_generic_kernel");
 }
 

@@ -6,7 +6,7 @@ data; summation order differs from numpy's pairwise sums, nothing else."""
 import numpy as np
 import pytest
 
-from conftest import assert_bitexact, assert_close, rng
+from conftest import graph_us, assert_bitexact, assert_close, rng
 
 pytestmark = pytest.mark.gpu
 RTOL, ATOL = 1e-4, 1e-5
@@ -252,3 +252,41 @@ def test_reduce_strided_axis(gpu, op, rows, n, cols):
         if op == "ReduceMean":
             want = want / np.float32(n)
     assert_bitexact(got, want, f"{op} [{rows},{n},{cols}]")
+
+
+@pytest.mark.parametrize("op", ["ReduceSum", "ReduceMean", "ReduceMax"])
+@pytest.mark.parametrize("n", [1, 2, 7, 16, 47, 48, 49, 95, 96, 97, 143, 144, 160, 191, 192, 193, 239, 240, 500])
+def test_reduce_one_axis_lengths(gpu, op, n):
+    """The rows of a view at an odd offset (unit stride) and a middle axis,
+    around the lengths where their kernels change and their batches end: the
+    terms in order in fp32 (the maximum keeps NaN), bit for bit."""
+    r = rng(51)
+    base = r.normal(0, 1, (3, 37, n + 4)).astype(np.float32)
+    for x, axis, dev in ((base[:, :, 1:n + 1], 2, gpu.to_device(base).slice_axis(2, 1, n + 1)),
+                         (base.transpose(0, 2, 1)[:, 2:n + 2], 1, gpu.to_device(base).transpose((0, 2, 1)).slice_axis(1, 2, n + 2)),
+                         (np.ascontiguousarray(base[:, :, :n].transpose(0, 2, 1)), 1, None)):
+        x = x.copy()
+        if op == "ReduceMax" and dev is None:
+            x[1, n - 1, 5] = np.nan
+        got = gpu.ops.reduce(op, dev if dev is not None else gpu.to_device(x), [axis]).numpy()
+        terms = np.moveaxis(x, axis, 0)
+        if op == "ReduceMax":
+            want = terms.max(axis=0)
+        else:
+            want = np.zeros(terms.shape[1:], np.float32)
+            for t in terms:
+                want = want + t
+            if op == "ReduceMean":
+                want = want / np.float32(n)
+        assert_bitexact(got, np.expand_dims(want, axis), f"{op} axis {axis} n {n}")
+
+
+def test_reduce_short_axis_time(gpu):
+    """An axis of two terms, four million outputs: the bytes of an elementwise
+    sum of two tensors, in no more than four times its time (1.5 measured)."""
+    x = gpu.to_device(rng(52).normal(0, 1, (64, 2, 65536)).astype(np.float32))
+    out = gpu.DeviceTensor.empty((64, 1, 65536), np.float32)
+    a, b = x.slice_axis(1, 0, 1), x.slice_axis(1, 1, 2)
+    red = graph_us(gpu, lambda: gpu._lib.call("kk_reduce", 0, out.desc(), x.desc(), 2))
+    add = graph_us(gpu, lambda: gpu._lib.call("kk_binary", 0, out.desc(), a.desc(), b.desc()))
+    assert red < 4 * add, f"reduction {red:.1f} us, sum of two tensors {add:.1f}"
