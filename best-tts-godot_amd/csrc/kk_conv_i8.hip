@@ -189,7 +189,7 @@ struct ConvI8Args {
 // [1,256,67641] 69 -> 55 / 72 -> 57, over 7280 13.7 -> 12.7 / 14.3 -> 13.5;
 // 512 -> 512 k3 over 364 14.7 -> 10.3 / 15.5 -> 10.7.
 template <int WM, int WN, int WK, int NI, int R, bool RES, bool WIDE>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(R == 3 ? 3 : 2)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(R > 3 ? 2 : NI == 2 ? 3 : 4)))
 conv_i8_kernel(ConvI8Args A) {
   constexpr int TM = 64 * WM, TN = 32 * NI * WN;
   constexpr int kPitch = TN + 8;                   // floats a row of the output area
@@ -362,7 +362,7 @@ conv_i8_kernel(ConvI8Args A) {
       __syncthreads();  // every wave is done with the previous window
 #pragma unroll
       for (int i = 0; i < R; ++i) lda(st0 + lb + i, f[i]);
-      stage(c0, nc, std::integral_constant<int, NI == 2 && WK == 1 ? 2 : 4>{});
+      stage(c0, nc, std::integral_constant<int, WK == 1 ? 2 : 4>{});
     } else if (tid < TM) {
       // v = acc + cst[co] - wz * S, with cst = K wz xz - xz sum(a) (+ bias) and
       // S = sum of b over the receptive field; the weight zero point is one
@@ -517,28 +517,30 @@ conv_i8_kernel(ConvI8Args A) {
 #pragma unroll
       for (int mi = 0; mi < kMi; ++mi) {
         float yv[16][kNi];
+        if (kFull || row0 + 32 * mi < c_rem) {  // (a half past the channels stores nothing; wave-uniform)
 #pragma unroll
-        for (int reg = 0; reg < 16; ++reg)
+          for (int reg = 0; reg < 16; ++reg)
 #pragma unroll
-          for (int ni = 0; RES && ni < kNi; ++ni)  // (past the batch's end a load reads 0)
-            yv[reg][ni] = __builtin_bit_cast(
-                float, __builtin_amdgcn_raw_buffer_load_b32(
-                           rrs, r_off + static_cast<uint32_t>(32 * mi + 8 * (reg / 4) + reg % 4) * lout4 + 128u * ni, 0, 0));
+            for (int ni = 0; RES && ni < kNi; ++ni)  // (past the batch's end a load reads 0)
+              yv[reg][ni] = __builtin_bit_cast(
+                  float, __builtin_amdgcn_raw_buffer_load_b32(
+                             rrs, r_off + static_cast<uint32_t>(32 * mi + 8 * (reg / 4) + reg % 4) * lout4 + 128u * ni, 0, 0));
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const v4i c = *reinterpret_cast<const v4i*>(cst + lane_c + 32 * mi + 8 * q);
-          const f4a sc = *reinterpret_cast<const f4a*>(scl + lane_c + 32 * mi + 8 * q);
+          for (int q = 0; q < 4; ++q) {
+            const v4i c = *reinterpret_cast<const v4i*>(cst + lane_c + 32 * mi + 8 * q);
+            const f4a sc = *reinterpret_cast<const f4a*>(scl + lane_c + 32 * mi + 8 * q);
 #pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            const int reg = 4 * q + k, cr = 32 * mi + 8 * q + k;
-            if (!kFull && lane_c + cr >= c_rem) continue;
+            for (int k = 0; k < 4; ++k) {
+              const int reg = 4 * q + k, cr = 32 * mi + 8 * q + k;
+              if (!kFull && lane_c + cr >= c_rem) continue;
 #pragma unroll
-            for (int ni = 0; ni < kNi; ++ni) {
-              if (!kFull && lane_j + 32 * ni >= l_rem) continue;
-              const int v = t[mi][ni][reg] + c[k] + zS[ni];
-              const float y = static_cast<float>(v) * sc[k];
-              yv[reg][ni] = RES ? y + yv[reg][ni] : A.outf ? y : __builtin_bit_cast(float, v);
-              *reinterpret_cast<float*>(ob + (lane_off + static_cast<uint32_t>(cr) * lout4 + 128u * ni)) = yv[reg][ni];
+              for (int ni = 0; ni < kNi; ++ni) {
+                if (!kFull && lane_j + 32 * ni >= l_rem) continue;
+                const int v = t[mi][ni][reg] + c[k] + zS[ni];
+                const float y = static_cast<float>(v) * sc[k];
+                yv[reg][ni] = RES ? y + yv[reg][ni] : A.outf ? y : __builtin_bit_cast(float, v);
+                *reinterpret_cast<float*>(ob + (lane_off + static_cast<uint32_t>(cr) * lout4 + 128u * ni)) = yv[reg][ni];
+              }
             }
           }
         }
@@ -644,25 +646,30 @@ static bool conv_leaves_fit(int64_t stride, int64_t dilation, int64_t K) {
 }
 
 // The launch's block.  128 x 128 outputs when such blocks still give every
-// CU two (three share a CU); else 128 x 64 where those give every other CU
-// one (256 -> 256 k3 over 7280 steps, 228 blocks: 10.6 us against 12.0 for
+// CU two (three share a CU), and for more than 16 steps of 64 where a CU would
+// hold four blocks of 128 x 64 (256 -> 256 k11 over 30,280 steps 34 us against
+// 38; of fewer steps 128 x 64: k1 15.8 against 16.9);
+// else 128 x 64 (four share a CU) where those give every other CU one (256 -> 256 k3 over 7280 steps, 228 blocks: 10.6 us against 12.0 for
 // 64 x 64; k7 over 14560, 456 blocks: 19.0 against 25.2); else 64 x 64, its
 // waves sharing the reduction, for short rows, whose few blocks are bound by
 // the chain of steps of each (512 -> 512 k3 over 364, 24 blocks: 10.7 us
 // against 13.2), and up to a block a CU for reductions of more than 32 steps
-// of 64 (256 -> 256 k11 over 7280: 15.6 against 17.6).
+// (256 -> 256 k11 over 7280: 15.6 against 17.6).  Below 11 steps' worth of
+// channels the waves have too few to share (over 1000 steps: 22 -> 22 k3 6.9
+// against 5.4, k11 7.2 against 6.7; 128 -> 128 k3 7.5 against 6.8, k5 7.6 either
+// way; 64 -> 64 k11 7.1 against 7.4).
 struct ConvShape {
   int tm, tn;
 };
 static ConvShape conv_launch_shape(int64_t stride, int64_t dilation, int64_t K, int64_t N,
-                                   int64_t CinP, int64_t CoutP, int64_t Lout) {
+                                   int64_t Cin, int64_t CoutP, int64_t Lout) {
   const int tn = conv_tile_n(stride, dilation, K);
   const int64_t cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
-  if (tn == 128 && (N * (CoutP / kTileM) * ceil_div(Lout, 128) >= 2 * cus ||
-                    conv_lds(conv_rows(64, stride, dilation, K)) > kConvLds))
-    return {128, 128};
+  if (tn == 128 && N * (CoutP / kTileM) * ceil_div(Lout, 128) >= 2 * cus) return {128, 128};
   const int64_t blocks = N * (CoutP / kTileM) * ceil_div(Lout, 64);
-  return {2 * blocks < cus || (blocks < cus && CinP / kCinAlign * K > 32) ? 64 : 128, 64};
+  const int64_t steps = ceil_div(Cin, kCinAlign) * K;
+  if (tn == 128 && blocks > 3 * cus && steps > 16) return {128, 128};
+  return {(2 * blocks < cus && Cin * K >= 11 * kCinAlign) || (blocks < cus && steps > 32) ? 64 : 128, 64};
 }
 
 // The allocation-free entry point's workspace: a file-scope device array of
@@ -769,7 +776,6 @@ static int check_conv_integer(const kk_tensor* out, const kk_tensor* x, const kk
 }
 
 static int conv_launch(void (*kernel)(ConvI8Args), const dim3& grid, size_t lds, const ConvI8Args& A) {
-  if (lds > 65536) KK_TRY(allow_large_lds(reinterpret_cast<const void*>(kernel)));
   KK_LAUNCH(kernel, grid, dim3(256), lds, ctx().stream, A);
   return check_launch("conv_i8_kernel");
 }
@@ -842,7 +848,7 @@ static int conv_integer_run(const kk_tensor* out, const kk_tensor* x, const kk_t
     A.resid = resid ? static_cast<const float*>(resid->data) : nullptr;
     // leaf sums need the 128-step tiles (checked to fit by the caller)
     const ConvShape sh = leaves ? ConvShape{128, 128}
-                                : conv_launch_shape(stride, dilation, Kw, N, CinP, CoutP, Lout);
+                                : conv_launch_shape(stride, dilation, Kw, N, Cin, CoutP, Lout);
     if (leaves) {
       A.leaf = static_cast<float*>(leaves->data);
       A.nleaf = (Lout / 8192) * 64;
@@ -850,7 +856,9 @@ static int conv_integer_run(const kk_tensor* out, const kk_tensor* x, const kk_t
     A.W4 = static_cast<int>(conv_rows(sh.tn, stride, dilation, Kw));
     // Channels staged at once: all of them if three blocks a CU (two of the
     // smaller tiles, whose blocks are few) keep their LDS, else equal shares.
-    const int64_t lds_max = sh.tn == 128 ? 53248 : kConvLds;
+    const int64_t cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
+    const int64_t per_cu = sh.tm == 64 ? 2 : ceil_div(N * (CoutP / kTileM) * ceil_div(Lout, sh.tn), cus);
+    const int64_t lds_max = sh.tn == 128 || per_cu == 3 ? 53248 : per_cu > 3 ? 40960 : kConvLds;
     int64_t parts = 1;
     while (parts < CinP / kCinAlign &&
            conv_lds(A.W4, ceil_div(CinP / kCinAlign, parts) * kCinAlign) > lds_max)
@@ -858,7 +866,7 @@ static int conv_integer_run(const kk_tensor* out, const kk_tensor* x, const kk_t
     A.SC = static_cast<int>(ceil_div(CinP / kCinAlign, parts) * kCinAlign);
     // the window, or after it the outputs (64 x 136 or 128 x 72 floats; with
     // the reduction shared, the waves' 12 exchanged tiles of 4 KB)
-    const int out_area = sh.tm == 64 ? 49152 + 1024 : sh.tn == 64 ? 128 * 72 * 4 : 64 * 136 * 4;
+    const int out_area = sh.tm == 64 ? 49152 + 1024 : sh.tn == 64 ? 0 : 64 * 136 * 4;
     A.area = static_cast<int>(std::max<int64_t>(A.W4 * int64_t{A.SC + 16}, out_area));
     const dim3 grid(static_cast<unsigned>(ceil_div(Lout, sh.tn)),
                     static_cast<unsigned>(ceil_div(Cout, sh.tm)), static_cast<unsigned>(N));

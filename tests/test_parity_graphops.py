@@ -312,6 +312,35 @@ def test_conv_integer_rows_at_any_alignment(gpu, n, cin, L, pad, dil, skip):
     assert_bitexact(got, want.astype(np.int32), f"ConvInteger L={L} skip={skip}")
 
 
+@pytest.mark.parametrize("cin,cout,k,L,dil", [
+    (64, 64, 11, 700, 1), (64, 64, 7, 701, 1), (22, 22, 11, 999, 2),      # 64 x 64 outputs a block; too few steps for it
+    (40, 300, 3, 17281, 1), (1024, 512, 1, 12801, 1),   # 128 x 64, four blocks a CU: one window, several
+    (512, 256, 5, 19233, 9),                            # three a CU, two windows
+    (256, 200, 5, 24700, 1), (512, 130, 3, 25001, 1)])  # 128 x 128 for many steps
+def test_conv_integer_launch_shapes(gpu, cin, cout, k, L, dil):
+    """Every block shape and share of the channels staged at once, partial
+    blocks among them: int32 sums bit for bit (products of at most 2^31 in
+    float64 are exact), and the scaled residual form from the same sums."""
+    r = rng(53)
+    dv, pad = gpu.to_device, dil * (k - 1) // 2
+    x = r.integers(0, 256, (1, cin, L)).astype(np.uint8)
+    w = r.integers(0, 256, (cout, cin, k)).astype(np.uint8)
+    rows = np.unique(np.r_[0:16, cout // 2 - 8:cout // 2 + 8, cout - 16:cout] % cout)  # (the channels checked)
+    xp = np.pad(x[0].astype(np.float64) - 99, ((0, 0), (pad, pad)))
+    wf = w[rows].astype(np.float64) - 140
+    lout = L + 2 * pad - dil * (k - 1)
+    want = sum(wf[:, :, t] @ xp[:, t * dil:t * dil + lout] for t in range(k)).astype(np.int32)
+    args = (dv(x), dv(w), dv(np.array(99, np.uint8)), dv(np.array(140, np.uint8)))
+    kw = dict(pads=(pad, pad), dilation=dil)
+    assert_bitexact(gpu.ops.conv_integer(*args, **kw).numpy()[0, rows], want, "sums")
+    bias = r.integers(-10 ** 6, 10 ** 6, cout).astype(np.int32)
+    sc = r.uniform(1e-4, 1e-3, cout).astype(np.float32)
+    res = r.normal(0, 1, (1, cout, lout)).astype(np.float32)
+    got = gpu.ops.conv_integer_scaled(*args, dv(bias), dv(sc), resid=dv(res), **kw).numpy()
+    y = (want + bias[rows, None]).astype(np.float32) * sc[rows, None]
+    assert_bitexact(got[0, rows], y + res[0, rows], "scaled, with a residual")
+
+
 def test_conv_integer_exact_beyond_2_24(gpu, oracle):
     """Sums above 2^24: the device is exact int32 (int8 matrix cores), while
     the reference convolves the shifted integers in float32 and rounds
