@@ -174,8 +174,7 @@ struct ConvI8Args {
 // With WK = 4 the waves take a quarter of the steps each and add their int32
 // tiles through LDS (exact in any order).
 // RES: the scaled fp32 output plus A.resid.  WIDE: the results leave through
-// LDS (aliasing the staged window), 16 bytes a lane, so that a row which
-// starts off a 128-byte line touches five lines a block instead of eight.
+// LDS (aliasing the staged window), 16 bytes a lane.
 //
 // Bound, a block at a time, by a chain of phases (128 -> 128 k11 over 405841
 // steps, three blocks a CU: window 2 us, products 7 us with the SIMD's matrix
@@ -193,13 +192,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(R > 3 
 conv_i8_kernel(ConvI8Args A) {
   constexpr int TM = 64 * WM, TN = 32 * NI * WN;
   constexpr int kPitch = TN + 8;                   // floats a row of the output area
-  constexpr int kPhases = TM * kPitch * 4 > 40960 ? 2 : 1;  // halves (mi) of the tile that pass through it
-  constexpr int kRows = TM / kPhases;              // output rows in the area at a time
-  constexpr int kVec = kRows * TN / 4 / 256;       // float4 a thread of one pass
   extern __shared__ __align__(16) int8_t conv_lds[];
   const int pitch = A.SC + 16;                                    // odd multiple of 16: staggered banks
   int8_t* Bw = conv_lds;                                          // [W4][pitch]
-  float* ep = reinterpret_cast<float*>(conv_lds);                 // [kRows][kPitch], after the reduction
+  float* ep = reinterpret_cast<float*>(conv_lds);                 // [64][kPitch], after the reduction
   int* cst = reinterpret_cast<int*>(conv_lds + A.area);           // [TM] constant term
   float* scl = reinterpret_cast<float*>(cst + TM);                // [TM] scale
   const int tid = threadIdx.x, lane = tid & 63;
@@ -562,52 +558,46 @@ conv_i8_kernel(ConvI8Args A) {
     else store(std::false_type{});
     return;
   }
-  lds_barrier();  // the window (or the exchanged tiles) may be overwritten
-  // a thread's float4 k of half ph: rows tid / (TN / 4) + kStep k of the area
-  constexpr int kStep = 256 / (TN / 4);
-  const int e0 = tid / (TN / 4), c4 = tid % (TN / 4);
+  lds_barrier();  // the window may be overwritten
+  // WIDE: 128 x 128 outputs of whole channel blocks, 64 rows (half mi) at a
+  // time; a thread's float4 k: rows tid / 32 + 8 k of the area
+  static_assert(!WIDE || (WM == 2 && TN == 128 && WK == 1), "the area holds 64 rows of 128");
+  const int e0 = tid / 32, c4 = tid % 32;
   const uint32_t off0 = static_cast<uint32_t>(e0) * lout4 + 16u * c4;
-  // row e of the output area in half ph: its channel in the block
-  auto chan = [&](int e, int ph) { return kPhases == 2 ? (e >> 5) * 64 + 32 * ph + (e & 31) : e; };
+  // row e of the area in half mi: its channel in the block
+  auto chan = [](int e, int mi) { return (e >> 5) * 64 + 32 * mi + (e & 31); };
 #pragma unroll
-  for (int ph = 0; ph < kPhases; ++ph) {
+  for (int mi = 0; mi < kMi; ++mi) {
 #pragma unroll
-    for (int mi = 0; mi < kMi; ++mi) {
-      if (kPhases == 2 && mi != ph) continue;
+    for (int q = 0; q < 4; ++q) {
+      // rows 8q + 4g .. + 3 of the 32 x 32 tile: registers 4q .. 4q + 3
+      const int cl = lane_c + 32 * mi + 8 * q, e = wm * 32 + 8 * q + 4 * g;
+      const v4i c = *reinterpret_cast<const v4i*>(cst + cl);
+      const f4a sc = *reinterpret_cast<const f4a*>(scl + cl);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        // rows 8q + 4g .. + 3 of the 32 x 32 tile: registers 4q .. 4q + 3
-        const int cl = lane_c + 32 * mi + 8 * q;
-        const int e = kPhases == 2 ? wm * 32 + 8 * q + 4 * g : cl;
-        const v4i c = *reinterpret_cast<const v4i*>(cst + cl);
-        const f4a sc = *reinterpret_cast<const f4a*>(scl + cl);
+      for (int k = 0; k < 4; ++k)
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
-#pragma unroll
-          for (int ni = 0; ni < kNi; ++ni) {
-            const int v = t[mi][ni][4 * q + k] + c[k] + zS[ni];
-            ep[(e + k) * kPitch + lane_j + 32 * ni] =
-                A.outf ? static_cast<float>(v) * sc[k] : __builtin_bit_cast(float, v);
-          }
-      }
+        for (int ni = 0; ni < kNi; ++ni) {
+          const int v = t[mi][ni][4 * q + k] + c[k] + zS[ni];
+          ep[(e + k) * kPitch + lane_j + 32 * ni] =
+              A.outf ? static_cast<float>(v) * sc[k] : __builtin_bit_cast(float, v);
+        }
     }
     lds_barrier();
-    if (full) {
+    if (l_rem == TN) {
 #pragma unroll
-      for (int k = 0; k < kVec; ++k)
-        *reinterpret_cast<f4u*>(ob + (off0 + static_cast<uint32_t>(chan(kStep * k, ph)) * lout4)) =
-            *reinterpret_cast<const f4a*>(ep + (e0 + kStep * k) * kPitch + 4 * c4);
+      for (int k = 0; k < 8; ++k)
+        *reinterpret_cast<f4u*>(ob + (off0 + static_cast<uint32_t>(chan(8 * k, mi)) * lout4)) =
+            *reinterpret_cast<const f4a*>(ep + (e0 + 8 * k) * kPitch + 4 * c4);
     } else {
-      for (int k = tid; k < kRows * TN; k += 256) {
-        const int e = k / TN, col = k % TN, cl = chan(e, ph);
-        if (cl >= c_rem || col >= l_rem) continue;
-        *reinterpret_cast<float*>(ob + (static_cast<uint32_t>(cl) * lout4 + 4u * col)) = ep[e * kPitch + col];
+      for (int k = tid; k < 64 * TN; k += 256) {
+        const int e = k / TN, col = k % TN;
+        if (col < l_rem)
+          *reinterpret_cast<float*>(ob + (static_cast<uint32_t>(chan(e, mi)) * lout4 + 4u * col)) = ep[e * kPitch + col];
       }
     }
-    if constexpr (TN == 128) {
-      if (leafy) leaf_sums(ph);
-    }
-    if (ph + 1 < kPhases) lds_barrier();  // (the next half reuses the area)
+    if (leafy) leaf_sums(mi);
+    if (mi + 1 < kMi) lds_barrier();  // (the next half reuses the area)
   }
 }
 
@@ -639,8 +629,8 @@ static int conv_tile_n(int64_t stride, int64_t dilation, int64_t K) {
   return 0;
 }
 
-// Whether leaf sums can be formed: the window of a 128-step tile and 64 rows
-// of its outputs side by side in 64 KB.
+// Whether leaf sums are formed: the window of a 128-step tile and 64 rows of
+// its outputs within 64 KB (they alias; the bound is what callers know).
 static bool conv_leaves_fit(int64_t stride, int64_t dilation, int64_t K) {
   return ceil_div(conv_lds(conv_rows(128, stride, dilation, K)), 16) * 16 + 64 * 136 * 4 <= kConvLds;
 }
@@ -864,9 +854,19 @@ static int conv_integer_run(const kk_tensor* out, const kk_tensor* x, const kk_t
            conv_lds(A.W4, ceil_div(CinP / kCinAlign, parts) * kCinAlign) > lds_max)
       ++parts;
     A.SC = static_cast<int>(ceil_div(CinP / kCinAlign, parts) * kCinAlign);
-    // the window, or after it the outputs (64 x 136 or 128 x 72 floats; with
-    // the reduction shared, the waves' 12 exchanged tiles of 4 KB)
-    const int out_area = sh.tm == 64 ? 49152 + 1024 : sh.tn == 64 ? 0 : 64 * 136 * 4;
+    // 16-byte stores through LDS, for whole channel blocks without a residual
+    // into an output that the last-level cache (256 MB) does not hold; with leaf
+    // sums, which pass through LDS anyway, from 160 MB on.  us without -> with
+    // them, 128 -> 128 k11 / k3, 256 -> 256 k3: 208 MB 114 -> 119 / 63 -> 73 / 96 ->
+    // 98, with leaf sums 118 -> 114 / 76 -> 74 / 98 -> 94; 300 MB 190 -> 176 / 131
+    // -> 122 / 180 -> 167; 140 MB 77 -> 88 / 44 -> 54 / 65 -> 74, with leaf sums
+    // 82 -> 80 / 50 -> 50 / 70 -> 69.  Rows of any length alike; with 64 channels,
+    // half a block, or a residual they never paid.
+    const bool wide = sh.tn == 128 && !A.resid && Cout % kTileM == 0 &&
+                      N * Cout * Lout * 4 > (leaves ? int64_t{160} : int64_t{256}) << 20;
+    // the window, or after it the exchanged tiles (12 of 4 KB) or half a
+    // block's outputs (64 x 136 floats)
+    const int out_area = sh.tm == 64 ? 49152 + 1024 : wide || leaves ? 64 * 136 * 4 : 0;
     A.area = static_cast<int>(std::max<int64_t>(A.W4 * int64_t{A.SC + 16}, out_area));
     const dim3 grid(static_cast<unsigned>(ceil_div(Lout, sh.tn)),
                     static_cast<unsigned>(ceil_div(Cout, sh.tm)), static_cast<unsigned>(N));
@@ -875,13 +875,7 @@ static int conv_integer_run(const kk_tensor* out, const kk_tensor* x, const kk_t
       const size_t lds = static_cast<size_t>(A.area + 2 * 4 * sh.tm);
 #define KK_CONV_LAUNCH(...) rc = A.resid ? conv_launch(conv_i8_kernel<__VA_ARGS__, true, false>, grid, lds, A) \
                                          : conv_launch(conv_i8_kernel<__VA_ARGS__, false, false>, grid, lds, A)
-      // Rows of odd length into an output that the last-level cache does not
-      // hold: 16-byte stores through LDS ([1,128,405841] k11 114.4 -> 109.6
-      // us, with leaf sums 113.7 -> 107.3; into 69 MB, [1,256,67641] k7, they
-      // cost 2.6 us).  With a residual they never paid.
-      const bool beyond_llc = N * Cout * Lout * 4 > (int64_t{128} << 20);
-      if (sh.tn == 128 && !A.resid && Lout % 2 != 0 && beyond_llc)
-        rc = conv_launch(conv_i8_kernel<2, 2, 1, 2, 3, false, true>, grid, lds, A);
+      if (wide) rc = conv_launch(conv_i8_kernel<2, 2, 1, 2, 3, false, true>, grid, lds, A);
       else if (sh.tn == 128) KK_CONV_LAUNCH(2, 2, 1, 2, 3);
       else if (sh.tm == 128) KK_CONV_LAUNCH(2, 2, 1, 1, 3);
       else KK_CONV_LAUNCH(1, 1, 4, 2, 6);

@@ -825,6 +825,48 @@ def test_conv_leaf_sums(gpu, cin, cout, k, L, pad, dil, resid):
     assert_bitexact(lv, ref.astype(np.float32), f"leaf sums {cin}->{cout} k{k}")
 
 
+@pytest.mark.parametrize("form,N,cout,L", [
+    ("int32", 1, 128, 524_293), ("fp32", 1, 256, 262_150), ("fp32", 2, 128, 262_151),
+    ("leaves", 1, 128, 327_683), ("leaves", 2, 128, 163_847), ("leaves", 1, 256, 163_844)])
+def test_conv_integer_output_beyond_the_cache(gpu, form, N, cout, L):
+    """The 16-byte stores of outputs just past 256 MB (160 with leaf sums),
+    rows off a line and a last block of a few steps: every channel's edges
+    and some whole rows bit for bit."""
+    r = rng(54)
+    dv, cin, k = gpu.to_device, 5, 3
+    assert N * cout * L * 4 > (160 if form == "leaves" else 256) << 20
+    x = r.integers(0, 256, (N, cin, L)).astype(np.uint8)
+    w = r.integers(0, 256, (cout, cin, k)).astype(np.uint8)
+    bias = r.normal(0, 0.5, cout).astype(np.float32)
+    sa, sw = np.float32(0.0051), np.float32(0.0037)
+    dw, wz, xz = dv(w), dv(np.array(131, np.uint8)), dv(np.array(117, np.uint8))
+    leaves = None
+    if form == "int32":
+        got = gpu.ops.conv_integer(dv(x), dw, xz, wz, (1, 1)).numpy()
+    else:
+        res = gpu.ops.conv_integer_scaled_qbias(dv(x), dw, xz, wz, dv(bias), dv(np.array(sa)), dv(np.array(sw)),
+                                                pads=(1, 1), packed=gpu.ops.conv_integer_pack(dw, wz),
+                                                leaves=form == "leaves")
+        got, leaves = (res[0].numpy(), res[1].numpy()) if form == "leaves" else (res.numpy(), None)
+    sc = sa * sw
+    ib = np.floor(bias / sc).astype(np.int32)
+
+    def want(xs, rows):  # columns of a padded piece xs
+        sums = sum((w[rows, :, t].astype(np.int32) - 131) @ xs[:, t:t + xs.shape[1] - 2] for t in range(k))
+        return sums if form == "int32" else (sums + ib[rows, None]).astype(np.float32) * sc
+    for n in range(N):
+        xp = np.pad(x[n].astype(np.int32) - 117, ((0, 0), (1, 1)))
+        every = np.arange(cout)
+        for lo, hi in ((0, 300), (L // 2, L // 2 + 300), (L - 300, L)):
+            assert_bitexact(got[n, :, lo:hi], want(xp[:, lo:hi + 2], every), f"{form} item {n} columns {lo}..{hi}")
+        rows = np.array([0, 33, 64, 95, cout - 1])
+        assert_bitexact(got[n, rows], want(xp, rows), f"{form} item {n} rows")
+    if leaves is not None:
+        nleaf = (L // 8192) * 64
+        rows = got.reshape(N * cout, L)[:, :nleaf * 128].reshape(N * cout, nleaf, 128)
+        assert_bitexact(leaves.reshape(N * cout, nleaf), np.add.reduce(rows, axis=2), "leaf sums")
+
+
 @pytest.mark.parametrize("kind", ["leaky", "snake", "affine"])
 def test_instance_norm_quant_with_leaf_sums(gpu, kind):
     """kk_instance_norm_quant_leaves on a conv's output with that conv's leaf
