@@ -322,13 +322,30 @@ static int launch_fir(const kk_tensor* x, const kk_tensor* taps, int center, flo
   const float* hp = static_cast<const float*>(taps->data);
   const int t = static_cast<int>(numel(taps));
   if (t >= kMfmaMinTaps) {
-    // Tiles a wave: the blocks go round the CUs whole, and a block of one,
-    // two or four tiles a wave takes 5.5, 5.1 x 2 or 4.9 x 4 us (1023 taps):
-    // 1,060,000 samples 29.5, 31.4 and 38.3 us, 1,500,000 35.3, 32.5, 39.4,
-    // 2,029,200 45.4, 40.9, 40.6, 2,154,000 48.9, 50.9, 53.9.
+    // Tiles a wave: blocks of one, two or four go round the CUs whole.  Costs
+    // of a round, in hundredths of a tile's 10 ns a tap at 1023 taps, from
+    // 20,000 to 8,000,000 samples:
+    //  - three blocks and more a CU by their LDS: 47, 87 and 167 (51, 98, 183 for
+    //    the first block of a CU, alone there; 80 for two below 64 taps).  Four
+    //    are not worth their registers below 192 taps (800,000 samples x 128:
+    //    8.5, 8.6 and 9.3 us; 8,000,000: 34.6, 32.8, 34.7).
+    //  - from about 2,700 taps two blocks, from 3,800 one, whose window and
+    //    taps are staged with less or nothing in their shadow: half or all of a
+    //    tile's time more (4096 taps x 600,000: 99, 98 and 78 us; 1,060,000:
+    //    159, 142, 152; 3000 taps x 2,154,000: 161, 148, 153).
+    // 1023 taps: 400,000 samples 16.4, 18.0 and 25.4 us, 800,000 25.8, 25.9, 26.6,
+    // 1,060,000 32.1, 33.7, 40.8, 1,500,000 37.8, 34.7, 41.4, 2,029,200 48.4, 43.1,
+    // 42.7.  (32 to 47 taps over 2,000,000 to 2,600,000 samples take up to 1.06
+    // times the VALU kernel's time, below and above that less.)
     const int64_t cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
-    auto rounds = [&](int64_t tiles) { return ceil_div(ceil_div(n, 1024 * tiles), cus); };
-    const int64_t c1 = 55 * rounds(1), c2 = 102 * rounds(2), c4 = 196 * rounds(4);
+    const int resident = 163840 / fir_lds(1024, fir_units(t));
+    auto cost = [&](int64_t nc) {
+      const int64_t rounds = ceil_div(ceil_div(n, 1024 * nc), cus);
+      if (resident < 3) return rounds * (nc * 50 + (resident < 2 ? 50 : 25));
+      if (rounds <= 1) return nc == 1 ? int64_t{51} : nc == 2 ? int64_t{98} : int64_t{183};
+      return rounds * (nc == 1 ? 47 : nc == 2 ? (t < 64 ? 80 : 87) : 167);
+    };
+    const int64_t c1 = cost(1), c2 = cost(2), c4 = t < 192 ? INT64_MAX : cost(4);
     auto run = [&](auto nc) {
       constexpr int kNc = decltype(nc)::value;
       return pcm ? launch_mfma<kNc, true>(xp, n, hp, t, center, y, pcm, gain)

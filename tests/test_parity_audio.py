@@ -70,6 +70,46 @@ def test_fir_matrix_core_tiles(gpu, oracle, n, t, c):
         assert (err <= bound[fin]).all(), f"{special}: max err/bound {float((err / bound[fin]).max()):.3g}"
 
 
+def fma_chain(h, x):
+    """sum_k h[k] x[k:k + m] in order, one correctly rounded fused
+    multiply-add a term: the product is exact in float64, and its sum with
+    the accumulator is rounded to odd there, so that the rounding to float32
+    is that of the exact sum."""
+    m = x.size - h.size + 1
+    acc = np.zeros(m, np.float32)
+    for k in range(h.size):
+        p = np.float64(h[k]) * x[k:k + m].astype(np.float64)
+        a = acc.astype(np.float64)
+        s = p + a
+        b = s - p
+        err = (p - (s - b)) + (a - b)  # p + a - s, exactly
+        even = (s.view(np.int64) & 1) == 0
+        s = np.where((err != 0) & even, np.nextafter(s, np.where(err > 0, np.inf, -np.inf)), s)
+        acc = s.astype(np.float32)
+    return acc
+
+
+@pytest.mark.parametrize("n,t,c", [
+    (3000, 31, 4), (3000, 32, -1), (3001, 49, 7), (3003, 271, -1), (2999, 1023, -1), (2500, 4096, 100),
+    (1500001, 1023, -1),   # two tiles a wave
+    (2029203, 1023, -1), (1060001, 4096, -1), (3200003, 40, 3), (4000001, 255, 17)])  # four, and other costs
+def test_fir_is_the_tap_chain(gpu, n, t, c):
+    """The FIR, fp32 and PCM16, bit for bit the chain of fused multiply-adds
+    in tap order, at the waveform's edges and inside it."""
+    r = rng(55)
+    x = r.normal(0, 0.3, n).astype(np.float32)
+    h = r.normal(0, 0.05, t).astype(np.float32)
+    dx, dh = gpu.to_device(x), gpu.to_device(h)
+    got = gpu.ops.fir(dx, dh, c).numpy()
+    cc = (t - 1) // 2 if c < 0 else c
+    for lo in sorted({0, n // 2, max(0, n - 2500)}):
+        hi = min(n, lo + 2500)
+        piece = x[np.clip(np.arange(lo - cc, hi - cc + t - 1), 0, n - 1)]
+        np.testing.assert_array_equal(got[lo:hi].view(np.uint32), fma_chain(h, piece).view(np.uint32))
+    fused = gpu.to_host(gpu.ops.fir_pcm16(dx, dh, c, 0.9))
+    np.testing.assert_array_equal(fused, gpu.to_host(gpu.ops.pcm16(gpu.ops.fir(dx, dh, c), 0.9)))
+
+
 def test_fir_notch_removes_the_hop_tones(gpu, oracle):
     """A waveform carrying the iSTFT's 4800 / 9600 Hz ring: the device filter
     takes both tones down by at least 40 dB and leaves a 1 kHz tone within
