@@ -356,9 +356,10 @@ conv_i8_kernel(ConvI8Args A) {
     const int lb = first_step(nc), le = WK > 1 ? (wk + 1) * steps / WK : steps;
     if (c0 > 0) {
       __syncthreads();  // every wave is done with the previous window
+      // (the fragments after the window, whose items take their registers)
+      stage(c0, nc, std::integral_constant<int, 5>{});
 #pragma unroll
       for (int i = 0; i < R; ++i) lda(st0 + lb + i, f[i]);
-      stage(c0, nc, std::integral_constant<int, WK == 1 ? 2 : 4>{});
     } else if (tid < TM) {
       // v = acc + cst[co] - wz * S, with cst = K wz xz - xz sum(a) (+ bias) and
       // S = sum of b over the receptive field; the weight zero point is one
@@ -644,10 +645,10 @@ static bool conv_leaves_fit(int64_t stride, int64_t dilation, int64_t K) {
 // waves sharing the reduction, for short rows, whose few blocks are bound by
 // the chain of steps of each (512 -> 512 k3 over 364, 24 blocks: 10.7 us
 // against 13.2), and up to a block a CU for reductions of more than 32 steps
-// (256 -> 256 k11 over 7280: 15.6 against 17.6).  Below 11 steps' worth of
-// channels the waves have too few to share (over 1000 steps: 22 -> 22 k3 6.9
-// against 5.4, k11 7.2 against 6.7; 128 -> 128 k3 7.5 against 6.8, k5 7.6 either
-// way; 64 -> 64 k11 7.1 against 7.4).
+// (256 -> 256 k11 over 7280: 15.6 against 17.6).  Below 12 steps (11
+// of whole channels) the waves have too few to share (over 1000 steps: 22 -> 22
+// k3 6.9 against 5.4, k11 7.2 against 6.7; 128 -> 128 k3 7.5 against 6.8, k5 7.6
+// either way; 64 -> 64 k11 7.1 against 7.4, 22 -> 256 k12 stride 6 9.2 against 9.8).
 struct ConvShape {
   int tm, tn;
 };
@@ -659,7 +660,7 @@ static ConvShape conv_launch_shape(int64_t stride, int64_t dilation, int64_t K, 
   const int64_t blocks = N * (CoutP / kTileM) * ceil_div(Lout, 64);
   const int64_t steps = ceil_div(Cin, kCinAlign) * K;
   if (tn == 128 && blocks > 3 * cus && steps > 16) return {128, 128};
-  return {(2 * blocks < cus && Cin * K >= 11 * kCinAlign) || (blocks < cus && steps > 32) ? 64 : 128, 64};
+  return {(2 * blocks < cus && (steps >= 12 || Cin * K >= 11 * kCinAlign)) || (blocks < cus && steps > 32) ? 64 : 128, 64};
 }
 
 // The allocation-free entry point's workspace: a file-scope device array of
