@@ -127,7 +127,7 @@ __global__ void __launch_bounds__(kThreads) fir_kernel(const float* __restrict__
 // Bound by the matrix cores (2,029,200 samples x 1023 taps: 27.7 us at their
 // rate).  A wave takes NC tiles, which share the taps' reads.  Measured, 1023
 // taps: 2,029,200 samples 67.4 -> 40.0 us (PCM16 65.1 -> 38.8), 1,060,000
-// 52.7 -> 29.5, 400,000 33.8 -> 14.2, 2400 32.1 -> 10.3; 64 taps over
+// 52.7 -> 29.5, 400,000 36.0 -> 16.4, 2400 32.1 -> 10.3; 64 taps over
 // 1,060,000 7.1 either way, over 24,000 5.2 -> 3.8.
 typedef float fir_f4 __attribute__((ext_vector_type(4)));
 
@@ -323,8 +323,8 @@ static int launch_fir(const kk_tensor* x, const kk_tensor* taps, int center, flo
   const int t = static_cast<int>(numel(taps));
   if (t >= kMfmaMinTaps) {
     // Tiles a wave: blocks of one, two or four go round the CUs whole.  Costs
-    // of a round, in hundredths of a tile's 10 ns a tap at 1023 taps, from
-    // 20,000 to 8,000,000 samples:
+    // of a round (0.1 us at 1023 taps), measured from 32 to 4096 taps and 20,000
+    // to 8,000,000 samples:
     //  - three blocks and more a CU by their LDS: 47, 87 and 167 (51, 98, 183 for
     //    the first block of a CU, alone there; 80 for two below 64 taps).  Four
     //    are not worth their registers below 192 taps (800,000 samples x 128:

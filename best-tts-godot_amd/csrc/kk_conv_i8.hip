@@ -179,7 +179,7 @@ struct ConvI8Args {
 // Bound, a block at a time, by a chain of phases (128 -> 128 k11 over 405841
 // steps, three blocks a CU: window 2 us, products 7 us with the SIMD's matrix
 // core shared by three waves, 2.4 alone, epilogue 4 us), the matrix cores
-// busy 27% of the time and HBM at half its rate.  What shortened the chain:
+// busy 29% of the time and HBM at half its rate.  What shortened the chain:
 // one round trip for the window instead of one per 64 channels and item, the
 // receptive fields' sums from the fragments in the products' shadow (a pass
 // over the staged rows and a barrier before), constants read as vectors.
