@@ -856,7 +856,8 @@ static bool make_args(CArgs* a, const Geo& g, bool taps_first, const kk_tensor* 
     a->qs = static_cast<int>(stride); a->ta = static_cast<int>(-pad0); a->tm = static_cast<int>(dilation);
     a->os = 1; a->oph = 0;
   }
-  a->wbytes = static_cast<int>(g.bytes);
+  // (no more than convh_pack wrote: a row tile past the last reads 0)
+  a->wbytes = static_cast<int>(g.MT * a->KS * 1024);
   return true;
 }
 

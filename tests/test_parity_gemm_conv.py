@@ -625,6 +625,29 @@ def test_8bit_conv_of_128_channel_rounds_windows(gpu, k, dil, stride):
                 assert err < np.sqrt(256 * k) * 2.0 ** -24, f"cout {cout} item {n}: relative error {err:.2e}"
 
 
+@pytest.mark.parametrize("k,dil,L", [(3, 40, 20000), (7, 14, 9000), (5, 1, 4000)])
+def test_8bit_conv_of_128_channel_rounds_packed_into_used_memory(gpu, k, dil, L):
+    """What the packed buffer's memory held before reaches no output: row
+    tiles past the last (130 channels) and taps the layout does not pad."""
+    r = rng(56)
+    dv, pad = gpu.to_device, dil * (k - 1) // 2
+    x = dv(r.normal(0, 1, (1, 128, L)).astype(np.float32))
+    w = dv(r.integers(-127, 128, (130, 128, k)).astype(np.int8))
+    kw = dict(w_scale=dv(np.array(np.float32(2.0 ** -8))))
+    size = gpu.ops.conv_pack(w, None, False, 1).shape[0]
+    got = []
+    for fill in (0, 255):
+        used = dv(np.full(size, fill, np.uint8))
+        at = used.ptr
+        gpu.sync()
+        del used
+        pk = gpu.ops.conv_pack(w, None, False, 1)
+        assert pk.ptr == at, "the pool gave other memory"
+        got.append(gpu.ops.conv1d(x, w, None, (pad, pad), 1, dil, packed=pk, **kw).numpy())
+        del pk
+    assert_bitexact(got[1], got[0], f"k{k} dilation {dil}")
+
+
 @pytest.mark.parametrize("cin,cout,k,dil,L", [(1024, 256, 7, 9, 9000), (512, 512, 2, 70, 2400), (512, 512, 4, 33, 2400)])
 def test_8bit_conv_of_wide_windows_time(gpu, cin, cout, k, dil, L):
     """Windows past what a block of 64 columns stages take no longer than the
