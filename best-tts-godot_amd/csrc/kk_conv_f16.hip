@@ -428,8 +428,9 @@ __global__ void __launch_bounds__(kThreads) convh_kernel(CArgs A) {
 // The factor keeps the lower parts of the smallest floats out of bf16's
 // subnormals (unscaled, activations below 2^-110 lost bits, and all but eight
 // at 1e-38); the sums leave it in the epilogue.  It costs a multiplication a
-// staged value (512 -> 512 k3 over 2400 steps 22.7 -> 23.0 us).  The reduction runs tap-major (k =
-// t' Cin + ci): no padded taps, and an operand is eight channels at one time.
+// staged value (512 -> 512 k3 over 2400 steps 22.7 -> 23.0 us).  The reduction
+// runs tap-major (k = t' Cin + ci): no padded taps, and an operand is eight
+// channels at one time.
 //
 // A block owns 64 rows x 32 NI columns; its four waves take a quarter of the
 // channels each and own nothing in common until they add their tiles.  A wave
@@ -447,11 +448,11 @@ __global__ void __launch_bounds__(kThreads) convh_kernel(CArgs A) {
 // scalar fp32 products.
 //
 // Bound by each wave's chain (a chunk: window, products) at one or two waves
-// a SIMD.  us, the kernel above -> this one: Conv1d 512 -> 512 k3 over 2400
-// steps 32.7 -> 22.9, over 7000 77 -> 46, over 40 18.8 -> 14.2; 256 -> 256 k3
-// over 2400 15.8 -> 11.2; 512 -> 512 k7 over 7000 135 -> 99; ConvTranspose1d
-// 512 -> 256 k20 s10 over 240 16.5 -> 13.7, over 700 28.9 -> 22.1.  No further
-// from 64 bits (2.0e-7 -> 1.9e-7 relative for the first).
+// a SIMD.  us, the kernel above (fp16 layout) -> this one: Conv1d 512 -> 512 k3
+// over 2400 steps 32.7 -> 22.9, over 7000 76 -> 45, over 40 18.9 -> 10.3; 256 ->
+// 256 k3 over 2400 15.5 -> 11.3; 512 -> 512 k7 over 7000 135 -> 87;
+// ConvTranspose1d 512 -> 256 k20 s10 over 240 16.4 -> 14.0, over 700 28.9 -> 22.6.
+// No further from 64 bits (2.0e-7 -> 1.9e-7 relative for the first).
 constexpr int kQPitch = 208;  // bytes a staged row: three parts of 32 channels, 16 to spare
 constexpr int kQRows = 64 * 16;  // bytes of the 64 rows' constants (static LDS)
 constexpr int kQExchange = 4 * 3 * 16 * 64 * 4;  // bytes the waves' tiles take
